@@ -338,13 +338,118 @@ __global__ void __launch_bounds__(kMaxJobs) k_schedule(Queues q, int cur) {
 }
 
 // ------------------------------------------------------------------ emit
+// Position in the emission order of emission slot s (largest k with emitPrefix[k] <= s).
+__device__ __forceinline__ int emitPosition(const Ctrl* c, int nOrder, unsigned s) {
+    int lo = 0, hi = nOrder;
+    while (lo + 1 < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (c->emitPrefix[mid] <= s) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Emitter of a photon by the job's power CDF; draws only where there are several.
+__device__ __forceinline__ int pickEmitter(const DevJob& J, Rng& rng) {
+    if (J.nEm <= 1) return 0;
+    const double u = rng.uniformD();
+    int lo = 0, hi = J.nEm - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (J.emCdf[mid] < u) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Contiguous share [lo, hi) of column `col` of n items.
+__device__ __forceinline__ void binRange(unsigned n, unsigned col, unsigned cols, unsigned& lo, unsigned& hi) {
+    lo = (unsigned)(((unsigned long long)n * col) / cols);
+    hi = (unsigned)(((unsigned long long)n * (col + 1)) / cols);
+}
+
+// Emission order. The key of a photon is the Morton code of the two uniform draws that
+// place it on what spreads its rays most: the direction of a cosine emitter (the draws
+// map to the hemisphere with equal area, so the keys fill evenly), the origin of a
+// collimated one. With several jobs or emitters the leading bits keep those apart.
+// The photon's stream is seeded again for it: the draws cost less than storing them.
+__device__ __forceinline__ unsigned spread2(unsigned v) {
+    v = (v | (v << 4)) & 0x0f0fu;
+    v = (v | (v << 2)) & 0x3333u;
+    return (v | (v << 1)) & 0x5555u;
+}
+
+__device__ __forceinline__ unsigned emitOrderKey(const Queues& q, const Ctrl* c, int nOrder, unsigned s) {
+    const int k = nOrder > 1 ? emitPosition(c, nOrder, s) : 0;
+    const DevJob& J = q.jobs[c->emitJob[k]];
+    Rng rng = seedPhoton(J.seedBase + (c->emitStart[k] + (s - c->emitPrefix[k])), J.salt);
+    const int ei = pickEmitter(J, rng);
+    unsigned a = rng.next(), b = rng.next();
+    if (!J.ems[ei].collimated) {
+        a = rng.next();
+        b = rng.next();
+    }
+    int bits = kBinBits;
+    unsigned key = 0;
+    if (nOrder > 1) {
+        bits -= 4;
+        key = ((unsigned)k & 15u) << bits;
+    }
+    if (J.nEm > 1) {
+        bits -= 2;
+        key |= ((unsigned)ei & 3u) << bits;
+    }
+    const unsigned z = (spread2(a >> 24) << 1) | spread2(b >> 24);   // 16 bits
+    return key | (z >> (16 - bits));
+}
+
+// Keys of column blockIdx.x's emission slots and their histogram.
+__global__ void __launch_bounds__(kBinThreads) k_emit_keys(Queues q) {
+    __shared__ unsigned h[kBins];
+    const Ctrl* c = q.ctrl;
+    const unsigned n = c->nEmit;
+    if (n < kEmitOrderMin) return;
+    const int nOrder = c->nOrder;
+    for (int b = threadIdx.x; b < kBins; b += blockDim.x) h[b] = 0u;
+    __syncthreads();
+    unsigned lo, hi;
+    binRange(n, blockIdx.x, kEmitCols, lo, hi);
+    for (unsigned s = lo + threadIdx.x; s < hi; s += blockDim.x) {
+        const unsigned key = emitOrderKey(q, c, nOrder, s);
+        q.emitKey[s] = (unsigned short)key;
+        atomicAdd(&h[key], 1u);
+    }
+    __syncthreads();
+    unsigned* out = q.emitHist + (size_t)blockIdx.x * kBins;
+    for (int b = threadIdx.x; b < kBins; b += blockDim.x) out[b] = h[b];
+}
+
+// Emission slots in key order: emitPerm[sorted position] = slot. Only these 4 bytes per
+// photon are scattered; k_emit reads them in order and writes its paths in order.
+__global__ void __launch_bounds__(kBinThreads) k_emit_perm(Queues q) {
+    __shared__ unsigned slot[kBins];
+    const unsigned n = q.ctrl->nEmit;
+    if (n < kEmitOrderMin) return;
+    const unsigned col = blockIdx.x, ch = col / (kEmitCols / kBinChunks);
+    const unsigned* colHist = q.emitHist + (size_t)col * kBins;
+    const unsigned* chunk = q.emitChunk + (size_t)ch * kBins;
+    for (int b = threadIdx.x; b < kBins; b += blockDim.x) slot[b] = q.emitTotal[b] + chunk[b] + colHist[b];
+    __syncthreads();
+    unsigned lo, hi;
+    binRange(n, col, kEmitCols, lo, hi);
+    for (unsigned s = lo + threadIdx.x; s < hi; s += blockDim.x) {
+        const unsigned at = atomicAdd(&slot[q.emitKey[s]], 1u);
+        if (at < n) q.emitPerm[at] = s;   // always: both passes read the same keys
+    }
+}
+
 // Launch bound: five waves per SIMD (96 registers, no spills; -2% k_emit time on c2).
 __global__ void __launch_bounds__(256, 5) k_emit(Queues q, int cur) {
     Ctrl* c = q.ctrl;
     const unsigned nEmit = c->nEmit;
     const int nOrder = c->nOrder;
     const int nJobs = c->nJobs;
-    // emission slot s goes to segment g (segEmit[g] <= s < segEmit[g + 1]), after
+    // emission position `at` goes to segment g (segEmit[g] <= at < segEmit[g + 1]), after
     // that segment's segBase[g] survivors
     SegMap em;
     unsigned emBase[kSegs];
@@ -362,32 +467,15 @@ __global__ void __launch_bounds__(256, 5) k_emit(Queues q, int cur) {
     AccAddr ea{q.jobs, kAccEnergy};
     AccAddr pa{q.jobs, kAccPhotons};
     const unsigned stride = gridDim.x * blockDim.x;
-    for (unsigned s = blockIdx.x * blockDim.x + threadIdx.x; s < nEmit; s += stride) {
-        int k = 0;
-        if (nOrder > 1) {
-            int lo = 0, hi = nOrder;   // largest k with emitPrefix[k] <= s
-            while (lo + 1 < hi) {
-                int mid = (lo + hi) >> 1;
-                if (c->emitPrefix[mid] <= s) lo = mid;
-                else hi = mid;
-            }
-            k = lo;
-        }
+    const bool ordered = q.emitOrder && nEmit >= kEmitOrderMin;
+    for (unsigned at = blockIdx.x * blockDim.x + threadIdx.x; at < nEmit; at += stride) {
+        const unsigned s = ordered ? q.emitPerm[at] : at;   // emission slot; `at` places the path
+        const int k = nOrder > 1 ? emitPosition(c, nOrder, s) : 0;
         const int j = c->emitJob[k];
         const DevJob& J = q.jobs[j];
         const unsigned long long idx = c->emitStart[k] + (s - c->emitPrefix[k]);
         Rng rng = seedPhoton(J.seedBase + idx, J.salt);
-        int ei = 0;
-        if (J.nEm > 1) {
-            double u = rng.uniformD();
-            int lo = 0, hi = J.nEm - 1;
-            while (lo < hi) {
-                int mid = (lo + hi) >> 1;
-                if (J.emCdf[mid] < u) lo = mid + 1;
-                else hi = mid;
-            }
-            ei = lo;
-        }
+        const int ei = pickEmitter(J, rng);
         const DevEmitter& E = J.ems[ei];
         float u1 = rng.uniform();
         float u2 = rng.uniform();
@@ -421,10 +509,10 @@ __global__ void __launch_bounds__(256, 5) k_emit(Queues q, int cur) {
         F3 o = org + dir * kRayEps;
         unsigned slot = 0;
         {
-            unsigned off = s, g0 = 0;
+            unsigned off = at, g0 = 0;
 #pragma unroll
             for (int g = 1; g < kSegs; ++g)
-                if (s >= em.pre[g]) { g0 = (unsigned)g; off = s - em.pre[g]; }
+                if (at >= em.pre[g]) { g0 = (unsigned)g; off = at - em.pre[g]; }
             unsigned b = emBase[0];
 #pragma unroll
             for (int g = 1; g < kSegs; ++g)
@@ -1017,11 +1105,6 @@ __global__ void __launch_bounds__(kTravThreads) k_mirror(Queues q) {
 // contiguous logical range [n c / C, n (c + 1) / C). The order inside a (column,
 // bin) run is that of LDS atomics; nothing downstream depends on it (films, ledgers
 // and counters are integer sums).
-__device__ __forceinline__ void binRange(unsigned n, unsigned col, unsigned cols, unsigned& lo, unsigned& hi) {
-    lo = (unsigned)(((unsigned long long)n * col) / cols);
-    hi = (unsigned)(((unsigned long long)n * (col + 1)) / cols);
-}
-
 // Histogram of column xcdBlock() into binHist[col][*].
 __global__ void __launch_bounds__(kBinThreads) k_bin_count(Queues q, int cur) {
     __shared__ unsigned h[kBins];
@@ -1041,12 +1124,20 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_count(Queues q, int cur) {
     for (int b = threadIdx.x; b < kBins; b += blockDim.x) out[b] = h[b];
 }
 
+// Tables of one counting sort: hist[cols][kBins], chunk[kBinChunks][kBins], total[kBins].
+struct BinTables {
+    unsigned* hist;
+    unsigned* chunk;
+    unsigned* total;
+    int cols;
+};
+
 // Per bin: exclusive prefix of the columns inside each of the kBinChunks column
 // chunks (in place), the chunks' exclusive prefix (binChunk[chunk][bin]) and the
 // bin's total (binTotal[bin]). A workgroup takes 32 bins x kBinChunks chunks at a
 // time, grid-stride over the kBins / 32 groups.
-__global__ void __launch_bounds__(256) k_bin_chunks(Queues q) {
-    const unsigned per = (unsigned)q.binCols / kBinChunks;
+__global__ void __launch_bounds__(256) k_bin_chunks(BinTables t) {
+    const unsigned per = (unsigned)t.cols / kBinChunks;
     __shared__ unsigned part[kBinChunks][32];
     const unsigned bl = threadIdx.x & 31u, ch = threadIdx.x >> 5;
     for (unsigned grp = blockIdx.x; grp < kBins / 32; grp += gridDim.x) {
@@ -1058,15 +1149,15 @@ __global__ void __launch_bounds__(256) k_bin_chunks(Queues q) {
         for (; c + 8 <= cEnd; c += 8) {
             unsigned v[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = q.binHist[(size_t)(c + k) * kBins + bin];
+            for (int k = 0; k < 8; ++k) v[k] = t.hist[(size_t)(c + k) * kBins + bin];
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                q.binHist[(size_t)(c + k) * kBins + bin] = run;
+                t.hist[(size_t)(c + k) * kBins + bin] = run;
                 run += v[k];
             }
         }
         for (; c < cEnd; ++c) {
-            unsigned* e = q.binHist + (size_t)c * kBins + bin;
+            unsigned* e = t.hist + (size_t)c * kBins + bin;
             const unsigned v = *e;
             *e = run;
             run += v;
@@ -1076,10 +1167,10 @@ __global__ void __launch_bounds__(256) k_bin_chunks(Queues q) {
         if (ch == 0) {
             unsigned acc = 0;
             for (unsigned k = 0; k < kBinChunks; ++k) {
-                q.binChunk[(size_t)k * kBins + bin] = acc;
+                t.chunk[(size_t)k * kBins + bin] = acc;
                 acc += part[k][bl];
             }
-            q.binTotal[bin] = acc;
+            t.total[bin] = acc;
         }
         __syncthreads();
     }
@@ -1087,14 +1178,14 @@ __global__ void __launch_bounds__(256) k_bin_chunks(Queues q) {
 
 // Exclusive scan of the kBins totals in place (one workgroup of 1024 threads).
 constexpr int kBinScanThreads = kBins < 1024 ? kBins : 1024;
-__global__ void __launch_bounds__(kBinScanThreads) k_bin_scan(Queues q) {
+__global__ void __launch_bounds__(kBinScanThreads) k_bin_scan(BinTables bt) {
     constexpr int kPer = kBins / kBinScanThreads;
     __shared__ unsigned sum[kBinScanThreads];
     const unsigned t = threadIdx.x;
     unsigned v[kPer], acc = 0;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-        v[k] = q.binTotal[t * kPer + k];
+        v[k] = bt.total[t * kPer + k];
         acc += v[k];
     }
     sum[t] = acc;
@@ -1108,7 +1199,7 @@ __global__ void __launch_bounds__(kBinScanThreads) k_bin_scan(Queues q) {
     unsigned base = t ? sum[t - 1] : 0u;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-        q.binTotal[t * kPer + k] = base;
+        bt.total[t * kPer + k] = base;
         base += v[k];
     }
 }
@@ -1317,10 +1408,19 @@ void launchExtend(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s
 #undef GP_CALLS
 #undef GP_CALL
 }
+void launchEmitOrder(const Queues& q, hipStream_t s) {
+    static_assert(kEmitCols % kBinChunks == 0, "emission columns split into the scan's chunks");
+    const BinTables bt{q.emitHist, q.emitChunk, q.emitTotal, kEmitCols};
+    hipLaunchKernelGGL(k_emit_keys, dim3(kEmitCols), dim3(kBinThreads), 0, s, q);
+    hipLaunchKernelGGL(k_bin_chunks, dim3(kBins / 32), dim3(kBinChunks * 32), 0, s, bt);
+    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kBinScanThreads), 0, s, bt);
+    hipLaunchKernelGGL(k_emit_perm, dim3(kEmitCols), dim3(kBinThreads), 0, s, q);
+}
 void launchBin(const Queues& q, int cur, hipStream_t s) {
     hipLaunchKernelGGL(k_bin_count, dim3(q.binCols), dim3(kBinThreads), 0, s, q, cur);
-    hipLaunchKernelGGL(k_bin_chunks, dim3(std::min(kBins / 32, q.binCols)), dim3(kBinChunks * 32), 0, s, q);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kBinScanThreads), 0, s, q);
+    const BinTables bt{q.binHist, q.binChunk, q.binTotal, q.binCols};
+    hipLaunchKernelGGL(k_bin_chunks, dim3(std::min(kBins / 32, q.binCols)), dim3(kBinChunks * 32), 0, s, bt);
+    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kBinScanThreads), 0, s, bt);
     hipLaunchKernelGGL(k_bin_scatter, dim3(q.binCols), dim3(kBinThreads), 0, s, q, cur);
 }
 void launchConnect(const Queues& q, const LaunchShape& ls, hipStream_t s) {

@@ -42,6 +42,14 @@ struct Queues {
     int connUseSpill;
     int stats;       // 1: k_extend / k_connect count traversal statistics per job
     int binned;      // 1: ray binning on (the binning kernels run and queue 2 is read)
+    // Emission order (emitOrder = 1): the key of every emission slot, the slots in key
+    // order, and the counting-sort tables (as ray binning's, kEmitCols columns).
+    int emitOrder;
+    unsigned short* emitKey;
+    unsigned* emitPerm;
+    unsigned* emitHist;
+    unsigned* emitChunk;
+    unsigned* emitTotal;
     int binCols;     // histogram columns (a multiple of kBinColStep, <= kBinCols)
     unsigned* binHist;    // kBinCols x kBins counts, one row per column; the scan turns
                           // them into offsets inside each (bin, chunk)
@@ -63,6 +71,8 @@ struct LaunchShape {
 };
 
 void launchSchedule(const Queues& q, int cur, hipStream_t s);
+// Sorts the iteration's emission slots (four kernels; only with q.emitOrder).
+void launchEmitOrder(const Queues& q, hipStream_t s);
 void launchEmit(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s);
 void launchExtend(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s);
 void launchShade(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s);

@@ -498,6 +498,11 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.co)) != GP_OK) return st;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.cd)) != GP_OK) return st;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.cx)) != GP_OK) return st;
+        if ((st = alloc(pcap * sizeof(unsigned short), (void**)&q.emitKey)) != GP_OK) return st;
+        if ((st = alloc(pcap * sizeof(unsigned), (void**)&q.emitPerm)) != GP_OK) return st;
+        if ((st = alloc((size_t)kEmitCols * kBins * sizeof(unsigned), (void**)&q.emitHist)) != GP_OK) return st;
+        if ((st = alloc((size_t)kBinChunks * kBins * sizeof(unsigned), (void**)&q.emitChunk)) != GP_OK) return st;
+        if ((st = alloc((size_t)kBins * sizeof(unsigned), (void**)&q.emitTotal)) != GP_OK) return st;
         GP_HIP(hipMalloc(&dCtrl, sizeof(Ctrl)));
         GP_HIP(hipMalloc(&dJobs, sizeof(DevJob) * kMaxJobs));
         GP_HIP(hipHostMalloc(&hCtrl, sizeof(Ctrl)));
@@ -596,7 +601,11 @@ gp_status Engine::enqueueIterations(int n) {
     for (int i = 0; i < n; ++i) {
         const int cur = parity;
         if ((st = timed(0, [&] { launchSchedule(q, cur, s); })) != GP_OK) return st;
-        if ((st = timed(1, [&] { launchEmit(q, cur, ls, s); })) != GP_OK) return st;
+        if ((st = timed(1, [&] {
+                 if (q.emitOrder) launchEmitOrder(q, s);
+                 launchEmit(q, cur, ls, s);
+             })) != GP_OK)
+            return st;
         if (q.binned)
             if ((st = timed(5, [&] { launchBin(q, cur, s); })) != GP_OK) return st;
         if ((st = timed(2, [&] { launchExtend(q, cur, ls, s); })) != GP_OK) return st;
@@ -638,7 +647,8 @@ gp_status Engine::runIterations(int n) {
     hipStream_t s = device().stream;
     const int K = chunkIterations(tun);
     if (!tun.use_graph || tun.profile || q.stats || parity != 0 || n < K) return enqueueIterations(n);
-    if (!graph || graphIters != K || graphLds != q.lds || graphMirror != mirrorActive || graphBinned != q.binned) {
+    if (!graph || graphIters != K || graphLds != q.lds || graphMirror != mirrorActive || graphBinned != q.binned ||
+        graphEmitOrder != q.emitOrder) {
         if (graph) { hipGraphExecDestroy(graph); graph = nullptr; }
         hipGraph_t g;
         GP_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -655,6 +665,7 @@ gp_status Engine::runIterations(int n) {
         graphLds = q.lds;
         graphMirror = mirrorActive;
         graphBinned = q.binned;
+        graphEmitOrder = q.emitOrder;
     }
     int done = 0;
     while (n - done >= K) {

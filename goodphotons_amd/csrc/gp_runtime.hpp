@@ -135,6 +135,7 @@ struct Engine {
     int graphLds = 0;
     int graphShape = 0;
     int graphBinned = 0;
+    int graphEmitOrder = 0;
     // k_mirror runs in each iteration while a job of a scene with flat mirrors is live
     // (set by the caller before runIterations; the graph is re-captured on a change)
     bool mirrorActive = false;
@@ -162,6 +163,11 @@ struct Engine {
     void releaseSpill();
     gp_status enqueueIterations(int n);       // plain launches, tracks parity
     gp_status runIterations(int n);           // graph replay when possible
+    // Whether new photons are emitted in sorted order (set by the caller before
+    // runIterations, from the most photons one job of the wavefront emits).
+    void setEmitOrder(uint64_t photons) {
+        q.emitOrder = photons >= kEmitOrderJobMin && capacity >= kEmitOrderMin ? 1 : 0;
+    }
     gp_status readCtrl();                     // synchronous copy of the control block
 };
 Engine& engine();

@@ -397,9 +397,10 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
     gp_status st;
     int maxStackNeed = 0;
     bool mirrors = false;
-    int64_t maxTris = 0;
+    int64_t maxTris = 0, maxPhotons = 0;
     for (auto& kv : srv->jobs) {
         if (kv.second.state == JobState::Finished) continue;   // its scene is no longer used
+        maxPhotons = std::max<int64_t>(maxPhotons, kv.second.desc.params.n_photons);
         maxStackNeed = std::max(maxStackNeed, kv.second.desc.scene->stackNeed);
         mirrors = mirrors || kv.second.desc.scene->nMirrors > 0;
         maxTris = std::max(maxTris, kv.second.desc.scene->nTris);
@@ -419,6 +420,7 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
     const unsigned oldCap = E.capacity, oldSeg = E.segCap;
     if ((st = E.ensure((unsigned)E.tun.queue_capacity, lds, maxStackNeed, 1, mirrors, maxTris)) != GP_OK) return st;
     E.mirrorActive = mirrors;
+    E.setEmitOrder((uint64_t)maxPhotons);
     const bool fresh = !srv->engineReady || E.capacity != oldCap || E.segCap != oldSeg || srv->epoch != E.epoch;
     if (fresh) {
         if (!srv->order.empty() || !srv->inflight.empty())
