@@ -325,8 +325,7 @@ def main():
     ap.add_argument("--autotune", action="store_true")
     ap.add_argument("--ray-sort", type=int, choices=[0, 1, 2], default=None,
                     help="gp_tuning.ray_sort: 0 queue order, 1 bin each iteration's paths by origin cell and "
-                         "direction octant, 2 automatic (the library default: binned for scenes of 4096 "
-                         "triangles and more)")
+                         "direction octant, 2 automatic (the library default: queue order)")
     ap.add_argument("--lds-stack", type=int, choices=[8, 12, 16, 24, 32], default=None,
                     help="gp_tuning.lds_stack: LDS traversal stack entries per lane (default 12)")
     ap.add_argument("--queue-capacity", type=int, default=None,

@@ -70,6 +70,11 @@ struct LaunchShape {
     int blocksShade, threadsShade;
 };
 
+// k_shade runs workgroups of kShadeThreads, as many threads in all as the other kernels
+// of `blocks` 256-thread workgroups.
+constexpr int kShadeThreads = 512;
+constexpr int shadeBlocks(int blocks) { return (blocks * 256 + kShadeThreads - 1) / kShadeThreads; }
+
 void launchSchedule(const Queues& q, int cur, hipStream_t s);
 // Sorts the iteration's emission slots (four kernels; only with q.emitOrder).
 void launchEmitOrder(const Queues& q, hipStream_t s);

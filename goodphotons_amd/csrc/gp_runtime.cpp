@@ -328,7 +328,7 @@ gp_tuning defaultTuning() {
     // with 16 entries and five waves); k_connect keeps 8.
     t.lds_stack = 12;
     t.profile = 0;
-    t.ray_sort = 2;   // automatic: binned for scenes of kBinAutoTris to kBinAutoMaxTris triangles
+    t.ray_sort = 2;   // automatic (see binningFor)
     return t;
 }
 
@@ -373,17 +373,17 @@ void Engine::release() {
 }
 
 // Largest number of items that the workgroups b with b % kSegs == g visit, over g,
-// when `blocks` workgroups of 256 threads grid-stride over cap items (the loop
+// when `blocks` workgroups of `threads` threads grid-stride over cap items (the loop
 // shape of k_emit and k_shade). A segment receives at most one path and one
 // connection per item its workgroups visit, so this bounds every segment's fill.
 // The items sum to cap over the segments, so kSegs * bound >= cap.
-unsigned segmentBound(unsigned cap, unsigned blocks) {
+unsigned segmentBound(unsigned cap, unsigned blocks, unsigned threads) {
     uint64_t per[kSegs] = {};
-    const uint64_t stride = (uint64_t)blocks * 256;
+    const uint64_t stride = (uint64_t)blocks * threads;
     for (unsigned b = 0; b < blocks; ++b) {
         uint64_t items = 0;
-        for (uint64_t start = (uint64_t)b * 256; start < cap; start += stride)
-            items += std::min<uint64_t>(256, cap - start);
+        for (uint64_t start = (uint64_t)b * threads; start < cap; start += stride)
+            items += std::min<uint64_t>(threads, cap - start);
         per[b % kSegs] += items;
     }
     uint64_t m = 0;
@@ -436,11 +436,9 @@ gp_status Engine::readJobAcc(int slot, unsigned long long ledger[5], unsigned lo
     return GP_OK;
 }
 
-bool binningFor(const gp_tuning& t, int64_t maxTris) {
-    return t.ray_sort == 1 || (t.ray_sort == 2 && maxTris >= kBinAutoTris && maxTris < kBinAutoMaxTris);
-}
+bool binningFor(const gp_tuning& t) { return t.ray_sort == 1; }
 
-gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mirrors, int64_t maxTris) {
+gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mirrors) {
     if (!tunSet) { tun = defaultTuning(); tunSet = true; }
     DeviceState& d = device();
     const int cus = d.cus > 0 ? d.cus : 256;
@@ -449,12 +447,14 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
     ls.blocksExtend = std::max(1, cus * tun.grid_waves_per_cu / 4);
     ls.blocksShade = std::max(1, cus * tun.grid_waves_per_cu / 4);
     const size_t threads = (size_t)ls.blocksExtend * 256 * kExtendGridScale;
-    const unsigned sc = segmentBound(cap, (unsigned)ls.blocksShade);
+    // k_emit appends connections and k_shade paths and connections, each over its own grid
+    const unsigned sc = std::max(segmentBound(cap, (unsigned)ls.blocksShade, 256),
+                                 segmentBound(cap, (unsigned)shadeBlocks(ls.blocksShade), kShadeThreads));
     const int camsNeed = std::max(camCap, std::max(1, cams));
     const bool needQueues = (cap != capacity) || sc != segCap || camsNeed != camCap || !dCtrl;
     const bool wantMirror = mirrors || mirrorQueue;
     const bool needMirrorAlloc = wantMirror && (needQueues || !q.mv[0]);
-    const int binned = binningFor(tun, maxTris) ? 1 : 0;
+    const int binned = binningFor(tun) ? 1 : 0;
     const bool needBinAlloc = binned && (needQueues || !q.pb);
     // Entries beyond the LDS stack live in the spill area (stack index sp >= SD maps to
     // spill[sp - SD], and sp < stackNeed). k_connect keeps as many entries in LDS as the

@@ -156,8 +156,7 @@ struct Engine {
 
     // stackNeed: traversal stack entries the traced scenes can need (gp_scene::stackNeed);
     // mirrors: allocate the mirror-vertex queue (kept from then on, like the camera count)
-    // maxTris: the largest triangle count of the traced scenes (automatic ray binning)
-    gp_status ensure(unsigned cap, int lds, int stackNeed, int cams = 1, bool mirrors = false, int64_t maxTris = 0);
+    gp_status ensure(unsigned cap, int lds, int stackNeed, int cams = 1, bool mirrors = false);
     void release();
     void releaseQueues();
     void releaseSpill();
@@ -177,10 +176,13 @@ gp_tuning defaultTuning();
 inline int chunkIterations(const gp_tuning& t) {
     return t.use_graph ? std::max(2, t.iters_per_graph & ~1) : std::max(1, t.iters_per_graph);
 }
-unsigned segmentBound(unsigned cap, unsigned blocks);
-// Whether the wavefront bins its rays (gp_tuning.ray_sort: 1 always, 2 when the largest
-// traced scene has kBinAutoTris to kBinAutoMaxTris - 1 triangles).
-bool binningFor(const gp_tuning& t, int64_t maxTris);
+unsigned segmentBound(unsigned cap, unsigned blocks, unsigned threads);
+// Whether the wavefront bins its rays: with gp_tuning.ray_sort = 1. Automatic (2) does
+// not: with new photons emitted in sorted order and survivors sorted per workgroup, the
+// full sort costs more than it gains on every scene measured (whole traces, queue order
+// against binned: 8K-triangle glass scene 28.2 vs 31.4 ms, icospheres of 5K / 82K 15.1 vs
+// 17.8 / 18.9 vs 21.7 ms, soups of 20K / 60K 4.8 vs 5.4 / 8.3 vs 8.7 ms).
+bool binningFor(const gp_tuning& t);
 // Sums the kSegs accumulator rows of one job: ledger[5] (fixed point) and
 // counters[kAccCounters] (the quantities from kAccPhotons on).
 void sumAccRows(const unsigned long long* rows, unsigned long long ledger[5], unsigned long long* counters);

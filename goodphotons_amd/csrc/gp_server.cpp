@@ -397,13 +397,12 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
     gp_status st;
     int maxStackNeed = 0;
     bool mirrors = false;
-    int64_t maxTris = 0, maxPhotons = 0;
+    int64_t maxPhotons = 0;
     for (auto& kv : srv->jobs) {
         if (kv.second.state == JobState::Finished) continue;   // its scene is no longer used
         maxPhotons = std::max<int64_t>(maxPhotons, kv.second.desc.params.n_photons);
         maxStackNeed = std::max(maxStackNeed, kv.second.desc.scene->stackNeed);
         mirrors = mirrors || kv.second.desc.scene->nMirrors > 0;
-        maxTris = std::max(maxTris, kv.second.desc.scene->nTris);
     }
     const int lds = E.tun.lds_stack;
     if (srv->engineReady && !srv->inflight.empty()) {
@@ -411,14 +410,14 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
         const int need = std::max(0, maxStackNeed - lds);
         const bool connSpill = maxStackNeed > std::max(lds, 24);
         if (need > E.spillDepth || (need > 0) != (E.q.useSpill != 0) || connSpill != (E.q.connUseSpill != 0) ||
-            (mirrors && !E.q.mv[0]) || mirrors != E.mirrorActive || binningFor(E.tun, maxTris) != (E.q.binned != 0)) {
+            (mirrors && !E.q.mv[0]) || mirrors != E.mirrorActive || binningFor(E.tun) != (E.q.binned != 0)) {
             while (!srv->inflight.empty())
                 if ((st = processOldest(E, srv)) != GP_OK) return st;
             GP_HIP(hipStreamSynchronize(device().stream));
         }
     }
     const unsigned oldCap = E.capacity, oldSeg = E.segCap;
-    if ((st = E.ensure((unsigned)E.tun.queue_capacity, lds, maxStackNeed, 1, mirrors, maxTris)) != GP_OK) return st;
+    if ((st = E.ensure((unsigned)E.tun.queue_capacity, lds, maxStackNeed, 1, mirrors)) != GP_OK) return st;
     E.mirrorActive = mirrors;
     E.setEmitOrder((uint64_t)maxPhotons);
     const bool fresh = !srv->engineReady || E.capacity != oldCap || E.segCap != oldSeg || srv->epoch != E.epoch;

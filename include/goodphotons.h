@@ -419,8 +419,8 @@ typedef struct gp_tuning {
                                 (8 x 8 x 8 over the scene) and direction octant before
                                 the closest-hit kernel, a counting sort into a third
                                 path queue, so that the lanes of a wave trace similar
-                                rays; 0 = queue order; 2 = automatic (default): 1 while
-                                the largest traced scene has 4096 to 65535 triangles.
+                                rays; 0 = queue order; 2 = automatic (default): queue
+                                order, the faster one on every scene measured.
                                 Results are identical in every mode; gp_autotune tries
                                 0 and 1. */
 } gp_tuning;
