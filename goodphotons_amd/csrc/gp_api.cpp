@@ -585,29 +585,28 @@ gp_status gp_trace_shared(gp_scene* s, int32_t n_cams, const gp_camera_desc* cam
         gp_trace_params cp = *p;
         cp.n_photons = n;
         cp.seed_base = p->seed_base + (uint64_t)done;
-        DevJob J;
-        if ((st = fillJob(s, cams, films, n_cams, cp, 0, J, E.hJobCams)) != GP_OK) return st;
-        E.hJobs[0] = J;
-        Ctrl& C = *E.hCtrl;
-        E.initCtrl();
-        C.nJobs = 1;
-        C.nOrder = 1;
-        C.order[0] = 0;
-        C.nextPhoton[0] = 0;
-        C.endPhoton[0] = (unsigned long long)n;
-        C.active[0] = 1;
-        C.lastEmitIter[0] = -1;
-        GP_HIP(hipMemcpyAsync(E.dJobs, E.hJobs, sizeof(DevJob), hipMemcpyHostToDevice, strm));
-        GP_HIP(hipMemcpyAsync(E.dJobCams, E.hJobCams, sizeof(DevCamera) * (size_t)n_cams, hipMemcpyHostToDevice, strm));
-        GP_HIP(hipMemcpyAsync(E.dCtrl, E.hCtrl, sizeof(Ctrl), hipMemcpyHostToDevice, strm));
-        if ((st = E.resetJobAcc(0)) != GP_OK) return st;
+        const bool once = (uint64_t)n <= E.capacity;
+        TraceStart ts{};
+        DevJob& J = ts.job;
+        if ((st = fillJob(s, cams, films, n_cams, cp, 0, J, ts.cams)) != GP_OK) return st;
+        ts.photons = (unsigned long long)n;
+        ts.capacity = E.capacity;
+        ts.nCams = n_cams;
+        ts.once = once ? 1 : 0;
+        launchStartTrace(E.q, ts, strm);
+        GP_HIP(hipGetLastError());
         E.parity = 0;
+        const Ctrl& C = *E.hCtrl;
+        int64_t iters = 0;
+        if (once) {
+            if ((st = E.traceOnce((unsigned)n, n_cams, p->max_depth)) != GP_OK) return st;
+            iters = E.onceIterations;
+        }
         const int K = chunkIterations(E.tun);
         // Every iteration retires or advances each live path by one segment, so the
         // loop needs at most ceil(n / capacity) refills times maxDepth iterations.
         const int64_t maxIters = ((n + E.capacity - 1) / E.capacity + 2) * (int64_t)(p->max_depth + 2) * 2 + 64;
-        int64_t iters = 0;
-        while (true) {
+        while (!once) {
             if ((st = E.runIterations(K)) != GP_OK) return st;
             iters += K;
             if ((st = E.readCtrl()) != GP_OK) return st;
@@ -617,14 +616,14 @@ gp_status gp_trace_shared(gp_scene* s, int32_t n_cams, const gp_camera_desc* cam
             if (iters > maxIters) return fail(GP_ERR_STATE, "wavefront did not drain");
         }
         unsigned long long ev[5], cv[kAccCounters];
-        if ((st = E.readJobAcc(0, ev, cv)) != GP_OK) return st;
+        sumAccRows(E.traceRows(), ev, cv);
         eacc.emitted += (double)ev[0] / J.energyScale;
         eacc.absorbed += (double)ev[1] / J.energyScale;
         eacc.sensor += (double)ev[2] / J.energyScale;
         eacc.escaped += (double)ev[3] / J.energyScale;
         eacc.residual += (double)ev[4] / J.energyScale;
         addCounters(cv, acc);
-        acc.iterations += C.iter;
+        acc.iterations += (uint64_t)iters;
         done += n;
     }
     auto t1 = std::chrono::steady_clock::now();

@@ -1,7 +1,10 @@
 // Wavefront forward light-tracing kernels for CDNA4 (gfx950).
 //
 // One iteration of the wavefront:
-//   k_schedule  (1 block)  refill free queue slots from the jobs' photon budgets
+//   k_schedule  (1 block)  refill free queue slots from the jobs' photon budgets (a trace
+//                          that fits the queue starts with k_start_trace instead and
+//                          emits once)
+//   k_emit_keys, k_bin_chunks, k_bin_scan, k_emit_perm  (large traces) sort the new photons
 //   k_emit                 emission + hero bundle + direct light->camera connection
 //   k_bin_*                (gp_tuning.ray_sort only) counting sort of the paths by
 //                          origin cell and direction octant into a third queue
@@ -532,9 +535,6 @@ __global__ void __launch_bounds__(256, 5) k_emit(Queues q, int cur) {
 }
 
 // ------------------------------------------------------------------ extend
-// One wave per workgroup: a workgroup's LDS (its lanes' stacks) is released as soon as
-// its own rays are done, instead of waiting for the slowest of four waves.
-constexpr int kExtendThreads = 64;
 // STATS: also count the traversal statistics (node visits, triangle tests) per job.
 // BIN: read the binned queue (ray binning) instead of queue `cur`.
 // The traversal waits on dependent node loads, so resident waves are what hides the
@@ -552,6 +552,12 @@ __global__ void __launch_bounds__(kExtendThreads, 6) k_extend(Queues q, int cur)
     __shared__ unsigned segTab[kSegs];
     SegMap sm;
     const unsigned n = loadSegMap(q.ctrl->pathCount[cur], q.segCap, sm);
+    if (q.resetCounts && blockIdx.x == 0 && threadIdx.x < kSegs) {
+        // nothing else of this kernel touches these; the last readers ran before it
+        q.ctrl->pathCount[cur ^ 1][threadIdx.x][0] = 0u;
+        q.ctrl->connCount[threadIdx.x][0] = 0u;
+        q.ctrl->mirrorCount[threadIdx.x][0] = 0u;
+    }
     if constexpr (!BIN) {
         initSegTab(sm, segTab);
         __syncthreads();
@@ -1379,6 +1385,47 @@ __global__ void __launch_bounds__(256) k_install_job(Queues q, JobInstall a) {
     for (int k = threadIdx.x; k < kSegs * kAccRow; k += blockDim.x) a.job.acc[k] = 0ull;
 }
 
+// Starts a trace: the control block, job slot 0, its cameras and zeroed ledger rows from
+// the kernel's arguments (one launch instead of three copies and a fill). With `once` the
+// whole budget fits the path queue: all photons are laid out over the segments as
+// k_schedule would in iteration 0, and the later iterations need no k_schedule or k_emit.
+__global__ void __launch_bounds__(256) k_start_trace(Queues q, TraceStart a) {
+    Ctrl* c = q.ctrl;
+    unsigned* words = (unsigned*)c;
+    for (unsigned k = threadIdx.x; k < sizeof(Ctrl) / sizeof(unsigned); k += blockDim.x) words[k] = 0u;
+    for (int k = threadIdx.x; k < kSegs * kAccRow; k += blockDim.x) a.job.acc[k] = 0ull;
+    __syncthreads();
+    c->lastEmitIter[threadIdx.x] = -1;
+    if (threadIdx.x < (unsigned)a.nCams) const_cast<DevCamera*>(a.job.cams)[threadIdx.x] = a.cams[threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const_cast<DevJob*>(q.jobs)[0] = a.job;
+    c->nJobs = 1;
+    c->nOrder = 1;
+    c->capacity = a.capacity;
+    c->segCap = q.segCap;
+    c->connSegCap = q.connSegCap;
+    c->mirrorSegCap = q.mirrorSegCap;
+    c->endPhoton[0] = a.photons;
+    c->active[0] = 1;
+    if (a.once) {
+        const unsigned n = (unsigned)a.photons;
+        unsigned placed = 0;
+        for (int g = 0; g < kSegs; ++g) {
+            const unsigned e = min(n - placed, q.segCap);
+            c->segEmit[g] = placed;
+            c->pathCount[0][g][0] = e;
+            placed += e;
+        }
+        c->segEmit[kSegs] = placed;
+        c->nEmit = n;
+        c->emitPrefix[1] = n;
+        c->nextPhoton[0] = a.photons;
+        c->lastEmitIter[0] = 0;
+        c->iter = 1;
+    }
+}
+
 __global__ void __launch_bounds__(kMaxJobs) k_set_order(Queues q, OrderUpdate a) {
     Ctrl* c = q.ctrl;
     c->order[threadIdx.x] = a.order[threadIdx.x];
@@ -1399,11 +1446,11 @@ void launchSchedule(const Queues& q, int cur, hipStream_t s) {
     hipLaunchKernelGGL(k_schedule, dim3(1), dim3(kMaxJobs), 0, s, q, cur);
 }
 void launchEmit(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s) {
-    hipLaunchKernelGGL(k_emit, dim3(ls.blocksShade), dim3(256), 0, s, q, cur);
+    hipLaunchKernelGGL(k_emit, dim3(ls.emit), dim3(256), 0, s, q, cur);
 }
 void launchShade(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s) {
-    if (q.binned) hipLaunchKernelGGL(k_shade<true>, dim3(shadeBlocks(ls.blocksShade)), dim3(kShadeThreads), 0, s, q, cur);
-    else hipLaunchKernelGGL(k_shade<false>, dim3(shadeBlocks(ls.blocksShade)), dim3(kShadeThreads), 0, s, q, cur);
+    if (q.binned) hipLaunchKernelGGL(k_shade<true>, dim3(ls.shade), dim3(kShadeThreads), 0, s, q, cur);
+    else hipLaunchKernelGGL(k_shade<false>, dim3(ls.shade), dim3(kShadeThreads), 0, s, q, cur);
 }
 // Kernel instances by LDS stack depth and spill use.
 #define GP_BY_STACK(LDS, SPILL, CALL) \
@@ -1439,7 +1486,7 @@ void launchShade(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s)
     } while (0)
 
 void launchExtend(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s) {
-    const dim3 grid(ls.blocksExtend * kExtendGridScale * (kTravThreads / kExtendThreads));
+    const dim3 grid(ls.extend);
 #define GP_CALL(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, false, false>), grid, dim3(kExtendThreads), 0, s, q, cur)
 #define GP_CALLS(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, true, false>), grid, dim3(kExtendThreads), 0, s, q, cur)
 #define GP_CALLB(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, false, true>), grid, dim3(kExtendThreads), 0, s, q, cur)
@@ -1472,15 +1519,15 @@ void launchBin(const Queues& q, int cur, hipStream_t s) {
     hipLaunchKernelGGL(k_bin_scatter, dim3(q.binCols), dim3(kBinThreads), 0, s, q, cur);
 }
 void launchConnect(const Queues& q, const LaunchShape& ls, hipStream_t s) {
-#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_connect<SD, SP, false>), dim3(ls.blocksExtend), dim3(kTravThreads), 0, s, q)
-#define GP_CALLS(SD, SP) hipLaunchKernelGGL((k_connect<SD, SP, true>), dim3(ls.blocksExtend), dim3(kTravThreads), 0, s, q)
+#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_connect<SD, SP, false>), dim3(ls.connect), dim3(kTravThreads), 0, s, q)
+#define GP_CALLS(SD, SP) hipLaunchKernelGGL((k_connect<SD, SP, true>), dim3(ls.connect), dim3(kTravThreads), 0, s, q)
     if (q.stats) GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALLS);
     else GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALL);
 #undef GP_CALLS
 #undef GP_CALL
 }
 void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s) {
-#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_mirror<SD, SP>), dim3(ls.blocksExtend), dim3(kTravThreads), 0, s, q)
+#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_mirror<SD, SP>), dim3(ls.mirror), dim3(kTravThreads), 0, s, q)
     GP_BY_STACK(q.lds, q.useSpill, GP_CALL);
 #undef GP_CALL
 }
@@ -1503,6 +1550,10 @@ void launchProbeAny(const float4* nodes, const float4* tris, const float* rays, 
 #undef GP_BY_STACK
 void launchInstallJob(const Queues& q, const JobInstall& a, hipStream_t s) {
     hipLaunchKernelGGL(k_install_job, dim3(1), dim3(256), 0, s, q, a);
+}
+void launchStartTrace(const Queues& q, const TraceStart& a, hipStream_t s) {
+    static_assert(kMaxJobs == 256, "one thread per job slot");
+    hipLaunchKernelGGL(k_start_trace, dim3(1), dim3(256), 0, s, q, a);
 }
 void launchSetOrder(const Queues& q, const OrderUpdate& a, hipStream_t s) {
     hipLaunchKernelGGL(k_set_order, dim3(1), dim3(kMaxJobs), 0, s, q, a);

@@ -56,6 +56,8 @@ struct Queues {
     unsigned* binChunk;   // kBins x kBinChunks exclusive prefixes of the column chunks
     unsigned* binTotal;   // kBins totals, then (after the scan) kBins first slots
     unsigned segCap, connSegCap, mirrorSegCap;
+    int resetCounts;   // k_extend zeroes the counters of this iteration's appends (traces of
+                       // one refill, which run k_schedule's work once, in k_start_trace)
 };
 
 // The closest-hit kernel's grid holds kExtendGridScale times the threads of the other
@@ -65,15 +67,15 @@ struct Queues {
 // further).
 constexpr int kExtendGridScale = 4;
 
-struct LaunchShape {
-    int blocksExtend, threadsExtend;
-    int blocksShade, threadsShade;
-};
-
-// k_shade runs workgroups of kShadeThreads, as many threads in all as the other kernels
-// of `blocks` 256-thread workgroups.
+// Threads of a workgroup of k_extend (one wave: a workgroup's LDS, its lanes' stacks, is
+// released as soon as its own rays are done) and k_shade; the others run 256.
+constexpr int kExtendThreads = 64;
 constexpr int kShadeThreads = 512;
-constexpr int shadeBlocks(int blocks) { return (blocks * 256 + kShadeThreads - 1) / kShadeThreads; }
+
+// Workgroups per launch of each kernel.
+struct LaunchShape {
+    int emit, extend, shade, connect, mirror;
+};
 
 void launchSchedule(const Queues& q, int cur, hipStream_t s);
 // Sorts the iteration's emission slots (four kernels; only with q.emitOrder).
@@ -105,6 +107,18 @@ struct JobInstall {
     int32_t slot;
     int32_t pad[3];
 };
+// Start of a gp_trace: job slot 0, its cameras and the control block. `once`: the whole
+// budget fits the path queue, so the first iteration's emission is laid out here.
+struct TraceStart {
+    DevJob job;
+    DevCamera cams[kMaxCams];
+    unsigned long long photons;
+    unsigned capacity;
+    int32_t nCams, once;
+    int32_t pad;
+};
+static_assert(sizeof(TraceStart) + sizeof(Queues) <= 4096, "kernel arguments");
+void launchStartTrace(const Queues& q, const TraceStart& a, hipStream_t s);
 struct OrderUpdate {
     int32_t order[kMaxJobs];
     int32_t nOrder, nJobs;

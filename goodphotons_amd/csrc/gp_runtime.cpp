@@ -341,15 +341,12 @@ void Engine::releaseQueues() {
     if (graph) { hipGraphExecDestroy(graph); graph = nullptr; }
     for (int i = 0; i < nbufs; ++i) hipFree(bufs[i]);
     nbufs = 0;
-    if (dCtrl) hipFree(dCtrl);
+    if (dCtrl) hipFree(dCtrl);   // dJobAcc lies behind it
     if (dJobs) hipFree(dJobs);
     if (hCtrl) hipHostFree(hCtrl);
-    if (hJobs) hipHostFree(hJobs);
-    if (dJobAcc) hipFree(dJobAcc);
     if (dJobCams) hipFree(dJobCams);
-    if (hJobCams) hipHostFree(hJobCams);
-    dCtrl = nullptr; dJobs = nullptr; hCtrl = nullptr; hJobs = nullptr;
-    dJobAcc = nullptr; dJobCams = nullptr; hJobCams = nullptr;
+    dCtrl = nullptr; dJobs = nullptr; hCtrl = nullptr;
+    dJobAcc = nullptr; dJobCams = nullptr;
     int2* sp = q.spill;
     q = Queues{};
     q.spill = sp;
@@ -400,12 +397,6 @@ void Engine::initCtrl() {
     for (int k = 0; k < kMaxJobs; ++k) hCtrl->lastEmitIter[k] = -1;
 }
 
-gp_status Engine::resetJobAcc(int slot) {
-    launchFill64(dJobAcc + (size_t)slot * kSegs * kAccRow, (size_t)kSegs * kAccRow, 0ull, device().stream);
-    GP_HIP(hipGetLastError());
-    return GP_OK;
-}
-
 void sumAccRows(const unsigned long long* rows, unsigned long long ledger[5], unsigned long long* counters) {
     for (int k = 0; k < 5; ++k) ledger[k] = 0;
     for (int k = 0; k < kAccCounters; ++k) counters[k] = 0;
@@ -427,14 +418,6 @@ void addCounters(const unsigned long long* cv, gp_trace_stats& st) {
     st.shadow_tri_tests += cv[kAccAnyTriTests - kAccPhotons];
 }
 
-gp_status Engine::readJobAcc(int slot, unsigned long long ledger[5], unsigned long long* counters) {
-    unsigned long long rows[kSegs * kAccRow];
-    GP_HIP(hipMemcpyAsync(rows, dJobAcc + (size_t)slot * kSegs * kAccRow, sizeof rows,
-                          hipMemcpyDeviceToHost, device().stream));
-    GP_HIP(hipStreamSynchronize(device().stream));
-    sumAccRows(rows, ledger, counters);
-    return GP_OK;
-}
 
 bool binningFor(const gp_tuning& t) { return t.ray_sort == 1; }
 
@@ -442,14 +425,14 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
     if (!tunSet) { tun = defaultTuning(); tunSet = true; }
     DeviceState& d = device();
     const int cus = d.cus > 0 ? d.cus : 256;
-    ls.threadsExtend = 256;
-    ls.threadsShade = 256;
-    ls.blocksExtend = std::max(1, cus * tun.grid_waves_per_cu / 4);
-    ls.blocksShade = std::max(1, cus * tun.grid_waves_per_cu / 4);
-    const size_t threads = (size_t)ls.blocksExtend * 256 * kExtendGridScale;
+    const int blocks = std::max(1, cus * tun.grid_waves_per_cu / 4);
+    ls.emit = ls.connect = ls.mirror = blocks;
+    ls.shade = (blocks * 256 + kShadeThreads - 1) / kShadeThreads;
+    ls.extend = blocks * kExtendGridScale * (256 / kExtendThreads);
+    const size_t threads = (size_t)ls.extend * kExtendThreads;
     // k_emit appends connections and k_shade paths and connections, each over its own grid
-    const unsigned sc = std::max(segmentBound(cap, (unsigned)ls.blocksShade, 256),
-                                 segmentBound(cap, (unsigned)shadeBlocks(ls.blocksShade), kShadeThreads));
+    const unsigned sc = std::max(segmentBound(cap, (unsigned)ls.emit, 256),
+                                 segmentBound(cap, (unsigned)ls.shade, kShadeThreads));
     const int camsNeed = std::max(camCap, std::max(1, cams));
     const bool needQueues = (cap != capacity) || sc != segCap || camsNeed != camCap || !dCtrl;
     const bool wantMirror = mirrors || mirrorQueue;
@@ -470,7 +453,7 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
     const int useSpill = needSpill > 0 ? 1 : 0;
     if (!needQueues && !needSpillAlloc && !needMirrorAlloc && !needBinAlloc && q.lds == lds &&
         q.useSpill == useSpill && q.connLds == connLds && q.connUseSpill == connUseSpill &&
-        graphShape == ls.blocksExtend && q.binned == binned)
+        graphShape == ls.extend && q.binned == binned)
         return GP_OK;
     if (graph) { hipGraphExecDestroy(graph); graph = nullptr; }
     if (needQueues) {
@@ -503,15 +486,14 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
         if ((st = alloc((size_t)kEmitCols * kBins * sizeof(unsigned), (void**)&q.emitHist)) != GP_OK) return st;
         if ((st = alloc((size_t)kBinChunks * kBins * sizeof(unsigned), (void**)&q.emitChunk)) != GP_OK) return st;
         if ((st = alloc((size_t)kBins * sizeof(unsigned), (void**)&q.emitTotal)) != GP_OK) return st;
-        GP_HIP(hipMalloc(&dCtrl, sizeof(Ctrl)));
+        // the ledger rows behind the control block, so that one copy reads a trace's both
+        constexpr size_t slotAcc = sizeof(unsigned long long) * kSegs * kAccRow;
+        GP_HIP(hipMalloc((void**)&dCtrl, kCtrlStride + slotAcc * kMaxJobs));
+        dJobAcc = (unsigned long long*)((char*)dCtrl + kCtrlStride);
         GP_HIP(hipMalloc(&dJobs, sizeof(DevJob) * kMaxJobs));
-        GP_HIP(hipHostMalloc(&hCtrl, sizeof(Ctrl)));
-        GP_HIP(hipHostMalloc(&hJobs, sizeof(DevJob) * kMaxJobs));
-        GP_HIP(hipMalloc(&dJobAcc, sizeof(unsigned long long) * kMaxJobs * kSegs * kAccRow));
+        GP_HIP(hipHostMalloc((void**)&hCtrl, kCtrlStride + slotAcc));
         GP_HIP(hipMalloc(&dJobCams, sizeof(DevCamera) * kMaxJobs * kMaxCams));
-        GP_HIP(hipHostMalloc(&hJobCams, sizeof(DevCamera) * kMaxJobs * kMaxCams));
         std::memset(hCtrl, 0, sizeof(Ctrl));
-        std::memset(hJobs, 0, sizeof(DevJob) * kMaxJobs);
         capacity = cap;
         segCap = sc;
         q.ctrl = dCtrl;
@@ -579,41 +561,92 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
     q.binned = binned;
     q.binCols = std::min(kBinCols, std::max(kBinColStep, (cus * 4) / kBinColStep * kBinColStep));
     static_assert(kBinColStep % kBinChunks == 0 && kBinCols % kBinColStep == 0, "binning column shape");
-    graphShape = ls.blocksExtend;
+    graphShape = ls.extend;
     return GP_OK;
+}
+
+// One launch, timed with HIP events while gp_tuning.profile is set.
+template <class F>
+gp_status Engine::timed(int k, F&& launch) {
+    if (!tun.profile) { launch(); return GP_OK; }
+    hipStream_t s = device().stream;
+    std::array<hipEvent_t, 2> ev;
+    GP_HIP(hipEventCreate(&ev[0]));
+    GP_HIP(hipEventCreate(&ev[1]));
+    GP_HIP(hipEventRecord(ev[0], s));
+    launch();
+    GP_HIP(hipEventRecord(ev[1], s));
+    pending[k].push_back(ev);
+    return GP_OK;
+}
+
+gp_status Engine::enqueueEmit(const LaunchShape& sh) {
+    hipStream_t s = device().stream;
+    return timed(1, [&] {
+        if (q.emitOrder) launchEmitOrder(q, s);
+        launchEmit(q, parity, sh, s);
+    });
+}
+
+// Closest hit, scatter and connections of the paths in queue `parity`.
+gp_status Engine::enqueueBounce(const LaunchShape& sh) {
+    hipStream_t s = device().stream;
+    const int cur = parity;
+    gp_status st;
+    if (q.binned)
+        if ((st = timed(5, [&] { launchBin(q, cur, s); })) != GP_OK) return st;
+    if ((st = timed(2, [&] { launchExtend(q, cur, sh, s); })) != GP_OK) return st;
+    if ((st = timed(3, [&] { launchShade(q, cur, sh, s); })) != GP_OK) return st;
+    if ((st = timed(4, [&] { launchConnect(q, sh, s); })) != GP_OK) return st;
+    if (mirrorActive && q.mv[0])
+        if ((st = timed(4, [&] { launchMirror(q, sh, s); })) != GP_OK) return st;
+    parity ^= 1;
+    return GP_OK;
+}
+
+gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
+    // Workgroups for n items, at most the full grid. A segment's fill stays within its
+    // bound: of G workgroups over n items a segment sees at most G / kSegs + 1.
+    const bool fit = (uint64_t)n + kSegs * kShadeThreads <= capacity;
+    auto blocks = [&](uint64_t items, unsigned threads, int full) {
+        return fit ? (int)std::min<uint64_t>((uint64_t)full, (items + threads - 1) / threads) : full;
+    };
+    LaunchShape sh = ls;
+    sh.emit = blocks(n, 256, ls.emit);
+    sh.extend = blocks(n, kExtendThreads, ls.extend);
+    sh.shade = blocks(n, kShadeThreads, ls.shade);
+    // the first iteration connects the emitted photons and the shaded vertices
+    sh.connect = blocks(2 * (uint64_t)n * (uint64_t)cams, 256, ls.connect);
+    sh.mirror = blocks(2 * (uint64_t)n, 256, ls.mirror);
+    gp_status st;
+    if ((st = enqueueEmit(sh)) != GP_OK) return st;
+    for (int i = 0; i < maxDepth;) {
+        const int stop = std::min(maxDepth, i + kOnceChunk);
+        for (; i < stop; ++i) {
+            q.resetCounts = i > 0 ? 1 : 0;
+            st = enqueueBounce(sh);
+            q.resetCounts = 0;
+            if (st != GP_OK) return st;
+            sh.connect = blocks((uint64_t)n * (uint64_t)cams, 256, ls.connect);
+            sh.mirror = blocks(n, 256, ls.mirror);
+        }
+        onceIterations = i;
+        GP_HIP(hipGetLastError());
+        if ((st = readCtrl()) != GP_OK) return st;
+        unsigned live = 0;
+        for (int g = 0; g < kSegs; ++g) live += hCtrl->pathCount[parity][g][0];
+        if (live == 0) return GP_OK;
+    }
+    return fail(GP_ERR_STATE, "paths alive past their depth limit");
 }
 
 gp_status Engine::enqueueIterations(int n) {
     hipStream_t s = device().stream;
-    const bool prof = tun.profile != 0;
-    auto timed = [&](int k, auto&& launch) -> gp_status {
-        if (!prof) { launch(); return GP_OK; }
-        std::array<hipEvent_t, 2> ev;
-        GP_HIP(hipEventCreate(&ev[0]));
-        GP_HIP(hipEventCreate(&ev[1]));
-        GP_HIP(hipEventRecord(ev[0], s));
-        launch();
-        GP_HIP(hipEventRecord(ev[1], s));
-        pending[k].push_back(ev);
-        return GP_OK;
-    };
     gp_status st;
     for (int i = 0; i < n; ++i) {
-        const int cur = parity;
-        if ((st = timed(0, [&] { launchSchedule(q, cur, s); })) != GP_OK) return st;
-        if ((st = timed(1, [&] {
-                 if (q.emitOrder) launchEmitOrder(q, s);
-                 launchEmit(q, cur, ls, s);
-             })) != GP_OK)
-            return st;
-        if (q.binned)
-            if ((st = timed(5, [&] { launchBin(q, cur, s); })) != GP_OK) return st;
-        if ((st = timed(2, [&] { launchExtend(q, cur, ls, s); })) != GP_OK) return st;
-        if ((st = timed(3, [&] { launchShade(q, cur, ls, s); })) != GP_OK) return st;
-        if ((st = timed(4, [&] { launchConnect(q, ls, s); })) != GP_OK) return st;
-        if (mirrorActive && q.mv[0])
-            if ((st = timed(4, [&] { launchMirror(q, ls, s); })) != GP_OK) return st;
-        parity ^= 1;
+        if ((st = timed(0, [&] { launchSchedule(q, parity, s); })) != GP_OK) return st;
+        if ((st = enqueueEmit(ls)) != GP_OK) return st;
+        if ((st = enqueueBounce(ls)) != GP_OK) return st;
     }
     GP_HIP(hipGetLastError());
     return GP_OK;
@@ -678,7 +711,8 @@ gp_status Engine::runIterations(int n) {
 
 gp_status Engine::readCtrl() {
     hipStream_t s = device().stream;
-    GP_HIP(hipMemcpyAsync(hCtrl, dCtrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s));
+    GP_HIP(hipMemcpyAsync(hCtrl, dCtrl, kCtrlStride + sizeof(unsigned long long) * kSegs * kAccRow,
+                          hipMemcpyDeviceToHost, s));
     GP_HIP(hipStreamSynchronize(s));
     if (hCtrl->overflow) return fail(GP_ERR_CAPACITY, "wavefront queue segment overflow");
     if (tun.profile) return collectProfile();

@@ -104,6 +104,8 @@ double sceneMinDistance(const gp_scene& s, const double p[3]);
 // Kernel timing slots: schedule, emit, extend, shade, connect (+ mirror), binning.
 constexpr int kKernelSlots = 6;
 
+constexpr size_t kCtrlStride = (sizeof(Ctrl) + 255) & ~size_t(255);
+
 // Wavefront engine: device queues, control block, job table, graphs.
 struct Engine {
     std::mutex mu;
@@ -118,14 +120,11 @@ struct Engine {
     Ctrl* dCtrl = nullptr;
     Ctrl* hCtrl = nullptr;              // pinned
     DevJob* dJobs = nullptr;
-    DevJob* hJobs = nullptr;            // pinned
-    unsigned long long* dJobAcc = nullptr;       // kMaxJobs * kSegs * kAccRow
+    unsigned long long* dJobAcc = nullptr;       // kMaxJobs * kSegs * kAccRow, behind dCtrl
     DevCamera* dJobCams = nullptr;               // kMaxJobs * kMaxCams
-    DevCamera* hJobCams = nullptr;               // pinned staging for gp_trace
     int camCap = 1;                              // cameras per job the connection queue is sized for
-    gp_status resetJobAcc(int slot);             // zero a slot's rows (stream-ordered)
-    // ledger[5] and counters[kAccCounters] (the quantities from kAccPhotons on)
-    gp_status readJobAcc(int slot, unsigned long long ledger[5], unsigned long long* counters);
+    // job slot 0's accumulator rows as of the last readCtrl
+    const unsigned long long* traceRows() const { return (const unsigned long long*)((const char*)hCtrl + kCtrlStride); }
     void initCtrl();                            // zero the host control block, set capacities
     void* bufs[40] = {};
     int nbufs = 0;
@@ -160,6 +159,19 @@ struct Engine {
     void release();
     void releaseQueues();
     void releaseSpill();
+    template <class F>
+    gp_status timed(int k, F&& launch);
+    gp_status enqueueEmit(const LaunchShape& sh);
+    gp_status enqueueBounce(const LaunchShape& sh);
+    // Runs a trace whose n photons fit the path queue, from k_start_trace (once) to the
+    // last path's end; reads the control block and slot 0's rows back. Every live path
+    // advances one segment per iteration, so maxDepth iterations end it; the host looks
+    // for an earlier end every kOnceChunk. Grids are sized for n, and only the first
+    // iteration schedules and emits: with five kernels an iteration on grids for the full
+    // queue a 5000-photon render of the box spent 64 us an iteration on empty workgroups.
+    gp_status traceOnce(unsigned n, int cams, int maxDepth);
+    static constexpr int kOnceChunk = 32;
+    int onceIterations = 0;
     gp_status enqueueIterations(int n);       // plain launches, tracks parity
     gp_status runIterations(int n);           // graph replay when possible
     // Whether new photons are emitted in sorted order (set by the caller before
@@ -167,7 +179,7 @@ struct Engine {
     void setEmitOrder(uint64_t photons) {
         q.emitOrder = photons >= kEmitOrderJobMin && capacity >= kEmitOrderMin ? 1 : 0;
     }
-    gp_status readCtrl();                     // synchronous copy of the control block
+    gp_status readCtrl();                     // synchronous copy of the control block and slot 0's rows
 };
 Engine& engine();
 gp_tuning defaultTuning();

@@ -71,7 +71,7 @@ constexpr int kBinCellsPerAxis = 8;
 // each of the 4096 keys).
 constexpr int kEmitCols = 256;
 constexpr unsigned kEmitOrderMin = 1u << 16;
-constexpr uint64_t kEmitOrderJobMin = 1u << 21;
+constexpr uint64_t kEmitOrderJobMin = 1u << 19;
 
 // Leaf links are negative: ~((first << 3) | (count - 1)).
 inline constexpr int leafCode(int first, int count) { return ~((first << 3) | (count - 1)); }

@@ -410,7 +410,10 @@ typedef struct gp_tuning {
                                   the traversal kernels (persistent threads)         */
     int32_t iters_per_graph; /* iterations per host read of the wavefront state (per
                                 captured hipGraph: even, 2..64; 1..64 without graphs) */
-    int32_t use_graph;       /* 1 = replay captured graphs, 0 = plain launches       */
+    int32_t use_graph;       /* 1 = replay captured graphs, 0 = plain launches (a trace
+                                that fits the path queue always runs plain launches
+                                on grids of its own size, read back every 32
+                                iterations)                                          */
     int32_t lds_stack;       /* traversal stack entries per lane held in LDS: 8, 12,
                                 16, 24 or 32 (default 12; deeper entries spill to
                                 global memory)                                       */
