@@ -196,23 +196,28 @@ static gp_status createScene(const gp_scene_desc* d, int builder, gp_scene** out
         if ((st = validateSpectrum(m.ior, "ior", d)) != GP_OK) return st;
         if (!std::isfinite(m.roughness)) return fail(GP_ERR_INVALID, "non-finite roughness");
     }
-    for (int64_t i = 0; i < d->n_tris; ++i) {
-        if (d->mat_ids[i] < 0 || d->mat_ids[i] >= d->n_materials)
-            return fail(GP_ERR_INVALID, "triangle material id out of range");
+    gp_status st;
+    DeviceTris dtris;
+    if (builder == GP_BVH_DEVICE_LBVH && requireDevice() == GP_OK) {
+        // uploaded as they are, checked and bounded there
+        if ((st = scanTrisDevice(d->verts, d->mat_ids, d->n_tris, d->n_materials, dtris)) != GP_OK) return st;
+    } else {
+        for (int64_t i = 0; i < d->n_tris; ++i) {
+            if (d->mat_ids[i] < 0 || d->mat_ids[i] >= d->n_materials)
+                return fail(GP_ERR_INVALID, "triangle material id out of range");
+        }
+        for (int64_t i = 0; i < 9 * d->n_tris; ++i)
+            if (!std::isfinite(d->verts[i])) return fail(GP_ERR_INVALID, "non-finite vertex");
     }
-    for (int64_t i = 0; i < 9 * d->n_tris; ++i)
-        if (!std::isfinite(d->verts[i])) return fail(GP_ERR_INVALID, "non-finite vertex");
     for (int i = 0; i < d->n_emitters; ++i) {
         const gp_emitter& e = d->emitters[i];
         if (!finite3(e.origin) || !finite3(e.u) || !finite3(e.v) || !finite3(e.normal) || !(e.area > 0.0))
             return fail(GP_ERR_INVALID, "bad emitter geometry");
-        gp_status st = validateSpectrum(e.spd, "emitter spd", d);
-        if (st != GP_OK) return st;
+        if ((st = validateSpectrum(e.spd, "emitter spd", d)) != GP_OK) return st;
     }
     if (builder == GP_BVH_PREBUILT && (!d->bvh_nodes || d->n_bvh_nodes <= 0 || !d->bvh_prim_index ||
                                        d->n_bvh_prim_index <= 0))
         return fail(GP_ERR_INVALID, "GP_BVH_PREBUILT needs bvh_nodes and bvh_prim_index");
-    gp_status st;
     // the device builder needs the device now; the host trees are built (and a
     // caller's tree checked) first
     if (builder == GP_BVH_DEVICE_LBVH && (st = requireDevice()) != GP_OK) return st;
@@ -221,7 +226,7 @@ static gp_status createScene(const gp_scene_desc* d, int builder, gp_scene** out
     s->nTris = d->n_tris;
     s->builder = builder;
     const size_t n = (size_t)d->n_tris;
-    std::vector<float4> tris(3 * n), trin(n);
+    std::vector<float4> tris, trin;   // leaf order (host-built trees)
     auto fillTri = [&](size_t k, int prim) {
         const float* v = d->verts + 9 * (size_t)prim;
         const int mat = d->mat_ids[prim];
@@ -238,30 +243,11 @@ static gp_status createScene(const gp_scene_desc* d, int builder, gp_scene** out
         trin[k] = make_float4((float)c[0], (float)c[1], (float)c[2], 0.f);
         std::memcpy(&trin[k].w, &mat, 4);
     };
-    {
-        // ray-binning grid: kBinCellsPerAxis cells per axis over the centroid box
-        float blo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, bhi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-        for (size_t k = 0; k < n; ++k) {
-            const float* v = d->verts + 9 * k;
-            for (int a = 0; a < 3; ++a) {
-                const float c = 0.5f * (std::min({v[a], v[3 + a], v[6 + a]}) + std::max({v[a], v[3 + a], v[6 + a]}));
-                blo[a] = std::min(blo[a], c);
-                bhi[a] = std::max(bhi[a], c);
-            }
-        }
-        for (int a = 0; a < 3; ++a) {
-            const float ext = bhi[a] - blo[a];
-            s->binLo[a] = blo[a];
-            s->binScale[a] = (ext > 0.f && std::isfinite(ext)) ? (float)kBinCellsPerAxis / ext : 0.f;
-        }
-    }
-    DeviceBvh dbvh;
-    std::vector<float> quads;   // four-wide nodes of the host-built tree
+    float clo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, chi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     if (builder == GP_BVH_DEVICE_LBVH) {
-        // input order; the device sorts, builds and gathers
-        float clo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, chi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+        for (int a = 0; a < 3; ++a) { clo[a] = dtris.centerLo[a]; chi[a] = dtris.centerHi[a]; }
+    } else {
         for (size_t k = 0; k < n; ++k) {
-            fillTri(k, (int)k);
             const float* v = d->verts + 9 * k;
             for (int a = 0; a < 3; ++a) {
                 const float c = 0.5f * (std::min({v[a], v[3 + a], v[6 + a]}) + std::max({v[a], v[3 + a], v[6 + a]}));
@@ -269,13 +255,17 @@ static gp_status createScene(const gp_scene_desc* d, int builder, gp_scene** out
                 chi[a] = std::max(chi[a], c);
             }
         }
-        DevBuf dIn, dInN;
-        GP_HIP(hipMalloc(&dIn.p, tris.size() * sizeof(float4)));
-        GP_HIP(hipMalloc(&dInN.p, trin.size() * sizeof(float4)));
-        GP_HIP(hipMemcpy(dIn.p, tris.data(), tris.size() * sizeof(float4), hipMemcpyHostToDevice));
-        GP_HIP(hipMemcpy(dInN.p, trin.data(), trin.size() * sizeof(float4), hipMemcpyHostToDevice));
-        if ((st = buildBvhDevice((const float4*)dIn.p, (const float4*)dInN.p, d->n_tris, clo, chi, dbvh)) != GP_OK)
-            return st;
+    }
+    for (int a = 0; a < 3; ++a) {
+        // ray-binning grid: kBinCellsPerAxis cells per axis over the centroid box
+        const float ext = chi[a] - clo[a];
+        s->binLo[a] = clo[a];
+        s->binScale[a] = (ext > 0.f && std::isfinite(ext)) ? (float)kBinCellsPerAxis / ext : 0.f;
+    }
+    DeviceBvh dbvh;
+    std::vector<float> quads;   // four-wide nodes of the host-built tree
+    if (builder == GP_BVH_DEVICE_LBVH) {
+        if ((st = buildBvhDevice(dtris, dbvh)) != GP_OK) return st;
         s->nNodes = dbvh.nPairs;
         s->depth = dbvh.depth;
         s->stackNeed = dbvh.stackNeed;

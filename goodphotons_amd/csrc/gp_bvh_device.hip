@@ -2,16 +2,22 @@
 // construction of BVHs, octrees, and k-d trees", HPG 2012) emitted in the child-pair
 // layout and collapsed into the four-wide nodes the traversal reads.
 //
+// The vertices and material ids are uploaded as the caller holds them; one kernel checks
+// them and reduces the bounds of the box centres (scanTrisDevice), and the tree's kernels
+// read them from there.
+//
 //   1. Morton code (21 bits per axis) of each triangle's box centre in the scene's
 //      centre bounds; sort (code, index) pairs (rocPRIM radix sort).
 //   2. One thread per internal node i finds the sorted range it covers and its split
 //      from the longest common prefixes of neighbouring codes (equal codes are told
 //      apart by their positions, so the tree is a valid binary tree for any input).
-//   3. Boxes and heights bottom-up: one thread per primitive climbs from its leaf; at
-//      each node the first arriving child stops, the second computes the union.
+//   3. Every node covers a contiguous sorted range, so its box is the union of a few
+//      entries of a binary tree of boxes over the sorted leaves (a segment tree built a
+//      workgroup at a time): no node waits for its children.
 //   4. Every internal node whose range holds more than kLeafMax primitives becomes a
 //      pair node; a child with at most kLeafMax primitives becomes a leaf over its
-//      contiguous sorted range. Triangles are gathered into sorted (leaf) order.
+//      contiguous sorted range. Triangles are gathered into sorted (leaf) order,
+//      with their normals.
 //   5. Pair node i becomes four-wide node i, whose slots are its grandchildren (a
 //      leaf child keeps its own slot), so links keep their indices; the root is
 //      node 0, and nodes at odd pair levels are built but never reached.
@@ -26,6 +32,7 @@
 #include <cfloat>
 #include <chrono>
 #include <cmath>
+#include <cstring>
 
 #include "gp_bvh_device.hpp"
 #include "gp_runtime.hpp"
@@ -60,24 +67,62 @@ __device__ __forceinline__ float roundUp(double v) {
     return ((double)f < v) ? nextafterf(f, FLT_MAX) : f;
 }
 
-// Padded box of input triangle t (float4 x3 per triangle, input order).
-__device__ __forceinline__ void triBox(const float4* __restrict__ tris, int t, float lo[3], float hi[3]) {
-    const float4 a = tris[3 * t], b = tris[3 * t + 1], c = tris[3 * t + 2];
-    const float va[3] = {a.x, a.y, a.z}, vb[3] = {b.x, b.y, b.z}, vc[3] = {c.x, c.y, c.z};
+// Padded box of input triangle t (nine floats per triangle, input order).
+__device__ __forceinline__ void triBox(const float* __restrict__ verts, int t, float lo[3], float hi[3]) {
+    const float* v = verts + 9 * (size_t)t;
     for (int k = 0; k < 3; ++k) {
-        const double l = fmin(fmin((double)va[k], (double)vb[k]), (double)vc[k]) - kPadD;
-        const double h = fmax(fmax((double)va[k], (double)vb[k]), (double)vc[k]) + kPadD;
+        const double l = fmin(fmin((double)v[k], (double)v[3 + k]), (double)v[6 + k]) - kPadD;
+        const double h = fmax(fmax((double)v[k], (double)v[3 + k]), (double)v[6 + k]) + kPadD;
         lo[k] = roundDown(l);
         hi[k] = roundUp(h);
     }
 }
 
-__global__ void k_morton(const float4* __restrict__ tris, int n, float3 lo, float3 inv,
+// Unsigned words that order like the floats.
+__device__ __forceinline__ unsigned orderedBits(float f) {
+    const unsigned u = (unsigned)__float_as_int(f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// Checks the triangles and reduces the bounds of their box centres into out[7] (zeroed):
+// maxima of the complemented ordered lower bounds, of the ordered upper bounds, and flags
+// (1: a material id out of range, 2: a vertex that is not finite). Reads 40 bytes a
+// triangle once. The host loops over the same data, with the 64 bytes a triangle that they
+// prepared and uploaded, took 8 of the 12.7 ms of a 400,000-triangle rebuild. At most 256
+// workgroups, so that the seven same-address atomics of each stay under 20 us.
+__global__ void __launch_bounds__(256) k_scan_tris(const float* __restrict__ verts, const int* __restrict__ mats,
+                                                   size_t n, int nMats, unsigned* __restrict__ out) {
+    __shared__ unsigned red[7];
+    if (threadIdx.x < 7) red[threadIdx.x] = 0u;
+    __syncthreads();
+    unsigned r[6] = {0u, 0u, 0u, 0u, 0u, 0u}, flags = 0u;
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
+        const float* v = verts + 9 * t;
+        const int m = mats[t];
+        if (m < 0 || m >= nMats) flags |= 1u;
+        for (int k = 0; k < 3; ++k) {
+            const float a = v[k], b = v[3 + k], c = v[6 + k];
+            if (!(fabsf(a) <= FLT_MAX && fabsf(b) <= FLT_MAX && fabsf(c) <= FLT_MAX)) flags |= 2u;
+            const float ctr = 0.5f * (fminf(fminf(a, b), c) + fmaxf(fmaxf(a, b), c));
+            const unsigned u = orderedBits(ctr);
+            r[k] = max(r[k], ~u);
+            r[3 + k] = max(r[3 + k], u);
+        }
+    }
+    for (int k = 0; k < 6; ++k) atomicMax(&red[k], r[k]);
+    if (flags) atomicOr(&red[6], flags);
+    __syncthreads();
+    if (threadIdx.x < 6) atomicMax(&out[threadIdx.x], red[threadIdx.x]);
+    if (threadIdx.x == 6 && red[6]) atomicOr(&out[6], red[6]);
+}
+
+__global__ void k_morton(const float* __restrict__ verts, int n, float3 lo, float3 inv,
                          unsigned long long* __restrict__ keys, unsigned* __restrict__ vals) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float bl[3], bh[3];
-    triBox(tris, i, bl, bh);
+    triBox(verts, i, bl, bh);
     const float cx = 0.5f * (bl[0] + bh[0]), cy = 0.5f * (bl[1] + bh[1]), cz = 0.5f * (bl[2] + bh[2]);
     auto q = [](float c, float l, float s) {
         float u = (c - l) * s;
@@ -98,7 +143,7 @@ __device__ __forceinline__ int lcp(const unsigned long long* __restrict__ k, int
 }
 
 __global__ void k_karras(const unsigned long long* __restrict__ keys, int n, KNode* __restrict__ nodes,
-                         int* __restrict__ parentInner, int* __restrict__ parentLeaf) {
+                         int* __restrict__ parent) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
     const int d = (lcp(keys, n, i, i + 1) - lcp(keys, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -121,75 +166,118 @@ __global__ void k_karras(const unsigned long long* __restrict__ keys, int n, KNo
     nd.last = max(i, j);
     if (nd.first == gamma) {
         nd.left = -(gamma + 1);
-        parentLeaf[gamma] = i;
     } else {
         nd.left = gamma;
-        parentInner[gamma] = i;
+        parent[gamma] = i;
     }
     if (nd.last == gamma + 1) {
         nd.right = -(gamma + 2);
-        parentLeaf[gamma + 1] = i;
     } else {
         nd.right = gamma + 1;
-        parentInner[gamma + 1] = i;
+        parent[gamma + 1] = i;
     }
+    if (i == 0) parent[0] = -1;   // the root is no node's child
     nodes[i] = nd;
 }
 
-__device__ __forceinline__ float aload(const float* p) {
-    return __int_as_float(__hip_atomic_load((const int*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-__device__ __forceinline__ int aloadi(const int* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// box[6] per leaf (sorted position) and per internal node; height per internal node
-// (pair-node levels below and including it; 0 for ranges of <= kLeafMax primitives)
-__global__ void k_leaf_boxes(const float4* __restrict__ tris, const unsigned* __restrict__ order, int n,
+// box[6] of every sorted leaf
+__global__ void k_leaf_boxes(const float* __restrict__ verts, const unsigned* __restrict__ order, int n,
                              float* __restrict__ leafBox) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     float lo[3], hi[3];
-    triBox(tris, (int)order[k], lo, hi);
+    triBox(verts, (int)order[k], lo, hi);
     for (int a = 0; a < 3; ++a) {
-        leafBox[6 * k + a] = lo[a];
-        leafBox[6 * k + 3 + a] = hi[a];
+        leafBox[6 * (size_t)k + a] = lo[a];
+        leafBox[6 * (size_t)k + 3 + a] = hi[a];
     }
 }
 
-__global__ void k_refit(const KNode* __restrict__ nodes, const int* __restrict__ parentInner,
-                        const int* __restrict__ parentLeaf, int n, const float* __restrict__ leafBox,
-                        float* __restrict__ box, int* __restrict__ height, unsigned* __restrict__ arrivals) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int p = parentLeaf[k];
-    while (p >= 0) {
-        __threadfence();
-        if (atomicAdd(&arrivals[p], 1u) == 0u) return;   // the sibling subtree is still open
-        __threadfence();
-        const KNode nd = nodes[p];
-        float lo[3], hi[3];
-        int h = 0;
-        for (int side = 0; side < 2; ++side) {
-            const int c = side ? nd.right : nd.left;
-            const float* b = c < 0 ? leafBox + 6 * (size_t)(-c - 1) : box + 6 * (size_t)c;
-            for (int a = 0; a < 3; ++a) {
-                const float l = aload(b + a), u = aload(b + 3 + a);
-                lo[a] = side ? fminf(lo[a], l) : l;
-                hi[a] = side ? fmaxf(hi[a], u) : u;
-            }
-            if (c >= 0) {
-                const KNode cn = nodes[c];
-                if (cn.last - cn.first + 1 > kLeafMax) h = max(h, aloadi(height + c));
-            }
-        }
-        for (int a = 0; a < 3; ++a) {
-            box[6 * (size_t)p + a] = lo[a];
-            box[6 * (size_t)p + 3 + a] = hi[a];
-        }
-        height[p] = (nd.last - nd.first + 1 > kLeafMax) ? h + 1 : 0;
-        p = parentInner[p];
+// Binary tree of boxes over the sorted leaves: entry i of level k is the union of the
+// leaves [i 2^k, (i + 1) 2^k) below n. Level 0 is leafBox; level k >= 1 starts at off[k].
+constexpr int kMaxLevels = 30;   // triangles < 2^28
+struct BoxLevels {
+    unsigned size[kMaxLevels];
+    unsigned off[kMaxLevels];
+    int count;
+};
+
+__device__ __forceinline__ void growBox(float b[6], const float* __restrict__ p) {
+    for (int a = 0; a < 3; ++a) {
+        b[a] = fminf(b[a], p[a]);
+        b[3 + a] = fmaxf(b[3 + a], p[3 + a]);
     }
+}
+
+// Levels base + 1 .. base + kBoxStep from level `base`: a workgroup folds 2^kBoxStep
+// entries, level by level, through LDS.
+constexpr int kBoxStep = 9;
+__global__ void __launch_bounds__(1 << (kBoxStep - 1)) k_box_levels(BoxLevels L, int base,
+                                                                  const float* __restrict__ leafBox,
+                                                                  float* __restrict__ up) {
+    __shared__ float sh[1 << (kBoxStep - 1)][6];
+    const float* src = base ? up + 6 * (size_t)L.off[base] : leafBox;
+    const unsigned t = threadIdx.x;
+    for (int s = 1; s <= kBoxStep && base + s < L.count; ++s) {
+        const unsigned width = 1u << (kBoxStep - s);          // entries of level base + s here
+        const unsigned e = blockIdx.x * width + t;            // entry of that level
+        const bool have = t < width && e < L.size[base + s];
+        float b[6];
+        if (have) {
+            const bool two = 2 * e + 1 < L.size[base + s - 1];
+            const float* l = s == 1 ? src + 12 * (size_t)e : sh[2 * t];
+            for (int a = 0; a < 6; ++a) b[a] = l[a];
+            if (two) growBox(b, s == 1 ? l + 6 : sh[2 * t + 1]);
+        }
+        __syncthreads();   // the level below is read
+        if (have) {
+            float* o = up + 6 * (size_t)(L.off[base + s] + e);
+            for (int a = 0; a < 6; ++a) { sh[t][a] = b[a]; o[a] = b[a]; }
+        }
+        __syncthreads();
+    }
+}
+
+// Box of every internal node: the union over its sorted range, at most two entries of
+// each level. A climb from the leaves in which the second child to arrive merges the boxes
+// needs a device-wide fence at each node, which writes back an XCD's whole L2: 2500 us for
+// 400,000 triangles, against 14 us for this, 17 us for the levels and 28 us for k_height.
+__global__ void k_node_boxes(BoxLevels L, const KNode* __restrict__ nodes, int nInner,
+                             const float* __restrict__ leafBox, const float* __restrict__ up,
+                             float* __restrict__ box) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nInner) return;
+    const KNode nd = nodes[i];
+    float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    unsigned l = (unsigned)nd.first, r = (unsigned)nd.last + 1u;
+    for (int k = 0; l < r; ++k, l >>= 1, r >>= 1) {
+        const float* lev = k ? up + 6 * (size_t)L.off[k] : leafBox;
+        if (l & 1u) growBox(b, lev + 6 * (size_t)l++);
+        if (r & 1u) growBox(b, lev + 6 * (size_t)--r);
+    }
+    for (int a = 0; a < 6; ++a) box[6 * (size_t)i + a] = b[a];
+}
+
+// Pair-node levels of the tree: the longest chain of ancestors above a pair node without
+// pair-node children. height[0] (zeroed) receives the maximum.
+__global__ void __launch_bounds__(256) k_height(const KNode* __restrict__ nodes, const int* __restrict__ parent,
+                                                int nInner, int* __restrict__ height) {
+    __shared__ int best;
+    if (threadIdx.x == 0) best = 0;
+    __syncthreads();
+    auto isPair = [&](int c) { return c >= 0 && nodes[c].last - nodes[c].first + 1 > kLeafMax; };
+    int mine = 0;
+    const int stride = (int)(gridDim.x * blockDim.x);
+    for (int64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nInner; i += stride) {
+        const KNode nd = nodes[i];
+        if (nd.last - nd.first + 1 <= kLeafMax || isPair(nd.left) || isPair(nd.right)) continue;
+        int h = 0;
+        for (int p = (int)i; p >= 0; p = parent[p]) ++h;
+        mine = max(mine, h);
+    }
+    if (mine) atomicMax(&best, mine);
+    __syncthreads();
+    if (threadIdx.x == 0 && best) atomicMax(height, best);
 }
 
 __device__ __forceinline__ int childLink(const KNode* __restrict__ nodes, int c) {
@@ -276,16 +364,26 @@ __global__ void k_lone_leaf(const float* __restrict__ leafBox, int n, float4* __
     pairs[3] = make_float4(hi[0], hi[1], hi[2], 0.0f);
 }
 
-__global__ void k_gather(const float4* __restrict__ trisIn, const float4* __restrict__ trinIn,
+// Triangles and their geometric normals in sorted order, from the input arrays (the
+// normal as the host builder's scene upload computes it: in double, no contraction).
+__global__ void k_gather(const float* __restrict__ verts, const int* __restrict__ mats,
                          const unsigned* __restrict__ order, int n, float4* __restrict__ tris,
                          float4* __restrict__ trin) {
+#pragma clang fp contract(off)
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    const unsigned t = order[k];
-    tris[3 * (size_t)k + 0] = trisIn[3 * (size_t)t + 0];
-    tris[3 * (size_t)k + 1] = trisIn[3 * (size_t)t + 1];
-    tris[3 * (size_t)k + 2] = trisIn[3 * (size_t)t + 2];
-    trin[k] = trinIn[t];
+    const int t = (int)order[k];
+    const float* v = verts + 9 * (size_t)t;
+    const float mat = __int_as_float(mats[t]);
+    tris[3 * (size_t)k + 0] = make_float4(v[0], v[1], v[2], __int_as_float(t));
+    tris[3 * (size_t)k + 1] = make_float4(v[3], v[4], v[5], mat);
+    tris[3 * (size_t)k + 2] = make_float4(v[6], v[7], v[8], 0.f);
+    const double e1[3] = {(double)v[3] - v[0], (double)v[4] - v[1], (double)v[5] - v[2]};
+    const double e2[3] = {(double)v[6] - v[0], (double)v[7] - v[1], (double)v[8] - v[2]};
+    double c[3] = {e1[1] * e2[2] - e1[2] * e2[1], e1[2] * e2[0] - e1[0] * e2[2], e1[0] * e2[1] - e1[1] * e2[0]};
+    const double l = sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
+    if (l > 0) { c[0] /= l; c[1] /= l; c[2] /= l; } else { c[0] = 0; c[1] = 0; c[2] = 1; }
+    trin[k] = make_float4((float)c[0], (float)c[1], (float)c[2], mat);
 }
 
 // ---- eye-to-scene distance (brute force, double; Ericson 5.1.5)
@@ -361,110 +459,153 @@ int blocks(int64_t n) { return (int)std::max<int64_t>(1, (n + 255) / 256); }
 
 }  // namespace
 
-gp_status buildBvhDevice(const float4* dTrisIn, const float4* dTrinIn, int64_t n64, const float centerLo[3],
-                         const float centerHi[3], DeviceBvh& out) {
-    hipStream_t s = device().stream;
-    const int n = (int)n64;
-    auto t0 = std::chrono::steady_clock::now();
-    auto alloc = [&](DevBuf& b, size_t bytes) -> gp_status {
-        hipError_t e = hipMalloc(&b.p, std::max<size_t>(bytes, 16));
-        if (e != hipSuccess) return fail(GP_ERR_OOM, std::string("BVH build: hipMalloc: ") + hipGetErrorString(e));
-        return GP_OK;
-    };
-    gp_status st;
-    DevBuf keys, keys2, vals, vals2, leafBox;
-    if ((st = alloc(keys, sizeof(unsigned long long) * n)) != GP_OK) return st;
-    if ((st = alloc(keys2, sizeof(unsigned long long) * n)) != GP_OK) return st;
-    if ((st = alloc(vals, sizeof(unsigned) * n)) != GP_OK) return st;
-    if ((st = alloc(vals2, sizeof(unsigned) * n)) != GP_OK) return st;
-    if ((st = alloc(leafBox, sizeof(float) * 6 * (size_t)n)) != GP_OK) return st;
-    float3 lo = make_float3(centerLo[0], centerLo[1], centerLo[2]);
-    auto invExt = [](float l, float h) { return h > l ? 1.0f / (h - l) : 0.0f; };
-    float3 inv = make_float3(invExt(centerLo[0], centerHi[0]), invExt(centerLo[1], centerHi[1]),
-                             invExt(centerLo[2], centerHi[2]));
-    hipLaunchKernelGGL(k_morton, dim3(blocks(n)), dim3(256), 0, s, dTrisIn, n, lo, inv,
-                       (unsigned long long*)keys.p, (unsigned*)vals.p);
-    GP_HIP(hipGetLastError());
-    size_t tempBytes = 0;
-    GP_HIP(rocprim::radix_sort_pairs(nullptr, tempBytes, (unsigned long long*)keys.p, (unsigned long long*)keys2.p,
-                                     (unsigned*)vals.p, (unsigned*)vals2.p, (size_t)n, 0u, 63u, s));
-    DevBuf temp;
-    if ((st = alloc(temp, tempBytes)) != GP_OK) return st;
-    GP_HIP(rocprim::radix_sort_pairs(temp.p, tempBytes, (unsigned long long*)keys.p, (unsigned long long*)keys2.p,
-                                     (unsigned*)vals.p, (unsigned*)vals2.p, (size_t)n, 0u, 63u, s));
-    const unsigned long long* skeys = (const unsigned long long*)keys2.p;
-    const unsigned* order = (const unsigned*)vals2.p;
-    hipLaunchKernelGGL(k_leaf_boxes, dim3(blocks(n)), dim3(256), 0, s, dTrisIn, order, n, (float*)leafBox.p);
-    GP_HIP(hipGetLastError());
+DeviceTris::~DeviceTris() {
+    if (verts) hipFree(verts);
+}
 
-    const size_t nPairs = (size_t)std::max(1, n - 1);
-    float4* pairs = nullptr;
-    {
-        hipError_t e = hipMalloc((void**)&pairs, nPairs * 4 * sizeof(float4));
-        if (e != hipSuccess) return fail(GP_ERR_OOM, "BVH build: node allocation failed");
+gp_status scanTrisDevice(const float* verts, const int32_t* mats, int64_t n, int nMats, DeviceTris& out) {
+    hipStream_t s = device().stream;
+    const size_t vb = sizeof(float) * 9 * (size_t)n, mb = sizeof(int32_t) * (size_t)n;
+    const size_t words = ((vb + mb + 255) & ~size_t(255));   // the reduced words behind both arrays
+    hipError_t e = hipMalloc((void**)&out.verts, words + 8 * sizeof(unsigned));
+    if (e != hipSuccess) {
+        out.verts = nullptr;
+        return fail(GP_ERR_OOM, std::string("scene upload: hipMalloc: ") + hipGetErrorString(e));
     }
-    struct PairsGuard {
-        float4*& p;
-        bool keep = false;
-        ~PairsGuard() { if (!keep && p) hipFree(p); }
-    } pg{pairs};
-    float4* quads = nullptr;
-    {
-        hipError_t e = hipMalloc((void**)&quads, nPairs * 8 * sizeof(float4));
-        if (e != hipSuccess) return fail(GP_ERR_OOM, "BVH build: node allocation failed");
+    out.mats = (int32_t*)((char*)out.verts + vb);
+    out.n = n;
+    unsigned* red = (unsigned*)((char*)out.verts + words);
+    GP_HIP(hipMemcpyAsync(out.verts, verts, vb, hipMemcpyHostToDevice, s));
+    GP_HIP(hipMemcpyAsync(out.mats, mats, mb, hipMemcpyHostToDevice, s));
+    launchFill64((unsigned long long*)red, 4, 0ull, s);
+    hipLaunchKernelGGL(k_scan_tris, dim3(std::min(256, blocks(n))), dim3(256), 0, s, (const float*)out.verts,
+                       (const int*)out.mats, (size_t)n, nMats, red);
+    GP_HIP(hipGetLastError());
+    unsigned r[8];
+    GP_HIP(hipMemcpyAsync(r, red, sizeof r, hipMemcpyDeviceToHost, s));
+    GP_HIP(hipStreamSynchronize(s));
+    if (r[6] & 1u) return fail(GP_ERR_INVALID, "triangle material id out of range");
+    if (r[6] & 2u) return fail(GP_ERR_INVALID, "non-finite vertex");
+    auto toFloat = [](unsigned u) {
+        u = (u & 0x80000000u) ? (u & 0x7fffffffu) : ~u;
+        float f;
+        std::memcpy(&f, &u, sizeof f);
+        return f;
+    };
+    for (int a = 0; a < 3; ++a) {
+        out.centerLo[a] = toFloat(~r[a]);
+        out.centerHi[a] = toFloat(r[3 + a]);
     }
-    PairsGuard qg{quads};
-    int height = 1;
-    if (n <= kLeafMax) {
-        hipLaunchKernelGGL(k_lone_leaf, dim3(1), dim3(64), 0, s, (const float*)leafBox.p, n, pairs);
-        hipLaunchKernelGGL(k_collapse4, dim3(1), dim3(64), 0, s, (const KNode*)nullptr, 1, (const float4*)pairs,
-                           quads);
-        GP_HIP(hipGetLastError());
-    } else {
-        DevBuf nodes, parentInner, parentLeaf, box, heights, arrivals;
-        if ((st = alloc(nodes, sizeof(KNode) * (size_t)(n - 1))) != GP_OK) return st;
-        if ((st = alloc(parentInner, sizeof(int) * (size_t)(n - 1))) != GP_OK) return st;
-        if ((st = alloc(parentLeaf, sizeof(int) * (size_t)n)) != GP_OK) return st;
-        if ((st = alloc(box, sizeof(float) * 6 * (size_t)(n - 1))) != GP_OK) return st;
-        if ((st = alloc(heights, sizeof(int) * (size_t)(n - 1))) != GP_OK) return st;
-        if ((st = alloc(arrivals, sizeof(unsigned) * (size_t)(n - 1))) != GP_OK) return st;
-        GP_HIP(hipMemsetAsync(arrivals.p, 0, sizeof(unsigned) * (size_t)(n - 1), s));
-        GP_HIP(hipMemsetAsync(parentInner.p, 0xff, sizeof(int) * (size_t)(n - 1), s));   // root: -1
-        hipLaunchKernelGGL(k_karras, dim3(blocks(n - 1)), dim3(256), 0, s, skeys, n, (KNode*)nodes.p,
-                           (int*)parentInner.p, (int*)parentLeaf.p);
-        hipLaunchKernelGGL(k_refit, dim3(blocks(n)), dim3(256), 0, s, (const KNode*)nodes.p,
-                           (const int*)parentInner.p, (const int*)parentLeaf.p, n, (const float*)leafBox.p,
-                           (float*)box.p, (int*)heights.p, (unsigned*)arrivals.p);
-        hipLaunchKernelGGL(k_emit_pairs, dim3(blocks(n - 1)), dim3(256), 0, s, (const KNode*)nodes.p, n,
-                           (const float*)leafBox.p, (const float*)box.p, pairs);
-        hipLaunchKernelGGL(k_collapse4, dim3(blocks(n - 1)), dim3(256), 0, s, (const KNode*)nodes.p, n - 1,
-                           (const float4*)pairs, quads);
-        GP_HIP(hipGetLastError());
-        GP_HIP(hipMemcpyAsync(&height, heights.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    return GP_OK;
+}
+
+gp_status buildBvhDevice(const DeviceTris& in, DeviceBvh& out) {
+    hipStream_t s = device().stream;
+    const int n = (int)in.n;
+    auto t0 = std::chrono::steady_clock::now();
+    float3 lo = make_float3(in.centerLo[0], in.centerLo[1], in.centerLo[2]);
+    auto invExt = [](float l, float h) { return h > l ? 1.0f / (h - l) : 0.0f; };
+    float3 inv = make_float3(invExt(in.centerLo[0], in.centerHi[0]), invExt(in.centerLo[1], in.centerHi[1]),
+                             invExt(in.centerLo[2], in.centerHi[2]));
+    const size_t inner = (size_t)std::max(1, n - 1);
+    BoxLevels L{};
+    unsigned upper = 0;
+    L.size[0] = (unsigned)n;
+    L.count = 1;
+    while (L.size[L.count - 1] > 1) {
+        L.size[L.count] = (L.size[L.count - 1] + 1) / 2;
+        L.off[L.count] = upper;
+        upper += L.size[L.count++];
     }
-    float4 *tris = nullptr, *trin = nullptr;
+    size_t tempBytes = 0;
+    GP_HIP(rocprim::radix_sort_pairs(nullptr, tempBytes, (unsigned long long*)nullptr, (unsigned long long*)nullptr,
+                                     (unsigned*)nullptr, (unsigned*)nullptr, (size_t)n, 0u, 63u, s));
+    // one allocation holds every temporary (a dozen allocations and frees of their own took
+    // more than the tree's kernels)
+    size_t need = 0;
+    auto part = [&](size_t bytes) {
+        const size_t at = need;
+        need += (std::max<size_t>(bytes, 16) + 255) & ~size_t(255);
+        return at;
+    };
+    const size_t oKeys = part(sizeof(unsigned long long) * n), oKeys2 = part(sizeof(unsigned long long) * n);
+    const size_t oVals = part(sizeof(unsigned) * n), oVals2 = part(sizeof(unsigned) * n);
+    const size_t oLeaf = part(sizeof(float) * 6 * (size_t)n), oUp = part(sizeof(float) * 6 * (size_t)upper);
+    const size_t oNodes = part(sizeof(KNode) * inner), oParent = part(sizeof(int) * inner);
+    const size_t oBox = part(sizeof(float) * 6 * inner), oPairs = part(sizeof(float4) * 4 * inner);
+    const size_t oHeight = part(sizeof(unsigned long long)), oTemp = part(tempBytes);
+    DevBuf arena;
     {
-        hipError_t e1 = hipMalloc((void**)&tris, sizeof(float4) * 3 * (size_t)n);
-        hipError_t e2 = hipMalloc((void**)&trin, sizeof(float4) * (size_t)n);
-        if (e1 != hipSuccess || e2 != hipSuccess) {
-            if (tris) hipFree(tris);
-            if (trin) hipFree(trin);
-            return fail(GP_ERR_OOM, "BVH build: triangle allocation failed");
+        hipError_t e = hipMalloc(&arena.p, need);
+        if (e != hipSuccess) {
+            arena.p = nullptr;
+            return fail(GP_ERR_OOM, std::string("BVH build: hipMalloc: ") + hipGetErrorString(e));
         }
     }
-    hipLaunchKernelGGL(k_gather, dim3(blocks(n)), dim3(256), 0, s, dTrisIn, dTrinIn, order, n, tris, trin);
+    auto at = [&](size_t o) { return (void*)((char*)arena.p + o); };
+    unsigned long long *keys = (unsigned long long*)at(oKeys), *skeys = (unsigned long long*)at(oKeys2);
+    unsigned *vals = (unsigned*)at(oVals), *order = (unsigned*)at(oVals2);
+    float *leafBox = (float*)at(oLeaf), *up = (float*)at(oUp), *box = (float*)at(oBox);
+    float4* pairs = (float4*)at(oPairs);
+    hipLaunchKernelGGL(k_morton, dim3(blocks(n)), dim3(256), 0, s, (const float*)in.verts, n, lo, inv, keys, vals);
+    GP_HIP(hipGetLastError());
+    GP_HIP(rocprim::radix_sort_pairs(at(oTemp), tempBytes, keys, skeys, vals, order, (size_t)n, 0u, 63u, s));
+    hipLaunchKernelGGL(k_leaf_boxes, dim3(blocks(n)), dim3(256), 0, s, (const float*)in.verts, (const unsigned*)order,
+                       n, leafBox);
+    GP_HIP(hipGetLastError());
+
+    struct Out {
+        void* p = nullptr;
+        bool keep = false;
+        ~Out() { if (!keep && p) hipFree(p); }
+    } quads, tris, trin;
+    if (hipMalloc(&quads.p, inner * 8 * sizeof(float4)) != hipSuccess) {
+        quads.p = nullptr;
+        return fail(GP_ERR_OOM, "BVH build: node allocation failed");
+    }
+    int height = 1;
+    if (n <= kLeafMax) {
+        hipLaunchKernelGGL(k_lone_leaf, dim3(1), dim3(64), 0, s, (const float*)leafBox, n, pairs);
+        hipLaunchKernelGGL(k_collapse4, dim3(1), dim3(64), 0, s, (const KNode*)nullptr, 1, (const float4*)pairs,
+                           (float4*)quads.p);
+        GP_HIP(hipGetLastError());
+    } else {
+        KNode* nodes = (KNode*)at(oNodes);
+        int *parent = (int*)at(oParent), *dHeight = (int*)at(oHeight);
+        launchFill64((unsigned long long*)dHeight, 1, 0ull, s);
+        hipLaunchKernelGGL(k_karras, dim3(blocks(n - 1)), dim3(256), 0, s, (const unsigned long long*)skeys, n, nodes,
+                           parent);
+        for (int base = 0; base + 1 < L.count; base += kBoxStep)
+            hipLaunchKernelGGL(k_box_levels, dim3((L.size[base] + (1u << kBoxStep) - 1) >> kBoxStep),
+                               dim3(1 << (kBoxStep - 1)), 0, s, L, base, (const float*)leafBox, up);
+        hipLaunchKernelGGL(k_node_boxes, dim3(blocks(n - 1)), dim3(256), 0, s, L, (const KNode*)nodes, n - 1,
+                           (const float*)leafBox, (const float*)up, box);
+        hipLaunchKernelGGL(k_height, dim3(std::min(256, blocks(n - 1))), dim3(256), 0, s, (const KNode*)nodes,
+                           (const int*)parent, n - 1, dHeight);
+        hipLaunchKernelGGL(k_emit_pairs, dim3(blocks(n - 1)), dim3(256), 0, s, (const KNode*)nodes, n,
+                           (const float*)leafBox, (const float*)box, pairs);
+        hipLaunchKernelGGL(k_collapse4, dim3(blocks(n - 1)), dim3(256), 0, s, (const KNode*)nodes, n - 1,
+                           (const float4*)pairs, (float4*)quads.p);
+        GP_HIP(hipGetLastError());
+        GP_HIP(hipMemcpyAsync(&height, dHeight, sizeof(int), hipMemcpyDeviceToHost, s));
+    }
+    if (hipMalloc(&tris.p, sizeof(float4) * 3 * (size_t)n) != hipSuccess) tris.p = nullptr;
+    if (hipMalloc(&trin.p, sizeof(float4) * (size_t)n) != hipSuccess) trin.p = nullptr;
+    if (!tris.p || !trin.p) {
+        hipStreamSynchronize(s);   // the height is still being written
+        return fail(GP_ERR_OOM, "BVH build: triangle allocation failed");
+    }
+    hipLaunchKernelGGL(k_gather, dim3(blocks(n)), dim3(256), 0, s, (const float*)in.verts, (const int*)in.mats,
+                       (const unsigned*)order, n, (float4*)tris.p, (float4*)trin.p);
     hipError_t ge = hipGetLastError();
     hipError_t se = hipStreamSynchronize(s);
-    if (ge != hipSuccess || se != hipSuccess) {
-        hipFree(tris);
-        hipFree(trin);
+    if (ge != hipSuccess || se != hipSuccess)
         return fail(GP_ERR_HIP, std::string("BVH build: ") + hipGetErrorString(ge != hipSuccess ? ge : se));
-    }
-    qg.keep = true;   // the pair nodes are freed on return
-    out.nodes = quads;
-    out.tris = tris;
-    out.trin = trin;
-    out.nPairs = (int64_t)nPairs;
+    quads.keep = tris.keep = trin.keep = true;
+    out.nodes = (float4*)quads.p;
+    out.tris = (float4*)tris.p;
+    out.trin = (float4*)trin.p;
+    out.nPairs = (int64_t)inner;
     out.depth = std::max(1, height);
     out.stackNeed = 3 * ((out.depth + 1) / 2);   // four-wide levels: pair levels 1, 3, 5, ...
     out.buildMs = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

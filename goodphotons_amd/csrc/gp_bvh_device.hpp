@@ -19,10 +19,25 @@ struct DeviceBvh {
     double buildMs = 0.0;
 };
 
-// dTrisIn / dTrinIn: input-order triangles (3 float4, .w = prim id / material) and
-// normals; centerLo/Hi bound the triangles' box centres. Synchronous.
-gp_status buildBvhDevice(const float4* dTrisIn, const float4* dTrinIn, int64_t n, const float centerLo[3],
-                         const float centerHi[3], DeviceBvh& out);
+// A caller's triangles on the device, as uploaded, and the bounds of their box centres.
+struct DeviceTris {
+    float* verts = nullptr;    // 9 floats per triangle; one allocation with mats behind it
+    int32_t* mats = nullptr;
+    int64_t n = 0;
+    float centerLo[3] = {}, centerHi[3] = {};
+
+    DeviceTris() = default;
+    DeviceTris(const DeviceTris&) = delete;
+    DeviceTris& operator=(const DeviceTris&) = delete;
+    ~DeviceTris();
+};
+
+// Uploads and checks n triangles (GP_ERR_INVALID: a material id outside [0, nMats) or a
+// vertex that is not finite) and reduces their bounds. Synchronous.
+gp_status scanTrisDevice(const float* verts, const int32_t* mats, int64_t n, int nMats, DeviceTris& out);
+
+// Synchronous.
+gp_status buildBvhDevice(const DeviceTris& in, DeviceBvh& out);
 
 // Smallest squared distance from p to any of n triangles (3 float4 each), in double.
 gp_status deviceMinDistance2(const float4* dTris, int64_t n, const double p[3], double& d2);

@@ -52,6 +52,9 @@ struct Group {
 
 void buildMirrorPlanes(const gp_scene_desc* d, std::vector<DevMirrorPlane>& out) {
     out.clear();
+    bool any = false;
+    for (int m = 0; m < d->n_materials; ++m) any = any || d->materials[m].type == GP_MAT_MIRROR;
+    if (!any) return;
     std::vector<Group> groups;
     std::map<std::array<long long, 4>, int> byKey;
     for (int64_t t = 0; t < d->n_tris; ++t) {
