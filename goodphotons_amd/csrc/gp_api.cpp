@@ -583,13 +583,14 @@ gp_status gp_trace_shared(gp_scene* s, int32_t n_cams, const gp_camera_desc* cam
         ts.capacity = E.capacity;
         ts.nCams = n_cams;
         ts.once = once ? 1 : 0;
+        const bool flies = E.flies((uint64_t)n, n_cams);
         launchStartTrace(E.q, ts, strm);
         GP_HIP(hipGetLastError());
         E.parity = 0;
         const Ctrl& C = *E.hCtrl;
         int64_t iters = 0;
         if (once) {
-            if ((st = E.traceOnce((unsigned)n, n_cams, p->max_depth)) != GP_OK) return st;
+            if ((st = flies ? E.fly((unsigned)n, p->max_depth) : E.traceOnce((unsigned)n, n_cams, p->max_depth)) != GP_OK) return st;
             iters = E.onceIterations;
         }
         const int K = chunkIterations(E.tun);

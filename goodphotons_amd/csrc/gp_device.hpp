@@ -531,10 +531,10 @@ __device__ __forceinline__ int traceClosest(const float4* __restrict__ nodes,
 
 // Any hit on [tmin, tmax) over the four-wide tree. Same loop shape; hit slots are
 // visited lowest slot first.
-template <int SD, bool SPILL, class Cnt>
+template <int SD, bool SPILL, class Cnt, int ST>
 __device__ __forceinline__ bool traceAny(const float4* __restrict__ nodes,
                                          const float4* __restrict__ tris, const RayPre& r,
-                                         float tmin, float tmax, Stack<SD, false, SPILL>& stk, Cnt& cnt) {
+                                         float tmin, float tmax, Stack<SD, false, SPILL, ST>& stk, Cnt& cnt) {
     int node = 0;
     stk.sp = 0;
     while (true) {
@@ -552,7 +552,7 @@ __device__ __forceinline__ bool traceAny(const float4* __restrict__ nodes,
 #pragma unroll
             for (int k = 3; k >= 0; --k) {
                 if (!SPILL) {
-                    stk.e1[stk.sp * kTravThreads] = next;
+                    stk.e1[stk.sp * ST] = next;
                     stk.sp += (h[k] && have) ? 1 : 0;
                 } else if (h[k] && have) {
                     stk.push(next, 0.0f);

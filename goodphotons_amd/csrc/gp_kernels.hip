@@ -13,6 +13,7 @@
 //                          survivors compacted into the other queue by wave ballot
 //   k_connect              any-hit for every connection; unoccluded ones splat into
 //                          the int64 fixed-point film with 64-bit atomics
+//   k_flight               (small traces, instead of all the others) whole paths in registers
 //   k_mirror               (scenes with flat mirrors only) camera connections of the
 //                          queued vertices through each mirror plane
 // All kernels are fixed-grid and grid-stride over counts that live on the device,
@@ -446,6 +447,33 @@ __global__ void __launch_bounds__(kBinThreads) k_emit_perm(Queues q) {
     }
 }
 
+// Photon `idx` of job J: where it leaves the light and in which direction, its bundle of
+// wavelengths and their weights. False for a photon without power at its wavelength.
+__device__ __forceinline__ bool emitPhoton(const DevJob& J, unsigned long long idx, Rng& rng, F3& org, F3& en,
+                                           F3& dir, float* lam, float* beta) {
+    rng = seedPhoton(J.seedBase + idx, J.salt);
+    const int ei = pickEmitter(J, rng);
+    const DevEmitter& E = J.ems[ei];
+    float u1 = rng.uniform();
+    float u2 = rng.uniform();
+    org = load3(E.origin) + load3(E.u) * u1 + load3(E.v) * u2;
+    en = load3(E.normal);
+    dir = E.collimated ? load3(E.beam) : cosineDir(en, rng);
+    const int C = J.heroC;
+    double ub = rng.uniformD();
+    double pdf0;
+    lam[0] = (float)invertCdf(E.cdf, E.guide, ub, pdf0);
+    for (int i = 1; i < C; ++i) {
+        double uu = ub + (double)i / (double)C;
+        if (uu >= 1.0) uu -= 1.0;
+        double pd;
+        lam[i] = (float)invertCdf(E.cdf, E.guide, uu, pd);
+    }
+    const float b = J.basePower / (float)C;
+    for (int i = 0; i < C; ++i) beta[i] = b;
+    return pdf0 > 0.0;
+}
+
 // Launch bound: five waves per SIMD (96 registers, no spills; -2% k_emit time on c2).
 __global__ void __launch_bounds__(256, 5) k_emit(Queues q, int cur) {
     Ctrl* c = q.ctrl;
@@ -477,29 +505,13 @@ __global__ void __launch_bounds__(256, 5) k_emit(Queues q, int cur) {
         const int j = c->emitJob[k];
         const DevJob& J = q.jobs[j];
         const unsigned long long idx = c->emitStart[k] + (s - c->emitPrefix[k]);
-        Rng rng = seedPhoton(J.seedBase + idx, J.salt);
-        const int ei = pickEmitter(J, rng);
-        const DevEmitter& E = J.ems[ei];
-        float u1 = rng.uniform();
-        float u2 = rng.uniform();
-        F3 org = load3(E.origin) + load3(E.u) * u1 + load3(E.v) * u2;
-        F3 en = load3(E.normal);
-        F3 dir = E.collimated ? load3(E.beam) : cosineDir(en, rng);
-        const int C = J.heroC;
-        double ub = rng.uniformD();
         float lam[kMaxHero] = {0.f, 0.f, 0.f, 0.f};
         float beta[kMaxHero] = {0.f, 0.f, 0.f, 0.f};
-        double pdf0;
-        lam[0] = (float)invertCdf(E.cdf, E.guide, ub, pdf0);
-        const bool dead = !(pdf0 > 0.0);
-        for (int i = 1; i < C; ++i) {
-            double uu = ub + (double)i / (double)C;
-            if (uu >= 1.0) uu -= 1.0;
-            double pd;
-            lam[i] = (float)invertCdf(E.cdf, E.guide, uu, pd);
-        }
-        const float b = J.basePower / (float)C;
-        for (int i = 0; i < C; ++i) beta[i] = b;
+        F3 org, en, dir;
+        Rng rng;
+        const int C = J.heroC;
+        const bool dead = !emitPhoton(J, idx, rng, org, en, dir, lam, beta);
+        const float b = beta[0];
         accumulate(eacc, j, eTab);
         accumulate(pacc, j, pTab);
         pacc.v[0] += 1;
@@ -609,6 +621,134 @@ __global__ void __launch_bounds__(kExtendThreads, 6) k_extend(Queues q, int cur)
 constexpr int kLocalKeys = 256;
 __device__ __forceinline__ unsigned localKey(unsigned key) { return ((key >> 7) << 3) | (key & 7u); }
 
+// What a path's hit at p (triangle `tri`, arriving along d) does: the scatter in place
+// (wavelengths, weights, stream), the vertex to connect to the cameras, and whether the
+// path goes on (from no along nd). led: absorbed, escaped, residual.
+struct Vertex {
+    bool diffuse = false;
+    F3 n{0.f, 0.f, 0.f};
+    float beta[kMaxHero] = {0.f, 0.f, 0.f, 0.f}, rho[kMaxHero] = {0.f, 0.f, 0.f, 0.f};
+};
+
+__device__ __forceinline__ bool scatterHit(const DevJob& J, F3 p, F3 d, int tri, unsigned photon, int bounce,
+                                           Rng& rng, const float* lam, float* beta, int& nUp,
+                                           unsigned long long* led, Vertex& v, F3& no, F3& nd) {
+    auto activeSum = [&]() {
+        double s = 0.0;
+        for (int k = 0; k < nUp; ++k) s += (double)beta[k];
+        return s;
+    };
+    const float4 tn = J.trin[tri];
+    const F3 gn = xyz(tn);
+    const DevMaterial& M = J.mats[__float_as_int(tn.w)];
+    const F3 n = (dot(d, gn) < 0.0f) ? gn : -gn;
+    rng.inc = photonInc(J.seedBase + photon, J.salt);
+    const bool roulette = bounce >= J.rrDepth;
+    bool alive = true;
+    if (M.type == 1) {
+        // Dielectric: de-hero, then Fresnel reflect or Snell refract (exterior
+        // index 1). The side is read off the geometric normal (entering when the
+        // ray runs against it), as the reference does.
+        if (nUp > 1) {
+            beta[0] *= (float)J.heroC;
+            nUp = 1;
+        }
+        const float eta_g = specEval(M.ior, lam[0]);
+        const bool entering = dot(d, gn) < 0.0f;
+        const F3 nl = entering ? gn : -gn;
+        const float n1 = entering ? 1.0f : eta_g;
+        const float n2 = entering ? eta_g : 1.0f;
+        const float eta = n1 / n2;
+        const float cosI = -dot(d, nl);
+        const float sin2t = eta * eta * (1.0f - cosI * cosI);
+        F3 out;
+        bool refracted = false;
+        if (sin2t > 1.0f) {
+            out = reflectDir(d, nl);
+        } else {
+            const float cosT = sqrtf(1.0f - sin2t);
+            const float rs = (n1 * cosI - n2 * cosT) / (n1 * cosI + n2 * cosT);
+            const float rp = (n1 * cosT - n2 * cosI) / (n1 * cosT + n2 * cosI);
+            const float R = 0.5f * (rs * rs + rp * rp);
+            if (rng.uniform() < R) {
+                out = reflectDir(d, nl);
+            } else {
+                out = d * eta + nl * (eta * cosI - cosT);
+                refracted = true;
+            }
+        }
+        out = normalize(out);
+        if (M.roughness > 1e-3f) {
+            F3 pert = glossyDir(out, M.roughness, rng);
+            bool ok = refracted ? (dot(pert, nl) < 0.0f) : (dot(pert, nl) > 0.0f);
+            if (ok) out = pert;
+        }
+        no = p + out * kRayEps;
+        nd = out;
+    } else {
+        float c[kMaxHero] = {0.f, 0.f, 0.f, 0.f};
+        float q0 = 0.0f;
+        for (int k = 0; k < nUp; ++k) {
+            float r = specEval(M.reflect, lam[k]);
+            c[k] = r < 0.0f ? 0.0f : (r > 1.0f ? 1.0f : r);
+            q0 = (k == 0 || c[k] > q0) ? c[k] : q0;
+        }
+        const bool diffuse = (M.type == 0);
+        if (diffuse) {
+            v.diffuse = true;
+            v.n = n;
+            for (int k = 0; k < kMaxHero; ++k) { v.beta[k] = beta[k]; v.rho[k] = c[k]; }
+        }
+        if (roulette) {
+            if (rng.uniform() >= q0) {
+                led[0] += toFixed(activeSum(), J.energyScale);
+                alive = false;
+            } else {
+                double ab = 0.0;
+                for (int k = 0; k < nUp; ++k) {
+                    float w = c[k] / q0;
+                    ab += (double)beta[k] * (double)(1.0f - w);
+                    beta[k] *= w;
+                }
+                led[0] += toFixed(ab, J.energyScale);
+            }
+        } else {
+            if (!(q0 > 0.0f)) {
+                led[0] += toFixed(activeSum(), J.energyScale);
+                alive = false;
+            } else {
+                double ab = 0.0;
+                for (int k = 0; k < nUp; ++k) {
+                    ab += (double)beta[k] * (double)(1.0f - c[k]);
+                    beta[k] *= c[k];
+                }
+                led[0] += toFixed(ab, J.energyScale);
+            }
+        }
+        if (alive) {
+            F3 wo;
+            if (diffuse) {
+                wo = cosineDir(n, rng);
+            } else if (M.type == 2) {
+                wo = reflectDir(d, n);
+            } else {
+                wo = glossyDir(reflectDir(d, n), M.roughness, rng);
+                if (dot(wo, n) <= 0.0f) {
+                    led[0] += toFixed(activeSum(), J.energyScale);
+                    alive = false;
+                }
+            }
+            no = p + n * kRayEps;
+            nd = wo;
+        }
+    }
+    if (alive && bounce + 1 >= J.maxDepth) {
+        led[2] += toFixed(activeSum(), J.energyScale);
+        alive = false;
+    }
+    return alive;
+}
+
 template <bool BIN>
 __global__ void __launch_bounds__(kShadeThreads, 4) k_shade(Queues q, int cur) {
     const int nxt = cur ^ 1;
@@ -678,118 +818,17 @@ __global__ void __launch_bounds__(kShadeThreads, 4) k_shade(Queues q, int cur) {
                 const float4 o4 = BIN ? rec[0] : q.ro[cur][i], d4 = BIN ? rec[1] : q.rd[cur][i];
                 const F3 d = xyz(d4);
                 const F3 p = xyz(o4) + d * h.x;
-                const float4 tn = J.trin[tri];
-                const F3 gn = xyz(tn);
-                const DevMaterial& M = J.mats[__float_as_int(tn.w)];
-                const F3 n = (dot(d, gn) < 0.0f) ? gn : -gn;
-                rng.inc = photonInc(J.seedBase + s4.z, J.salt);
-                const bool roulette = bounce >= J.rrDepth;
-                alive = true;
-                if (M.type == 1) {
-                    // Dielectric: de-hero, then Fresnel reflect or Snell refract (exterior
-                    // index 1). The side is read off the geometric normal (entering when the
-                    // ray runs against it), as the reference does.
-                    if (nUp > 1) {
-                        beta[0] *= (float)J.heroC;
-                        nUp = 1;
-                    }
-                    const float eta_g = specEval(M.ior, lam[0]);
-                    const bool entering = dot(d, gn) < 0.0f;
-                    const F3 nl = entering ? gn : -gn;
-                    const float n1 = entering ? 1.0f : eta_g;
-                    const float n2 = entering ? eta_g : 1.0f;
-                    const float eta = n1 / n2;
-                    const float cosI = -dot(d, nl);
-                    const float sin2t = eta * eta * (1.0f - cosI * cosI);
-                    F3 out;
-                    bool refracted = false;
-                    if (sin2t > 1.0f) {
-                        out = reflectDir(d, nl);
-                    } else {
-                        const float cosT = sqrtf(1.0f - sin2t);
-                        const float rs = (n1 * cosI - n2 * cosT) / (n1 * cosI + n2 * cosT);
-                        const float rp = (n1 * cosT - n2 * cosI) / (n1 * cosT + n2 * cosI);
-                        const float R = 0.5f * (rs * rs + rp * rp);
-                        if (rng.uniform() < R) {
-                            out = reflectDir(d, nl);
-                        } else {
-                            out = d * eta + nl * (eta * cosI - cosT);
-                            refracted = true;
-                        }
-                    }
-                    out = normalize(out);
-                    if (M.roughness > 1e-3f) {
-                        F3 pert = glossyDir(out, M.roughness, rng);
-                        bool ok = refracted ? (dot(pert, nl) < 0.0f) : (dot(pert, nl) > 0.0f);
-                        if (ok) out = pert;
-                    }
-                    no = p + out * kRayEps;
-                    nd = out;
-                } else {
-                    float c[kMaxHero] = {0.f, 0.f, 0.f, 0.f};
-                    float q0 = 0.0f;
-                    for (int k = 0; k < nUp; ++k) {
-                        float v = specEval(M.reflect, lam[k]);
-                        c[k] = v < 0.0f ? 0.0f : (v > 1.0f ? 1.0f : v);
-                        q0 = (k == 0 || c[k] > q0) ? c[k] : q0;
-                    }
-                    const bool diffuse = (M.type == 0);
-                    if (diffuse) {
-                        camN = J.nCams;
-                        mirrorsToo = J.nMirrors > 0;
-                        cams = J.cams;
-                        cjob = (unsigned)j;
-                        cUp = nUp;
-                        cp = p;
-                        cn = n;
-                        for (int k = 0; k < kMaxHero; ++k) { cbeta[k] = beta[k]; crho[k] = c[k]; }
-                    }
-                    if (roulette) {
-                        if (rng.uniform() >= q0) {
-                            eacc.v[0] += toFixed(activeSum(), J.energyScale);
-                            alive = false;
-                        } else {
-                            double ab = 0.0;
-                            for (int k = 0; k < nUp; ++k) {
-                                float w = c[k] / q0;
-                                ab += (double)beta[k] * (double)(1.0f - w);
-                                beta[k] *= w;
-                            }
-                            eacc.v[0] += toFixed(ab, J.energyScale);
-                        }
-                    } else {
-                        if (!(q0 > 0.0f)) {
-                            eacc.v[0] += toFixed(activeSum(), J.energyScale);
-                            alive = false;
-                        } else {
-                            double ab = 0.0;
-                            for (int k = 0; k < nUp; ++k) {
-                                ab += (double)beta[k] * (double)(1.0f - c[k]);
-                                beta[k] *= c[k];
-                            }
-                            eacc.v[0] += toFixed(ab, J.energyScale);
-                        }
-                    }
-                    if (alive) {
-                        F3 wo;
-                        if (diffuse) {
-                            wo = cosineDir(n, rng);
-                        } else if (M.type == 2) {
-                            wo = reflectDir(d, n);
-                        } else {
-                            wo = glossyDir(reflectDir(d, n), M.roughness, rng);
-                            if (dot(wo, n) <= 0.0f) {
-                                eacc.v[0] += toFixed(activeSum(), J.energyScale);
-                                alive = false;
-                            }
-                        }
-                        no = p + n * kRayEps;
-                        nd = wo;
-                    }
-                }
-                if (alive && bounce + 1 >= J.maxDepth) {
-                    eacc.v[2] += toFixed(activeSum(), J.energyScale);
-                    alive = false;
+                Vertex v;
+                alive = scatterHit(J, p, d, tri, s4.z, bounce, rng, lam, beta, nUp, eacc.v, v, no, nd);
+                if (v.diffuse) {
+                    camN = J.nCams;
+                    mirrorsToo = J.nMirrors > 0;
+                    cams = J.cams;
+                    cjob = (unsigned)j;
+                    cUp = nUp;
+                    cp = p;
+                    cn = v.n;
+                    for (int k = 0; k < kMaxHero; ++k) { cbeta[k] = v.beta[k]; crho[k] = v.rho[k]; }
                 }
                 if (alive) bkey = binKey(J, no, nd);
                 meta = packMeta((unsigned)j, (unsigned)(bounce + 1), (unsigned)nUp);
@@ -865,10 +904,11 @@ constexpr int kSplatProbe = 8;
 constexpr unsigned long long kSplatEmpty = ~0ull;
 
 // Slot of `key` (claimed if absent) within maxProbe linear probes, or -1.
+template <int SLOTS = kSplatSlots>
 __device__ __forceinline__ int splatSlot(unsigned long long* sKey, unsigned long long key, int maxProbe) {
     const unsigned h = (unsigned)((key * 0x9E3779B97F4A7C15ull) >> 56);
     for (int p = 0; p < maxProbe; ++p) {
-        const int s = (int)((h + (unsigned)p) & (kSplatSlots - 1));
+        const int s = (int)((h + (unsigned)p) & (SLOTS - 1));
         unsigned long long cur = __hip_atomic_load(&sKey[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         if (cur == kSplatEmpty) cur = atomicCAS(&sKey[s], kSplatEmpty, key);
         if (cur == kSplatEmpty || cur == key) return s;
@@ -886,10 +926,11 @@ __device__ __forceinline__ void splatAdd(unsigned long long* sVal, int s, unsign
 
 // Called by every thread of the workgroup after a barrier: adds every occupied
 // slot into its film, lane t taking word t % 4 of slot t / 4 (+ 64 per pass).
+template <int SLOTS = kSplatSlots>
 __device__ __forceinline__ void flushSplats(const DevJob* jobs, const unsigned long long* sKey,
                                             const unsigned long long* sVal) {
     const int w = threadIdx.x & 3;
-    for (int s = threadIdx.x >> 2; s < kSplatSlots; s += blockDim.x >> 2) {
+    for (int s = threadIdx.x >> 2; s < SLOTS; s += blockDim.x >> 2) {
         const unsigned long long key = sKey[s];
         if (key == kSplatEmpty) continue;
         const unsigned long long v = sVal[4 * s + w];
@@ -901,8 +942,9 @@ __device__ __forceinline__ void flushSplats(const DevJob* jobs, const unsigned l
     }
 }
 
+template <int SLOTS = kSplatSlots>
 __device__ __forceinline__ void clearSplats(unsigned long long* sKey, unsigned long long* sVal) {
-    for (int k = threadIdx.x; k < kSplatSlots; k += blockDim.x) {
+    for (int k = threadIdx.x; k < SLOTS; k += blockDim.x) {
         sKey[k] = kSplatEmpty;
         sVal[4 * k + 0] = 0; sVal[4 * k + 1] = 0; sVal[4 * k + 2] = 0; sVal[4 * k + 3] = 0;
     }
@@ -997,6 +1039,172 @@ __global__ void __launch_bounds__(kTravThreads, 6) k_connect(Queues q) {
     flushJobTable(cacc, cTab, nJobs, ca);   // ends with a barrier-ordered read of cTab
     __syncthreads();
     flushSplats(q.jobs, sKey, sVal);
+}
+
+// ------------------------------------------------------------------ flight
+// A whole small trace in one launch: each lane carries a photon from the light to the end
+// of its path, and connects its vertices on the way. A lane whose path has ended takes its
+// next photon (gtid, gtid + stride, ...) once a quarter of the wave's live lanes waits for
+// one, so that the emission code does not run for a lane or two at a time. Between
+// iterations of the wavefront a path goes through 200 bytes of memory and three launches;
+// here it stays in registers (128 of them: four waves per SIMD).
+// The wavefront's kernels are bound by launches and dependent loads while a trace does not
+// fill the chip: the 5000-photon preview of the box spent 470 of its 590 us in 26 kernels.
+// `lanes` of each wave carry photons: a trace of few photons is spread over more waves, so
+// that a wave's time is the longest of fewer paths.
+// One wave per workgroup, with a splat table of its own that is flushed only at the end: a
+// splat that finds no slot is added to its film by four lanes, one per word. Any hit and
+// closest hit use the lane's own stack column one after the other (8-byte entries for
+// both: lanes of a wave may be in different traversals).
+constexpr int kFlightThreads = 64;
+constexpr int kFlightSlots = 64;
+
+// Adds the splats of the lanes with `pending` to their films, four lanes per splat. The
+// records are staged in the stack array `stk` (no traversal is running: the whole wave is
+// here).
+__device__ __forceinline__ void splatDirect(int2* stk, bool pending, unsigned long long* at, unsigned long long X,
+                                            unsigned long long Y, unsigned long long Z, unsigned long long H) {
+    const unsigned long long mask = __ballot(pending);
+    if (mask == 0ull) return;
+    const unsigned lane = threadIdx.x;
+    unsigned long long* col = (unsigned long long*)stk;
+    const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+    if (pending) {
+        col[0 * kFlightThreads + rank] = X;
+        col[1 * kFlightThreads + rank] = Y;
+        col[2 * kFlightThreads + rank] = Z;
+        col[3 * kFlightThreads + rank] = H;
+        col[4 * kFlightThreads + rank] = (unsigned long long)at;
+    }
+    __builtin_amdgcn_wave_barrier();
+    const unsigned count = (unsigned)__popcll(mask);
+    for (unsigned b = 0; b < count; b += 16) {
+        const unsigned r = b + (lane >> 2);
+        if (r < count) {
+            const unsigned long long v = col[(lane & 3u) * kFlightThreads + r];
+            if (v) atomicAdd((unsigned long long*)col[4 * kFlightThreads + r] + (lane & 3u), v);
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <int SD, bool SPILL>
+__global__ void __launch_bounds__(kFlightThreads, 4) k_flight(Queues q, unsigned n, unsigned lanes) {
+    static_assert(SD >= 5, "splatDirect stages five words per lane");
+    __shared__ int2 sStk[SD * kFlightThreads];
+    __shared__ unsigned long long sKey[kFlightSlots];
+    __shared__ unsigned long long sVal[kFlightSlots * 4];
+    __shared__ unsigned long long sAcc[kAccRow];
+    clearSplats<kFlightSlots>(sKey, sVal);
+    if (threadIdx.x < kAccRow) sAcc[threadIdx.x] = 0ull;
+    __syncthreads();
+    const DevJob& J = q.jobs[0];
+    const unsigned gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    int2* spill = SPILL ? q.spill + (size_t)gtid * q.spillDepth : nullptr;
+    const unsigned stride = gridDim.x * lanes;
+    unsigned next = threadIdx.x < lanes ? min(blockIdx.x * lanes + threadIdx.x, n) : n;
+    unsigned long long led[3] = {}, emitted = 0;   // absorbed, escaped, residual; emitted
+    unsigned photons = 0, direct = 0, segments = 0, connections = 0, splats = 0;
+    bool alive = false;
+    F3 o{0.f, 0.f, 0.f}, d{0.f, 0.f, 0.f};
+    float lam[kMaxHero] = {0.f, 0.f, 0.f, 0.f}, beta[kMaxHero] = {0.f, 0.f, 0.f, 0.f};
+    Rng rng{};
+    unsigned photon = 0;
+    int bounce = 0, nUp = 0;
+    TravCount<false> tc;
+    while (true) {
+        const unsigned live = (unsigned)__popcll(__ballot(alive));
+        const unsigned waiting = (unsigned)__popcll(__ballot(!alive && next < n));
+        if (live + waiting == 0) break;
+        F3 vp{0.f, 0.f, 0.f};
+        Vertex v;
+        int vUp = 0;
+        bool atLight = false;
+        if (alive) {
+            Stack<SD, true, SPILL, kFlightThreads> stk{sStk + threadIdx.x, nullptr, spill, 0};
+            float t = INFINITY;
+            const int tri = traceClosest<SD, SPILL>(J.nodes, J.tris, prepareRay(o, d), kRayEps, t, stk, tc);
+            ++segments;
+            if (tri < 0) {
+                double s = 0.0;
+                for (int k = 0; k < nUp; ++k) s += (double)beta[k];
+                led[1] += toFixed(s, J.energyScale);
+                alive = false;
+            } else {
+                vp = o + d * t;
+                F3 no{0.f, 0.f, 0.f}, nd{0.f, 0.f, 0.f};
+                vUp = nUp;
+                alive = scatterHit(J, vp, d, tri, photon, bounce, rng, lam, beta, nUp, led, v, no, nd);
+                o = no;
+                d = nd;
+                ++bounce;
+            }
+        } else if (next < n && 4 * waiting >= live) {
+            for (int k = 0; k < kMaxHero; ++k) { lam[k] = 0.f; beta[k] = 0.f; }
+            photon = next;
+            next = n - next > stride ? next + stride : n;
+            F3 dir;
+            alive = emitPhoton(J, photon, rng, vp, v.n, dir, lam, beta);
+            ++photons;
+            o = vp + dir * kRayEps;
+            d = dir;
+            bounce = 0;
+            nUp = vUp = J.heroC;
+            if (alive) {
+                emitted += toFixed((double)beta[0] * (double)J.heroC, J.energyScale);
+                atLight = v.diffuse = true;
+                for (int k = 0; k < kMaxHero; ++k) { v.beta[k] = beta[k]; v.rho[k] = 1.0f; }
+            }
+        }
+        __syncthreads();   // one wave: the lanes are together from here to the next photon
+        const int nCams = v.diffuse ? J.nCams : 0;
+        for (int k = 0; __any(k < nCams); ++k) {
+            bool pending = false;
+            unsigned long long *at = nullptr, X = 0, Y = 0, Z = 0, H = 0;
+            if (k < nCams) {
+                const DevCamera& K = J.cams[k];
+                float4 co, cd, cx;
+                if (makeConnection(K, 0u, vp, v.n, lam, v.beta, v.rho, vUp, co, cd, cx)) {
+                    ++connections;
+                    direct += atLight ? 1u : 0u;
+                    Stack<SD, false, SPILL, 2 * kFlightThreads> stk{nullptr, (int*)(sStk + threadIdx.x), spill, 0};
+                    if (!traceAny<SD, SPILL>(J.nodes, J.tris, prepareRay(xyz(co), xyz(cd)), kRayEps, co.w, stk, tc)) {
+                        ++splats;
+                        const unsigned pix = (unsigned)__float_as_int(cd.w);
+                        X = min(toFixed((double)cx.x, K.filmScale), K.filmQmax);
+                        Y = min(toFixed((double)cx.y, K.filmScale), K.filmQmax);
+                        Z = min(toFixed((double)cx.z, K.filmScale), K.filmQmax);
+                        H = (unsigned long long)vUp;
+                        const int s = splatSlot<kFlightSlots>(sKey, ((unsigned long long)k << 32) | pix, kSplatProbe);
+                        if (s >= 0) {
+                            splatAdd(sVal, s, X, Y, Z, H);
+                        } else {
+                            pending = true;
+                            at = (unsigned long long*)K.film + 4 * (size_t)pix;
+                        }
+                    }
+                }
+            }
+            splatDirect(sStk, pending, at, X, Y, Z, H);
+        }
+    }
+    auto add = [&](int k, unsigned long long x) {
+        if (x) atomicAdd(&sAcc[k], x);
+    };
+    add(kAccEnergy + 0, emitted);
+    add(kAccEnergy + 1, led[0]);
+    add(kAccEnergy + 3, led[1]);
+    add(kAccEnergy + 4, led[2]);
+    add(kAccPhotons, photons);
+    add(kAccDirect, direct);
+    add(kAccSegments, segments);
+    add(kAccConnections, connections);
+    add(kAccSplats, splats);
+    __syncthreads();
+    if (threadIdx.x < kAccRow && sAcc[threadIdx.x])
+        atomicAdd(J.acc + (size_t)(blockIdx.x % kSegs) * kAccRow + threadIdx.x, sAcc[threadIdx.x]);
+    flushSplats<kFlightSlots>(q.jobs, sKey, sVal);
 }
 
 // ------------------------------------------------------------------ mirrors
@@ -1524,6 +1732,11 @@ void launchConnect(const Queues& q, const LaunchShape& ls, hipStream_t s) {
     if (q.stats) GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALLS);
     else GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALL);
 #undef GP_CALLS
+#undef GP_CALL
+}
+void launchFlight(const Queues& q, unsigned n, unsigned lanes, int blocks, hipStream_t s) {
+#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_flight<SD, SP>), dim3(blocks), dim3(kFlightThreads), 0, s, q, n, lanes)
+    GP_BY_STACK_EXT(q.lds, q.useSpill, GP_CALL);
 #undef GP_CALL
 }
 void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s) {

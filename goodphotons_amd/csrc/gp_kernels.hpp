@@ -87,6 +87,9 @@ void launchConnect(const Queues& q, const LaunchShape& ls, hipStream_t s);
 // Ray binning of queue `cur` into queue 2 (four kernels: count, chunk sums, bin scan,
 // scatter).
 void launchBin(const Queues& q, int cur, hipStream_t s);
+// A whole trace of n photons of job 0, `lanes` of each wave carrying photons; at most
+// the closest-hit kernel's threads (its spill area is sized for those).
+void launchFlight(const Queues& q, unsigned n, unsigned lanes, int blocks, hipStream_t s);
 void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s);
 
 // Batch probes over host-provided rays (already on the device).

@@ -640,6 +640,23 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
     return fail(GP_ERR_STATE, "paths alive past their depth limit");
 }
 
+bool Engine::flies(uint64_t n, int cams) const {
+    return n <= capacity && flightFits(n, cams, std::max(1, device().cus)) && !mirrorActive && !q.stats &&
+           !q.binned && !tun.profile;
+}
+
+gp_status Engine::fly(unsigned n, int maxDepth) {
+    const unsigned cus = (unsigned)std::max(1, device().cus);
+    // one wave per SIMD before a second photon joins a wave
+    unsigned lanes = 4;
+    while (lanes < 64 && (uint64_t)lanes * 4 * cus < n) lanes *= 2;
+    const unsigned most = std::min(kFlightWaves * cus, (unsigned)ls.extend);
+    launchFlight(q, n, lanes, (int)std::min(most, (n + lanes - 1) / lanes), device().stream);
+    GP_HIP(hipGetLastError());
+    onceIterations = maxDepth;
+    return readCtrl();
+}
+
 gp_status Engine::enqueueIterations(int n) {
     hipStream_t s = device().stream;
     gp_status st;

@@ -172,6 +172,10 @@ struct Engine {
     gp_status traceOnce(unsigned n, int cams, int maxDepth);
     static constexpr int kOnceChunk = 32;
     int onceIterations = 0;
+    // Whether a trace of n photons runs as one k_flight launch, and that run. Mirror planes,
+    // traversal statistics, kernel timing and ray binning belong to the wavefront's kernels.
+    bool flies(uint64_t n, int cams) const;
+    gp_status fly(unsigned n, int maxDepth);
     gp_status enqueueIterations(int n);       // plain launches, tracks parity
     gp_status runIterations(int n);           // graph replay when possible
     // Whether new photons are emitted in sorted order (set by the caller before

@@ -73,6 +73,22 @@ constexpr int kEmitCols = 256;
 constexpr unsigned kEmitOrderMin = 1u << 16;
 constexpr uint64_t kEmitOrderJobMin = 1u << 19;
 
+// A trace that the chip holds at once flies (k_flight) instead of running the wavefront.
+// kFlightWaves: resident waves of k_flight per CU. Per-trace times, wavefront -> flight, on
+// 256 CUs (262144 resident lanes):
+//   photons         4096          65536         262144        370816        524445
+//   box             552 -> 286    594 -> 365    729 -> 568    813 -> 787    929 -> 924 us
+//   glass, prism    1281 -> 427   1651 -> 684   1887 -> 938   1990 -> 1236  2118 -> 1486
+//   soup 100K tri.  2248 -> 646   3695 -> 1236  4187 -> 1508  4349 -> 2267  4502 -> 2622
+//   icosphere 1.3M  1651 -> 454   2672 -> 809   3195 -> 961   3298 -> 1366  3591 -> 1568
+// and 0.55-1.5x at 2^20: past about one and a half photons per lane a box loses. Six
+// cameras: 2068 -> 1745 us at 65536 photons, 2235 -> 2019 at 131080, 2332 -> 2480 at
+// 185386, so a camera more counts as a third of a photon.
+constexpr int kFlightWaves = 16;
+inline bool flightFits(uint64_t photons, int cams, int cus) {
+    return 2 * photons * (uint64_t)(2 + cams) <= 9 * (uint64_t)cus * kFlightWaves * 64;
+}
+
 // Leaf links are negative: ~((first << 3) | (count - 1)).
 inline constexpr int leafCode(int first, int count) { return ~((first << 3) | (count - 1)); }
 
