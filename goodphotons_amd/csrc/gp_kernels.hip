@@ -1056,7 +1056,6 @@ __global__ void __launch_bounds__(kTravThreads, 6) k_connect(Queues q) {
 // splat that finds no slot is added to its film by four lanes, one per word. Any hit and
 // closest hit use the lane's own stack column one after the other (8-byte entries for
 // both: lanes of a wave may be in different traversals).
-constexpr int kFlightThreads = 64;
 constexpr int kFlightSlots = 64;
 
 // Adds the splats of the lanes with `pending` to their films, four lanes per splat. The
@@ -1215,10 +1214,15 @@ __global__ void __launch_bounds__(kFlightThreads, 4) k_flight(Queues q, unsigned
 // specular geometry factor is 1 / D^2 over the unfolded length D. The geometry is
 // solved in double; the two legs are traced in float: the light side must be clear
 // (any hit), and the eye's closest hit must be a mirror triangle at R (within
-// 1e-4 (1 + |R - eye|)), whose reflectance tints the splat. One thread per queued
-// vertex walks the scene's planes (outer) and the job's cameras (inner); splats go
-// straight to the film with 64-bit atomics (they are few next to the direct
-// connections, and integer sums keep the film independent of their order).
+// 1e-4 (1 + |R - eye|)), whose reflectance tints the splat.
+// One wave per workgroup, in two steps: the wave's lanes solve the geometry of their
+// vertices against the scene's planes (outer) and the job's cameras (inner), most of which
+// end there, and list the rest in LDS; 64 listed connections are then traced together. The
+// two legs run on the lane's own stack column one after the other, as in k_flight, and
+// splats go through its per-wave table. As one thread per vertex in 256-thread workgroups,
+// solving and tracing under each other's masks with 199 registers and 52 KB of LDS (two
+// waves per SIMD) and a film atomic per word, the mirror box (2^20 photons) spent 1370 us
+// here, now 626 us.
 struct MirrorSolve {
     double wP[3];       // vertex -> mirror point, unit
     double dP;          // vertex -> mirror point distance
@@ -1278,87 +1282,142 @@ __device__ __forceinline__ bool solveMirror(const DevMirrorPlane& P, const DevCa
 }
 
 template <int SD, bool SPILL>
-__global__ void __launch_bounds__(kTravThreads) k_mirror(Queues q) {
-    // Separate LDS arrays for the two traversals: lanes of a workgroup run the light leg
-    // (any hit, int entries) and the eye leg (closest hit, int2 entries) at the same
-    // time, and two views of one array would overlap across lanes (lane t's int entry k
-    // and lane u's int2 entry r share a word whenever k*256 + t = 2*(r*256 + u) + 0/1).
-    __shared__ int2 sStk[SD * kTravThreads];
-    __shared__ int sStkAny[SD * kTravThreads];
-    __shared__ unsigned long long cTab[kMaxJobs * 2];
+__global__ void __launch_bounds__(kFlightThreads, 4) k_mirror(Queues q) {
+    static_assert(SD >= 5, "splatDirect stages five words per lane");
+    __shared__ int2 sStk[SD * kFlightThreads];
+    __shared__ unsigned long long sKey[kFlightSlots];
+    __shared__ unsigned long long sVal[kFlightSlots * 4];
+    __shared__ unsigned long long sCand[2 * kFlightThreads];   // vertex, plane << 32, camera << 40
+    __shared__ unsigned cTab[kMaxJobs * 2];   // ray queries, splats (legs not in the statistics)
+    clearSplats<kFlightSlots>(sKey, sVal);
     SegMap sm;
     const unsigned n = loadSegMap(q.ctrl->mirrorCount, q.mirrorSegCap, sm);
     const int nJobs = q.ctrl->nJobs;
-    initJobTable<2>(cTab, nJobs);
-    JobAcc<2> cacc;   // ray queries of the connections, splats (legs not in the statistics)
-    AccAddr ca{q.jobs, kAccConnections};
+    for (int r = threadIdx.x; r < nJobs * 2; r += kFlightThreads) cTab[r] = 0u;
+    __syncthreads();
     TravCount<false> tc;
-    const unsigned stride = gridDim.x * blockDim.x;
-    const unsigned gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    int2* spill = SPILL ? q.spill + (size_t)gtid * q.spillDepth : nullptr;
-    for (unsigned li = gtid; li < n; li += stride) {
-        const unsigned i = sm.slot(li);
-        const float4 a = q.mv[0][i], b = q.mv[1][i], l4 = q.mv[2][i], w4 = q.mv[3][i];
-        const unsigned tag = (unsigned)__float_as_int(a.w);
-        const int j = (int)(tag & 0xffffu);
-        const int nUp = (int)((tag >> 16) & 7u);
-        const DevJob& J = q.jobs[j];
-        accumulate(cacc, j, cTab);
-        const float lam[kMaxHero] = {l4.x, l4.y, l4.z, l4.w};
-        const float bw[kMaxHero] = {w4.x, w4.y, w4.z, w4.w};
-        const double p[3] = {(double)a.x, (double)a.y, (double)a.z};
-        const double np[3] = {(double)b.x, (double)b.y, (double)b.z};
-        for (int m = 0; m < J.nMirrors; ++m) {
-            const DevMirrorPlane P = J.mirrors[m];
-            for (int k = 0; k < J.nCams; ++k) {
-                const DevCamera& K = J.cams[k];
-                MirrorSolve g;
-                if (!solveMirror(P, K, p, np, g)) continue;
-                cacc.v[0] += 1;
-                const F3 wl{(float)g.wP[0], (float)g.wP[1], (float)g.wP[2]};
-                const F3 ol{(float)(p[0] + g.wP[0] * 1e-6), (float)(p[1] + g.wP[1] * 1e-6),
-                            (float)(p[2] + g.wP[2] * 1e-6)};
-                Stack<SD, false, SPILL> as{nullptr, sStkAny + threadIdx.x, spill, 0};
-                if (traceAny<SD, SPILL>(J.nodes, J.tris, prepareRay(ol, wl), kRayEps,
-                                        (float)((g.dP - 2e-6) - 1e-6), as, tc))
-                    continue;
-                cacc.v[0] += 1;
-                Stack<SD, true, SPILL> cs{sStk + threadIdx.x, nullptr, spill, 0};
-                float th = INFINITY;
-                const int tri = traceClosest<SD, SPILL>(
-                    J.nodes, J.tris, prepareRay(load3(K.eye), F3{(float)g.wE[0], (float)g.wE[1], (float)g.wE[2]}),
-                    kRayEps, th, cs, tc);
-                if (tri < 0 || fabs((double)th - g.dE) > 1e-4 * (1.0 + g.dE)) continue;
-                const DevMaterial& M = J.mats[__float_as_int(J.trin[tri].w)];
-                if (M.type != 2) continue;   // only Mirror is a planar mirror here
-                cacc.v[1] += 1;
-                double X = 0.0, Y = 0.0, Z = 0.0;
-                unsigned long long H = 0;
-                for (int c = 0; c < nUp; ++c) {
-                    float r = specEval(M.reflect, lam[c]);
-                    r = r < 0.0f ? 0.0f : (r > 1.0f ? 1.0f : r);
-                    const double contrib = (double)bw[c] * g.weight * (double)r;
-                    if (!(contrib > 0.0)) continue;
-                    const F3 cw = cie(lam[c]);
-                    X += (double)cw.x * contrib;
-                    Y += (double)cw.y * contrib;
-                    Z += (double)cw.z * contrib;
-                    ++H;
-                }
-                if (H) {
-                    unsigned long long* f = (unsigned long long*)K.film + 4 * (size_t)g.pix;
-                    const unsigned long long qx = min(toFixed(X, K.filmScale), K.filmQmax);
-                    const unsigned long long qy = min(toFixed(Y, K.filmScale), K.filmQmax);
-                    const unsigned long long qz = min(toFixed(Z, K.filmScale), K.filmQmax);
-                    if (qx) atomicAdd(f + 0, qx);
-                    if (qy) atomicAdd(f + 1, qy);
-                    if (qz) atomicAdd(f + 2, qz);
-                    atomicAdd(f + 3, H);
+    const unsigned lane = threadIdx.x, stride = gridDim.x * kFlightThreads;
+    int2* spill = SPILL ? q.spill + (size_t)(blockIdx.x * kFlightThreads + lane) * q.spillDepth : nullptr;
+    auto vertexAt = [&](unsigned i, double p[3], double np[3]) -> unsigned {
+        const float4 a = q.mv[0][i], b = q.mv[1][i];
+        p[0] = (double)a.x; p[1] = (double)a.y; p[2] = (double)a.z;
+        np[0] = (double)b.x; np[1] = (double)b.y; np[2] = (double)b.z;
+        return (unsigned)__float_as_int(a.w);
+    };
+    unsigned held = 0;                               // listed connections
+    unsigned base = blockIdx.x * kFlightThreads;     // this wave's vertices, plane and camera to solve
+    int m = 0, k = 0;
+    while (true) {
+        while (held < kFlightThreads && base < n) {
+            const unsigned li = base + lane;
+            const unsigned i = sm.slot(li < n ? li : base);
+            double p[3], np[3];
+            const DevJob& J = q.jobs[vertexAt(i, p, np) & 0xffffu];
+            const int nM = li < n ? J.nMirrors : 0, nC = J.nCams;
+            MirrorSolve g;
+            const bool ok = m < nM && k < nC && solveMirror(J.mirrors[m], J.cams[k], p, np, g);
+            const unsigned long long mask = __ballot(ok);
+            const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+            if (ok) sCand[held + rank] = i | ((unsigned long long)m << 32) | ((unsigned long long)k << 40);
+            held += (unsigned)__popcll(mask);
+            ++k;
+            if (!__any(m < nM && k < nC)) {
+                k = 0;
+                ++m;
+                if (!__any(m < nM)) {
+                    m = 0;
+                    base += stride;
+                    if (base < stride) base = n;   // past 2^32
                 }
             }
         }
+        if (held == 0) break;
+        __syncthreads();
+        const unsigned count = min(held, (unsigned)kFlightThreads);
+        bool pending = false;
+        unsigned long long *at = nullptr, X = 0, Y = 0, Z = 0, H = 0;
+        if (lane < count) {
+            const unsigned long long cand = sCand[lane];
+            const unsigned i = (unsigned)cand;
+            const int cam = (int)(cand >> 40);
+            double p[3], np[3];
+            const unsigned tag = vertexAt(i, p, np);
+            const int j = (int)(tag & 0xffffu);
+            const DevJob& J = q.jobs[j];
+            const DevCamera& K = J.cams[cam];
+            MirrorSolve g;
+            bool ok = solveMirror(J.mirrors[(cand >> 32) & 0xffu], K, p, np, g);   // solved before
+            unsigned queries = 0;
+            if (ok) {
+                queries = 1;
+                const F3 wl{(float)g.wP[0], (float)g.wP[1], (float)g.wP[2]};
+                const F3 ol{(float)(p[0] + g.wP[0] * 1e-6), (float)(p[1] + g.wP[1] * 1e-6),
+                            (float)(p[2] + g.wP[2] * 1e-6)};
+                Stack<SD, false, SPILL, 2 * kFlightThreads> as{nullptr, (int*)(sStk + lane), spill, 0};
+                ok = !traceAny<SD, SPILL>(J.nodes, J.tris, prepareRay(ol, wl), kRayEps,
+                                          (float)((g.dP - 2e-6) - 1e-6), as, tc);
+            }
+            int tri = -1;
+            if (ok) {
+                ++queries;
+                Stack<SD, true, SPILL, kFlightThreads> cs{sStk + lane, nullptr, spill, 0};
+                float th = INFINITY;
+                tri = traceClosest<SD, SPILL>(
+                    J.nodes, J.tris, prepareRay(load3(K.eye), F3{(float)g.wE[0], (float)g.wE[1], (float)g.wE[2]}),
+                    kRayEps, th, cs, tc);
+                ok = tri >= 0 && !(fabs((double)th - g.dE) > 1e-4 * (1.0 + g.dE));
+            }
+            if (queries) atomicAdd(&cTab[2 * j], queries);
+            if (ok) {
+                const DevMaterial& M = J.mats[__float_as_int(J.trin[tri].w)];
+                if (M.type == 2) {   // only Mirror is a planar mirror here
+                    atomicAdd(&cTab[2 * j + 1], 1u);
+                    const float4 l4 = q.mv[2][i], w4 = q.mv[3][i];
+                    const float lam[kMaxHero] = {l4.x, l4.y, l4.z, l4.w};
+                    const float bw[kMaxHero] = {w4.x, w4.y, w4.z, w4.w};
+                    const int nUp = (int)((tag >> 16) & 7u);
+                    double x = 0.0, y = 0.0, z = 0.0;
+                    for (int c = 0; c < nUp; ++c) {
+                        float r = specEval(M.reflect, lam[c]);
+                        r = r < 0.0f ? 0.0f : (r > 1.0f ? 1.0f : r);
+                        const double contrib = (double)bw[c] * g.weight * (double)r;
+                        if (!(contrib > 0.0)) continue;
+                        const F3 cw = cie(lam[c]);
+                        x += (double)cw.x * contrib;
+                        y += (double)cw.y * contrib;
+                        z += (double)cw.z * contrib;
+                        ++H;
+                    }
+                    if (H) {
+                        X = min(toFixed(x, K.filmScale), K.filmQmax);
+                        Y = min(toFixed(y, K.filmScale), K.filmQmax);
+                        Z = min(toFixed(z, K.filmScale), K.filmQmax);
+                        const unsigned long long key = ((unsigned long long)(j * kMaxCams + cam) << 32) | g.pix;
+                        const int s = splatSlot<kFlightSlots>(sKey, key, kSplatProbe);
+                        if (s >= 0) {
+                            splatAdd(sVal, s, X, Y, Z, H);
+                        } else {
+                            pending = true;
+                            at = (unsigned long long*)K.film + 4 * (size_t)g.pix;
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();   // one wave: together again
+        splatDirect(sStk, pending, at, X, Y, Z, H);
+        held -= count;
+        const unsigned long long rest = sCand[kFlightThreads + lane];
+        __syncthreads();
+        if (lane < held) sCand[lane] = rest;
+        __syncthreads();
     }
-    flushJobTable(cacc, cTab, nJobs, ca);
+    __syncthreads();
+    AccAddr ca{q.jobs, kAccConnections};
+    for (int r = threadIdx.x; r < nJobs * 2; r += kFlightThreads)
+        if (cTab[r]) atomicAdd(ca(r / 2, r % 2), (unsigned long long)cTab[r]);
+    flushSplats<kFlightSlots>(q.jobs, sKey, sVal);
 }
 
 // ------------------------------------------------------------------ ray binning
@@ -1740,8 +1799,8 @@ void launchFlight(const Queues& q, unsigned n, unsigned lanes, int blocks, hipSt
 #undef GP_CALL
 }
 void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s) {
-#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_mirror<SD, SP>), dim3(ls.mirror), dim3(kTravThreads), 0, s, q)
-    GP_BY_STACK(q.lds, q.useSpill, GP_CALL);
+#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_mirror<SD, SP>), dim3(ls.mirror), dim3(kFlightThreads), 0, s, q)
+    GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALL);
 #undef GP_CALL
 }
 void launchProbeClosest(const float4* nodes, const float4* tris, const float* rays, long long n,

@@ -67,6 +67,9 @@ struct Queues {
 // further).
 constexpr int kExtendGridScale = 4;
 
+// One-wave workgroups of k_flight and k_mirror.
+constexpr int kFlightThreads = 64;
+
 // Threads of a workgroup of k_extend (one wave: a workgroup's LDS, its lanes' stacks, is
 // released as soon as its own rays are done) and k_shade; the others run 256.
 constexpr int kExtendThreads = 64;

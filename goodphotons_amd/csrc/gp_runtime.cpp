@@ -426,7 +426,8 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
     DeviceState& d = device();
     const int cus = d.cus > 0 ? d.cus : 256;
     const int blocks = std::max(1, cus * tun.grid_waves_per_cu / 4);
-    ls.emit = ls.connect = ls.mirror = blocks;
+    ls.emit = ls.connect = blocks;
+    ls.mirror = blocks * (256 / kFlightThreads);
     ls.shade = (blocks * 256 + kShadeThreads - 1) / kShadeThreads;
     ls.extend = blocks * kExtendGridScale * (256 / kExtendThreads);
     const size_t threads = (size_t)ls.extend * kExtendThreads;
@@ -442,8 +443,8 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
     // Entries beyond the LDS stack live in the spill area (stack index sp >= SD maps to
     // spill[sp - SD], and sp < stackNeed). k_connect keeps as many entries in LDS as the
     // closest-hit kernel, 8 for its 12 (4-byte entries: at 8, six waves per SIMD fit its
-    // LDS; 12 or 16 leave room for five, 24 for four); k_mirror runs its 16-entry
-    // variant for 12. The spill area covers the shallowest of them.
+    // LDS; 12 or 16 leave room for five, 24 for four), and so does k_mirror. The spill area
+    // covers the shallower of the two.
     const int connLds = lds == 12 ? 8 : lds;
     const int needSpill = std::max(0, stackNeed - std::min(lds, connLds));
     const int connUseSpill = stackNeed > connLds ? 1 : 0;
@@ -617,7 +618,7 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
     sh.shade = blocks(n, kShadeThreads, ls.shade);
     // the first iteration connects the emitted photons and the shaded vertices
     sh.connect = blocks(2 * (uint64_t)n * (uint64_t)cams, 256, ls.connect);
-    sh.mirror = blocks(2 * (uint64_t)n, 256, ls.mirror);
+    sh.mirror = blocks(2 * (uint64_t)n, kFlightThreads, ls.mirror);
     gp_status st;
     if ((st = enqueueEmit(sh)) != GP_OK) return st;
     for (int i = 0; i < maxDepth;) {
@@ -628,7 +629,7 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
             q.resetCounts = 0;
             if (st != GP_OK) return st;
             sh.connect = blocks((uint64_t)n * (uint64_t)cams, 256, ls.connect);
-            sh.mirror = blocks(n, 256, ls.mirror);
+            sh.mirror = blocks(n, kFlightThreads, ls.mirror);
         }
         onceIterations = i;
         GP_HIP(hipGetLastError());
