@@ -457,37 +457,22 @@ gp_status gp_film_reset(gp_film* f) {
 gp_status gp_film_download_raw(gp_film* f, int64_t* words, double* scale) {
     if (!f) return fail(GP_ERR_INVALID, "null film");
     const size_t n = (size_t)f->rx * f->ry * 4;
-    if (words) GP_HIP(hipMemcpy(words, f->d, n * sizeof(int64_t), hipMemcpyDeviceToHost));
+    if (words) {
+        const gp_status st = copyDown(words, f->d, n * sizeof(int64_t), device().stream);
+        if (st != GP_OK) return st;
+    }
     if (scale) *scale = f->scale;
     return GP_OK;
 }
 
 gp_status gp_film_download(gp_film* f, double* xyz, double* hits) {
     if (!f) return fail(GP_ERR_INVALID, "null film");
-    const size_t np = (size_t)f->rx * f->ry;
-    std::vector<int64_t> w(np * 4);
-    GP_HIP(hipMemcpy(w.data(), f->d, w.size() * sizeof(int64_t), hipMemcpyDeviceToHost));
-    const double inv = f->scale > 0 ? 1.0 / f->scale : 0.0;
-    for (size_t i = 0; i < np; ++i) {
-        if (xyz) {
-            xyz[3 * i + 0] = (double)w[4 * i + 0] * inv;
-            xyz[3 * i + 1] = (double)w[4 * i + 1] * inv;
-            xyz[3 * i + 2] = (double)w[4 * i + 2] * inv;
-        }
-        if (hits) hits[i] = (double)w[4 * i + 3];
-    }
-    return GP_OK;
+    return downloadTotals(*f, xyz, hits, device().stream);
 }
 
 gp_status gp_film_download_hits(gp_film* f, double* hits) {
     if (!f || !hits) return fail(GP_ERR_INVALID, "null argument");
-    const size_t np = (size_t)f->rx * f->ry;
-    std::vector<int64_t> h(np);
-    // the fourth word of every pixel: a strided copy of 8 of each 32 bytes
-    GP_HIP(hipMemcpy2D(h.data(), sizeof(int64_t), f->d + 3, 4 * sizeof(int64_t), sizeof(int64_t), np,
-                       hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < np; ++i) hits[i] = (double)h[i];
-    return GP_OK;
+    return downloadTotals(*f, nullptr, hits, device().stream);
 }
 
 gp_status gp_film_seed(gp_film* f, gp_scene* s, const gp_camera_desc* cam, const gp_trace_params* p,

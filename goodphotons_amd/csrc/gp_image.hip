@@ -218,12 +218,33 @@ gp_status filmNorm(const gp_film* f, int64_t nPhotons, double& inv, double& norm
     return GP_OK;
 }
 
+// Film words to doubles, written straight to pinned host memory (or device memory): thread i
+// converts word i of the pixels' X, Y, Z and, past those, of their hit counts, so that the
+// stores of a wave are contiguous in either array. Bound by the link to the host (52 GB/s);
+// the same multiply on the host, over int64 words copied to pageable memory first, took
+// 8 ms of a 1024 x 1024 render and 22 ms of the 48 of a batch of 16 frames.
+__global__ void __launch_bounds__(256) k_film_totals(const long long* __restrict__ film, size_t n, double inv,
+                                                     double* __restrict__ xyz, double* __restrict__ hits) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x, first = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (xyz)
+        for (size_t i = first; i < 3 * n; i += stride) xyz[i] = (double)film[4 * (i / 3) + i % 3] * inv;
+    if (hits)
+        for (size_t i = first; i < n; i += stride) hits[i] = (double)film[4 * i + 3];
+}
+
 int gridFor(size_t n) {
     size_t b = (n + 255) / 256;
     return (int)(b < 4096 ? (b > 0 ? b : 1) : 4096);
 }
 
 }  // namespace
+
+void launchFilmTotals(const unsigned long long* film, size_t n, double inv, double* xyz, double* hits, hipStream_t s) {
+    // 512 workgroups keep the link busy and leave the rest of the chip to other streams
+    const size_t b = std::min<size_t>(512, std::max<size_t>(1, (3 * n + 255) / 256));
+    hipLaunchKernelGGL(k_film_totals, dim3((unsigned)b), dim3(256), 0, s, (const long long*)film, n, inv, xyz, hits);
+}
+
 }  // namespace gp
 
 using namespace gp;

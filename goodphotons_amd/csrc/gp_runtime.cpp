@@ -59,6 +59,73 @@ gp_status requireDevice() {
     return GP_OK;
 }
 
+// ------------------------------------------------------------------ staging
+Staging& staging() {
+    static Staging g;
+    return g;
+}
+
+gp_status Staging::ready() {
+    if (host) return GP_OK;
+    hipError_t e = hipHostMalloc((void**)&host, kSlot * kSlots);
+    if (e != hipSuccess) {
+        host = nullptr;
+        return fail(GP_ERR_OOM, std::string("staging memory: ") + hipGetErrorString(e));
+    }
+    for (hipEvent_t& v : ev)
+        if ((e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) != hipSuccess) {
+            v = nullptr;
+            free();
+            return fail(GP_ERR_HIP, std::string("staging event: ") + hipGetErrorString(e));
+        }
+    return GP_OK;
+}
+
+void Staging::free() {
+    for (hipEvent_t& v : ev) {
+        if (v) hipEventDestroy(v);
+        v = nullptr;
+    }
+    if (host) hipHostFree(host);
+    host = nullptr;
+}
+
+StagingUse::StagingUse() { ++staging().users; }
+
+StagingUse::~StagingUse() {
+    Staging& g = staging();
+    if (--g.users > 0) return;
+    std::lock_guard<std::mutex> lock(g.mu);
+    if (g.users == 0) g.free();
+}
+
+gp_status copyDown(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    return stagedDown(
+        bytes, 1, s,
+        [&](char* slot, size_t first, size_t n) {
+            return hipMemcpyAsync(slot, (const char*)src + first, n, hipMemcpyDeviceToHost, s);
+        },
+        [&](const char* slot, size_t first, size_t n) { std::memcpy((char*)dst + first, slot, n); });
+}
+
+gp_status downloadTotals(const gp_film& f, double* xyz, double* hits, hipStream_t s) {
+    const size_t each = (xyz ? 24 : 0) + (hits ? 8 : 0);
+    if (each == 0) return GP_OK;
+    const double inv = f.scale > 0 ? 1.0 / f.scale : 0.0;
+    return stagedDown(
+        (size_t)f.rx * f.ry, each, s,
+        [&](char* slot, size_t first, size_t n) {
+            double* x = (double*)slot;
+            launchFilmTotals(f.d + 4 * first, n, inv, xyz ? x : nullptr, hits ? x + (xyz ? 3 * n : 0) : nullptr, s);
+            return hipGetLastError();
+        },
+        [&](const char* slot, size_t first, size_t n) {
+            const double* x = (const double*)slot;
+            if (xyz) std::memcpy(xyz + 3 * first, x, n * 24);
+            if (hits) std::memcpy(hits + first, x + (xyz ? 3 * n : 0), n * 8);
+        });
+}
+
 // ------------------------------------------------------------------ camera
 static void sub3(const double* a, const double* b, double* o) { for (int i = 0; i < 3; ++i) o[i] = a[i] - b[i]; }
 static double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }

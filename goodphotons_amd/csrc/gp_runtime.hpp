@@ -4,6 +4,8 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
@@ -12,6 +14,35 @@
 #include "../../include/goodphotons.h"
 #include "gp_kernels.hpp"
 #include "gp_types.hpp"
+
+namespace gp {
+
+// Pinned host memory through which results leave the device and inputs reach it, in slots
+// filled and emptied in turn. A copy between the device and a caller's pageable array goes
+// through the runtime's own staging in small pieces, one after the other (1 MB: 430 us,
+// 32 MB into fresh pages: 7.8 ms, 14 times the pinned copy); here the device fills a slot
+// while the host empties another.
+// One ring per process, used by one call at a time, allocated by the first and given back
+// with the last scene or film (StagingUse).
+struct Staging {
+    static constexpr size_t kSlot = size_t(2) << 20;
+    static constexpr int kSlots = 4;
+    std::mutex mu;                  // held for a whole transfer
+    char* host = nullptr;           // kSlots * kSlot
+    hipEvent_t ev[kSlots] = {};     // the device is done with the slot
+    std::atomic<int> users{0};
+    gp_status ready();              // allocates (mu held)
+    void free();
+};
+Staging& staging();
+struct StagingUse {
+    StagingUse();
+    ~StagingUse();
+    StagingUse(const StagingUse&) = delete;
+    StagingUse& operator=(const StagingUse&) = delete;
+};
+
+}  // namespace gp
 
 struct gp_scene {
     int64_t nTris = 0;
@@ -45,6 +76,8 @@ struct gp_scene {
     int builder = GP_BVH_HOST_SAH;
     mutable std::map<std::array<double, 3>, double> eyeDist2;
 
+    gp::StagingUse staging;
+
     gp_scene() = default;
     gp_scene(const gp_scene&) = delete;
     gp_scene& operator=(const gp_scene&) = delete;
@@ -59,6 +92,8 @@ struct gp_film {
     unsigned long long qmax = 0;        // largest single splat value
     double splatBudget = 0.0;           // photons*(maxDepth+1) the scale was sized for
     double splatUsed = 0.0;
+
+    gp::StagingUse staging;
 
     gp_film() = default;
     gp_film(const gp_film&) = delete;
@@ -89,6 +124,52 @@ struct DeviceState {
 };
 DeviceState& device();
 gp_status requireDevice();
+
+// Moves `items` items of `each` bytes from the device: fill(slot, first, count) enqueues on
+// s what writes items [first, first + count) to the pinned slot, drain(slot, first, count)
+// takes them on the host. Returns when all are drained. One thread drains: what is left of
+// a copy is its page faults in the caller's fresh array (9-14 GB/s), and four threads
+// brought 118 MB of frames from 12.6 to 10.9 ms only.
+template <class Fill, class Drain>
+gp_status stagedDown(size_t items, size_t each, hipStream_t s, Fill&& fill, Drain&& drain) {
+    Staging& g = staging();
+    std::lock_guard<std::mutex> lock(g.mu);
+    gp_status st = g.ready();
+    if (st != GP_OK) return st;
+    const size_t per = std::max<size_t>(1, Staging::kSlot / each), chunks = (items + per - 1) / per;
+    hipError_t e = hipSuccess;
+    if (chunks == 1) {   // an event would cost a small copy more than it orders
+        e = fill(g.host, 0, items);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e == hipSuccess) drain((const char*)g.host, 0, items);
+    }
+    for (size_t c = 0, d = 0; chunks > 1 && d < chunks && e == hipSuccess;) {
+        const bool down = c == chunks || c - d == Staging::kSlots;
+        const size_t chunk = down ? d++ : c++, first = chunk * per, count = std::min(per, items - first);
+        const size_t k = chunk % Staging::kSlots;
+        char* slot = g.host + k * Staging::kSlot;
+        if (down) {
+            e = hipEventSynchronize(g.ev[k]);
+            if (e == hipSuccess) drain((const char*)slot, first, count);
+        } else {
+            e = fill(slot, first, count);
+            if (e == hipSuccess) e = hipEventRecord(g.ev[k], s);
+        }
+    }
+    if (e != hipSuccess) {
+        hipStreamSynchronize(s);   // nothing may still write to the slots
+        return fail(GP_ERR_HIP, std::string("staged copy: ") + hipGetErrorString(e));
+    }
+    return GP_OK;
+}
+// Plain copy of device memory to a caller's array, after the work on s.
+gp_status copyDown(void* dst, const void* src, size_t bytes, hipStream_t s);
+
+// Film words -> the doubles of gp_film_download: pixels [0, n) of `film` to xyz (3 n, may be
+// null) and hits (n, may be null), word * inv and word.
+void launchFilmTotals(const unsigned long long* film, size_t n, double inv, double* xyz, double* hits, hipStream_t s);
+// Those doubles into a caller's arrays (either may be null), after the work on s.
+gp_status downloadTotals(const gp_film& f, double* xyz, double* hits, hipStream_t s);
 
 // Camera basis as the reference's Camera::lookAt (src/camera.h:110-129), in double.
 struct CamBasis {

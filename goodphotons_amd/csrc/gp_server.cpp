@@ -84,7 +84,7 @@ struct gp_server {
         int64_t installSeq = 0;                  // first chunk that ran with the job installed
         unsigned long long remaining = 0;        // photons not yet emitted (last snapshot)
         unsigned long long* accHost = nullptr;   // pinned, kSegs * kAccRow words
-        long long* filmHost = nullptr;           // pinned, res * 4 words
+        double* filmHost = nullptr;              // pinned: XYZ of every pixel, then the hit counts
         hipEvent_t accEv = nullptr, filmEv = nullptr;
     };
     std::map<int64_t, Job> jobs;
@@ -245,8 +245,8 @@ gp_status admit(Engine& E, gp_server* srv) {
 gp_status startRetire(Engine& E, gp_server* srv, gp_server::Job& J, hipEvent_t chunkEv) {
     hipStream_t s = device().stream, cs = device().copyStream;
     J.accHost = (unsigned long long*)srv->pool.get(sizeof(unsigned long long) * kSegs * kAccRow);
-    const size_t filmBytes = (size_t)J.film->rx * J.film->ry * 4 * sizeof(long long);
-    J.filmHost = (long long*)srv->pool.get(filmBytes);
+    const size_t np = (size_t)J.film->rx * J.film->ry;
+    J.filmHost = (double*)srv->pool.get(np * 4 * sizeof(double));
     if (!J.accHost || !J.filmHost) return fail(GP_ERR_OOM, "pinned host buffer allocation failed");
     J.accEv = srv->event();
     J.filmEv = srv->event();
@@ -254,7 +254,8 @@ gp_status startRetire(Engine& E, gp_server* srv, gp_server::Job& J, hipEvent_t c
                           sizeof(unsigned long long) * kSegs * kAccRow, hipMemcpyDeviceToHost, s));
     GP_HIP(hipEventRecord(J.accEv, s));
     GP_HIP(hipStreamWaitEvent(cs, chunkEv, 0));
-    GP_HIP(hipMemcpyAsync(J.filmHost, J.film->d, filmBytes, hipMemcpyDeviceToHost, cs));
+    launchFilmTotals(J.film->d, np, J.film->scale > 0 ? 1.0 / J.film->scale : 0.0, J.filmHost, J.filmHost + 3 * np, cs);
+    GP_HIP(hipGetLastError());
     GP_HIP(hipEventRecord(J.filmEv, cs));
     J.state = JobState::Retiring;
     return GP_OK;
@@ -488,16 +489,8 @@ gp_status gp_server_take_result(gp_server* srv, int64_t jobId, gp_job_result* re
         if (J.filmEv) GP_HIP(hipEventSynchronize(J.filmEv));
         if (J.filmHost && (xyz || hits)) {
             const size_t np = (size_t)J.film->rx * J.film->ry;
-            const double inv = J.film->scale > 0 ? 1.0 / J.film->scale : 0.0;
-            const long long* w = J.filmHost;
-            for (size_t i = 0; i < np; ++i) {
-                if (xyz) {
-                    xyz[3 * i + 0] = (double)w[4 * i + 0] * inv;
-                    xyz[3 * i + 1] = (double)w[4 * i + 1] * inv;
-                    xyz[3 * i + 2] = (double)w[4 * i + 2] * inv;
-                }
-                if (hits) hits[i] = (double)w[4 * i + 3];
-            }
+            if (xyz) std::memcpy(xyz, J.filmHost, np * 3 * sizeof(double));
+            if (hits) std::memcpy(hits, J.filmHost + 3 * np, np * sizeof(double));
         }
         srv->pool.put(J.filmHost);
         J.filmHost = nullptr;
