@@ -261,9 +261,8 @@ struct Engine {
     gp_status runIterations(int n);           // graph replay when possible
     // Whether new photons are emitted in sorted order (set by the caller before
     // runIterations, from the most photons one job of the wavefront emits).
-    void setEmitOrder(uint64_t photons) {
-        q.emitOrder = photons >= kEmitOrderJobMin && capacity >= kEmitOrderMin ? 1 : 0;
-    }
+    bool wantsEmitOrder(uint64_t photons) const { return photons >= kEmitOrderJobMin && capacity >= kEmitOrderMin; }
+    void setEmitOrder(uint64_t photons) { q.emitOrder = wantsEmitOrder(photons) ? 1 : 0; }
     gp_status readCtrl();                     // synchronous copy of the control block and slot 0's rows
 };
 Engine& engine();

@@ -411,7 +411,8 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
         const int need = std::max(0, maxStackNeed - lds);
         const bool connSpill = maxStackNeed > std::max(lds, 24);
         if (need > E.spillDepth || (need > 0) != (E.q.useSpill != 0) || connSpill != (E.q.connUseSpill != 0) ||
-            (mirrors && !E.q.mv[0]) || mirrors != E.mirrorActive || binningFor(E.tun) != (E.q.binned != 0)) {
+            (mirrors && !E.q.mv[0]) || mirrors != E.mirrorActive || binningFor(E.tun) != (E.q.binned != 0) ||
+            E.wantsEmitOrder((uint64_t)maxPhotons) != (E.q.emitOrder != 0)) {
             while (!srv->inflight.empty())
                 if ((st = processOldest(E, srv)) != GP_OK) return st;
             GP_HIP(hipStreamSynchronize(device().stream));
