@@ -117,10 +117,144 @@ gp_status validateSpectrum(const gp_spectrum& s, const char* what, const gp_scen
     return GP_OK;
 }
 
-struct DevBuf {
-    void* p = nullptr;
-    ~DevBuf() { if (p) hipFree(p); }
+// Slots of the staging ring handed out in turn; a slot's results are taken when its turn
+// comes again, or at the end.
+struct Ring {
+    Staging& g;
+    hipStream_t s;
+    unsigned next = 0;
+    bool busy[Staging::kSlots] = {};
+    void* dst[Staging::kSlots] = {};      // where the slot's results go (null: none)
+    size_t bytes[Staging::kSlots] = {};
+    hipError_t settle(int k) {
+        if (!busy[k]) return hipSuccess;
+        busy[k] = false;
+        const hipError_t e = hipEventSynchronize(g.ev[k]);
+        if (e == hipSuccess && dst[k]) std::memcpy(dst[k], g.host + k * Staging::kSlot, bytes[k]);
+        return e;
+    }
+    hipError_t acquire(int& k) {
+        k = (int)(next++ % Staging::kSlots);
+        return settle(k);
+    }
+    hipError_t submitted(int k, void* to = nullptr, size_t n = 0) {
+        busy[k] = true;
+        dst[k] = to;
+        bytes[k] = n;
+        return hipEventRecord(g.ev[k], s);
+    }
+    hipError_t finish() {
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < Staging::kSlots && e == hipSuccess; ++i) e = settle((int)((next + i) % Staging::kSlots));
+        return e;
+    }
+    ~Ring() {
+        for (bool b : busy)
+            if (b) {   // an error: nothing may still use the slots
+                hipStreamSynchronize(s);
+                break;
+            }
+    }
 };
+
+// Rays per kernel. While one batch is traced the host copies the next one's rays to pinned
+// memory, which is what bounds large calls (30 GB/s); batches of 2^18 left the chip idle
+// between the last rays of one and the copy of the next (8 x 101 us of kernels for two million
+// occlusion rays, against 2 x 198). Before, a call allocated device memory for its rays,
+// results and spill (0.1 ms each), uploaded all, traced all and downloaded all.
+// Whole calls: 400,003 closest hits in 50,000 triangles 1.56 -> 1.06 ms, 2,000,003 occlusion
+// queries in 328,000 triangles 2.86 -> 2.42 ms.
+constexpr int64_t kProbeBatch = 1 << 20;
+// One-wave workgroups per CU: the resident ones. The spill area is sized for them.
+constexpr int kProbeWaves = 24;
+
+// A call of at most this many rays is read and answered by the kernel in pinned memory.
+constexpr int64_t kProbeDirect = (int64_t)(Staging::kSlot / 32);
+
+// A probe's input and output arrays and their bytes a ray.
+struct ProbeIo {
+    const void* in[2];
+    size_t inBytes[2];
+    void* out[2];
+    size_t outBytes[2];
+};
+
+template <class Launch>
+gp_status runProbe(gp_scene* s, int64_t n, const ProbeIo& io, int lds, Launch&& launch) {
+    hipStream_t strm = device().stream;
+    Staging& g = staging();
+    std::lock_guard<std::mutex> lock(g.mu);
+    gp_status st = g.ready();
+    if (st != GP_OK) return st;
+    const int64_t batch = std::min(n, kProbeBatch);
+    const int64_t most = (int64_t)kProbeWaves * std::max(1, device().cus);
+    auto blocksFor = [&](int64_t m) { return (int)std::min(most, (m + kExtendThreads - 1) / kExtendThreads); };
+    const int blocks = blocksFor(batch);
+    const int spillDepth = std::max(0, s->stackNeed - lds);
+    const size_t spillBytes = (size_t)blocks * kExtendThreads * (size_t)spillDepth * sizeof(int2);
+    auto pad = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const bool direct = n <= kProbeDirect;
+    size_t off[4] = {}, need = pad(spillBytes);
+    for (int k = 0; k < 4 && !direct; ++k) {
+        off[k] = need;
+        need += pad((size_t)batch * (k < 2 ? io.inBytes[k] : io.outBytes[k - 2]));
+    }
+    char* scratch = nullptr;
+    if (need && (st = g.scratchFor(need, &scratch)) != GP_OK) return st;
+    struct Trim {
+        Staging& g;
+        ~Trim() { g.trim(Staging::kScratch); }
+    } trim{g};
+    int2* spill = (int2*)scratch;
+    if (direct) {
+        char *in = g.host, *out = g.host + Staging::kSlot;
+        for (int k = 0; k < 2; ++k) {
+            if (io.in[k]) std::memcpy(in, io.in[k], (size_t)n * io.inBytes[k]);
+            in += (size_t)n * io.inBytes[k];
+        }
+        char* out1 = out + (size_t)n * io.outBytes[0];
+        launch(g.host, g.host + (size_t)n * io.inBytes[0], out, out1, (unsigned)n, spill, spillDepth, blocks, strm);
+        GP_HIP(hipGetLastError());
+        GP_HIP(hipStreamSynchronize(strm));
+        std::memcpy(io.out[0], out, (size_t)n * io.outBytes[0]);
+        if (io.out[1]) std::memcpy(io.out[1], out1, (size_t)n * io.outBytes[1]);
+        return GP_OK;
+    }
+    Ring ring{g, strm};
+    for (int64_t at = 0; at < n; at += batch) {
+        const size_t m = (size_t)std::min(batch, n - at);
+        for (int k = 0; k < 2; ++k) {
+            const size_t bytes = m * io.inBytes[k];
+            const char* src = (const char*)io.in[k] + (size_t)at * io.inBytes[k];
+            for (size_t o = 0; o < bytes; o += Staging::kSlot) {
+                const size_t c = std::min(Staging::kSlot, bytes - o);
+                int slot;
+                GP_HIP(ring.acquire(slot));
+                char* pinned = g.host + slot * Staging::kSlot;
+                std::memcpy(pinned, src + o, c);
+                GP_HIP(hipMemcpyAsync(scratch + off[k] + o, pinned, c, hipMemcpyHostToDevice, strm));
+                GP_HIP(ring.submitted(slot));
+            }
+        }
+        launch(scratch + off[0], scratch + off[1], scratch + off[2], scratch + off[3], (unsigned)m, spill, spillDepth,
+               blocksFor((int64_t)m), strm);
+        GP_HIP(hipGetLastError());
+        for (int k = 0; k < 2; ++k) {
+            const size_t bytes = m * io.outBytes[k];
+            char* dst = (char*)io.out[k] + (size_t)at * io.outBytes[k];
+            for (size_t o = 0; o < bytes; o += Staging::kSlot) {
+                const size_t c = std::min(Staging::kSlot, bytes - o);
+                int slot;
+                GP_HIP(ring.acquire(slot));
+                GP_HIP(hipMemcpyAsync(g.host + slot * Staging::kSlot, scratch + off[2 + k] + o, c,
+                                      hipMemcpyDeviceToHost, strm));
+                GP_HIP(ring.submitted(slot, dst + o, c));
+            }
+        }
+    }
+    GP_HIP(ring.finish());
+    return GP_OK;
+}
 
 }  // namespace
 }  // namespace gp
@@ -626,43 +760,22 @@ gp_status gp_trace(gp_scene* s, const gp_camera_desc* cam, gp_film* film, const 
 }
 
 // ------------------------------------------------------------------ probes
-static gp_status probeCommon(gp_scene* s, int64_t n, int& blocks, DevBuf& spill, int& spillDepth, int lds) {
-    if (!s || n < 0) return fail(GP_ERR_INVALID, "bad probe arguments");
-    gp_status st = requireDevice();
-    if (st != GP_OK) return st;
-    blocks = std::max(1, device().cus * 8);
-    spillDepth = std::max(0, s->stackNeed - lds);
-    if (spillDepth > 0) {
-        hipError_t e = hipMalloc(&spill.p, (size_t)blocks * 256 * spillDepth * sizeof(int2));
-        if (e != hipSuccess) return fail(GP_ERR_OOM, "probe spill allocation failed");
-    }
-    return GP_OK;
-}
-
 gp_status gp_probe_closest_hit(gp_scene* s, const float* rays, int64_t n, float tmin, int32_t* prim,
                                float* t) {
     if (!rays || !prim || !t) return fail(GP_ERR_INVALID, "null argument");
     Engine& E = engine();
     std::lock_guard<std::mutex> lock(E.mu);
     if (!E.tunSet) { E.tun = defaultTuning(); E.tunSet = true; }
+    if (!s || n < 0) return fail(GP_ERR_INVALID, "bad probe arguments");
+    gp_status st = requireDevice();
+    if (st != GP_OK || n == 0) return st;
     const int lds = E.tun.lds_stack;
-    int blocks = 0, spillDepth = 0;
-    DevBuf spill, dr, dp, dt;
-    gp_status st = probeCommon(s, n, blocks, spill, spillDepth, lds);
-    if (st != GP_OK) return st;
-    if (n == 0) return GP_OK;
-    GP_HIP(hipMalloc(&dr.p, (size_t)n * 6 * sizeof(float)));
-    GP_HIP(hipMalloc(&dp.p, (size_t)n * sizeof(int)));
-    GP_HIP(hipMalloc(&dt.p, (size_t)n * sizeof(float)));
-    hipStream_t strm = device().stream;
-    GP_HIP(hipMemcpyAsync(dr.p, rays, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, strm));
-    launchProbeClosest(s->dNodes, s->dTris, (const float*)dr.p, n, tmin, (int*)dp.p, (float*)dt.p,
-                       (int2*)spill.p, spillDepth, lds, blocks, 256, strm);
-    GP_HIP(hipGetLastError());
-    GP_HIP(hipMemcpyAsync(prim, dp.p, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, strm));
-    GP_HIP(hipMemcpyAsync(t, dt.p, (size_t)n * sizeof(float), hipMemcpyDeviceToHost, strm));
-    GP_HIP(hipStreamSynchronize(strm));
-    return GP_OK;
+    const ProbeIo io{{rays, nullptr}, {6 * sizeof(float), 0}, {prim, t}, {sizeof(int), sizeof(float)}};
+    return runProbe(s, n, io, lds, [&](char* r, char*, char* p, char* d, unsigned m, int2* spill, int depth,
+                                       int blocks, hipStream_t strm) {
+        launchProbeClosest(s->dNodes, s->dTris, (const float*)r, m, tmin, (int*)p, (float*)d, spill, depth, lds,
+                           blocks, strm);
+    });
 }
 
 gp_status gp_probe_any_hit(gp_scene* s, const float* rays, const float* tmax, int64_t n, float tmin,
@@ -671,24 +784,16 @@ gp_status gp_probe_any_hit(gp_scene* s, const float* rays, const float* tmax, in
     Engine& E = engine();
     std::lock_guard<std::mutex> lock(E.mu);
     if (!E.tunSet) { E.tun = defaultTuning(); E.tunSet = true; }
+    if (!s || n < 0) return fail(GP_ERR_INVALID, "bad probe arguments");
+    gp_status st = requireDevice();
+    if (st != GP_OK || n == 0) return st;
     const int lds = E.tun.lds_stack;
-    int blocks = 0, spillDepth = 0;
-    DevBuf spill, dr, dm, dpo;
-    gp_status st = probeCommon(s, n, blocks, spill, spillDepth, lds);
-    if (st != GP_OK) return st;
-    if (n == 0) return GP_OK;
-    GP_HIP(hipMalloc(&dr.p, (size_t)n * 6 * sizeof(float)));
-    GP_HIP(hipMalloc(&dm.p, (size_t)n * sizeof(float)));
-    GP_HIP(hipMalloc(&dpo.p, (size_t)n));
-    hipStream_t strm = device().stream;
-    GP_HIP(hipMemcpyAsync(dr.p, rays, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, strm));
-    GP_HIP(hipMemcpyAsync(dm.p, tmax, (size_t)n * sizeof(float), hipMemcpyHostToDevice, strm));
-    launchProbeAny(s->dNodes, s->dTris, (const float*)dr.p, (const float*)dm.p, n, tmin,
-                   (unsigned char*)dpo.p, (int2*)spill.p, spillDepth, lds, blocks, 256, strm);
-    GP_HIP(hipGetLastError());
-    GP_HIP(hipMemcpyAsync(occ, dpo.p, (size_t)n, hipMemcpyDeviceToHost, strm));
-    GP_HIP(hipStreamSynchronize(strm));
-    return GP_OK;
+    const ProbeIo io{{rays, tmax}, {6 * sizeof(float), sizeof(float)}, {occ, nullptr}, {1, 0}};
+    return runProbe(s, n, io, lds, [&](char* r, char* m0, char* o, char*, unsigned m, int2* spill, int depth,
+                                       int blocks, hipStream_t strm) {
+        launchProbeAny(s->dNodes, s->dTris, (const float*)r, (const float*)m0, m, tmin, (unsigned char*)o, spill,
+                       depth, lds, blocks, strm);
+    });
 }
 
 // ------------------------------------------------------------------ tuning

@@ -95,13 +95,13 @@ void launchBin(const Queues& q, int cur, hipStream_t s);
 void launchFlight(const Queues& q, unsigned n, unsigned lanes, int blocks, hipStream_t s);
 void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s);
 
-// Batch probes over host-provided rays (already on the device).
-void launchProbeClosest(const float4* nodes, const float4* tris, const float* rays, long long n,
-                        float tmin, int* prim, float* t, int2* spill, int spillDepth, int lds,
-                        int blocks, int threads, hipStream_t s);
-void launchProbeAny(const float4* nodes, const float4* tris, const float* rays, const float* tmax,
-                    long long n, float tmin, unsigned char* occ, int2* spill, int spillDepth,
-                    int lds, int blocks, int threads, hipStream_t s);
+// Batch probes of n rays (device or pinned host memory), `blocks` one-wave workgroups with
+// spillDepth spill entries per thread.
+void launchProbeClosest(const float4* nodes, const float4* tris, const float* rays, unsigned n, float tmin,
+                        int* prim, float* t, int2* spill, int spillDepth, int lds, int blocks, hipStream_t s);
+void launchProbeAny(const float4* nodes, const float4* tris, const float* rays, const float* tmax, unsigned n,
+                    float tmin, unsigned char* occ, int2* spill, int spillDepth, int lds, int blocks,
+                    hipStream_t s);
 
 // Stream-ordered job-table updates for a running wavefront. The data travel as
 // kernel arguments (copied at launch), so the host needs no buffer that outlives the

@@ -67,27 +67,39 @@ Staging& staging() {
 
 gp_status Staging::ready() {
     if (host) return GP_OK;
-    hipError_t e = hipHostMalloc((void**)&host, kSlot * kSlots);
-    if (e != hipSuccess) {
+    hipError_t e = hipSuccess;
+    for (hipEvent_t& v : ev)
+        if (!v && (e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) != hipSuccess) {
+            v = nullptr;
+            return fail(GP_ERR_HIP, std::string("staging event: ") + hipGetErrorString(e));
+        }
+    if ((e = hipHostMalloc((void**)&host, kSlot * kSlots)) != hipSuccess) {
         host = nullptr;
         return fail(GP_ERR_OOM, std::string("staging memory: ") + hipGetErrorString(e));
     }
-    for (hipEvent_t& v : ev)
-        if ((e = hipEventCreateWithFlags(&v, hipEventDisableTiming)) != hipSuccess) {
-            v = nullptr;
-            free();
-            return fail(GP_ERR_HIP, std::string("staging event: ") + hipGetErrorString(e));
-        }
     return GP_OK;
 }
 
-void Staging::free() {
-    for (hipEvent_t& v : ev) {
-        if (v) hipEventDestroy(v);
-        v = nullptr;
+gp_status Staging::scratchFor(size_t bytes, char** out) {
+    if (bytes > scratchBytes) {
+        if (scratch) hipFree(scratch);
+        scratchBytes = 0;
+        const hipError_t e = hipMalloc((void**)&scratch, bytes);
+        if (e != hipSuccess) {
+            scratch = nullptr;
+            return fail(GP_ERR_OOM, std::string("scratch memory: ") + hipGetErrorString(e));
+        }
+        scratchBytes = bytes;
     }
-    if (host) hipHostFree(host);
-    host = nullptr;
+    *out = scratch;
+    return GP_OK;
+}
+
+void Staging::trim(size_t most) {
+    if (scratchBytes <= most) return;
+    hipFree(scratch);
+    scratch = nullptr;
+    scratchBytes = 0;
 }
 
 StagingUse::StagingUse() { ++staging().users; }
@@ -96,7 +108,7 @@ StagingUse::~StagingUse() {
     Staging& g = staging();
     if (--g.users > 0) return;
     std::lock_guard<std::mutex> lock(g.mu);
-    if (g.users == 0) g.free();
+    if (g.users == 0) g.trim(Staging::kKeep);
 }
 
 gp_status copyDown(void* dst, const void* src, size_t bytes, hipStream_t s) {
