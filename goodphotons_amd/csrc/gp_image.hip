@@ -9,12 +9,16 @@
 // film bit for bit.
 //
 // The anchor is an exact order statistic: the element at (size_t)(0.99 (n - 1)) of
-// max(r, g, b, 0) over the pixels. It is found by an 8-pass radix select over the
+// max(r, g, b, 0) over the pixels. It is found by a 5-pass radix select over the
 // bit patterns of those non-negative doubles (which order like the values): each
-// pass builds a 256-bin histogram of the next byte among the keys that match the
-// bytes chosen so far, and one workgroup picks the bin holding the k-th key.
+// pass builds an 8192-bin histogram of the next 13 of their 63 bits (11 in the last)
+// among the keys that match the bits chosen so far, and one workgroup picks the bin
+// holding the k-th key. Eight passes of one byte each took 215 us at 1920 x 1080,
+// 65 us now: the first byte is the same for nearly every key (all sign and
+// exponent), so its histogram was one LDS address, while 13 bits reach into the mantissa.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -57,72 +61,94 @@ __device__ __forceinline__ double srgbGamma(double c) {
     return (c <= 0.0031308) ? 12.92 * c : 1.055 * pow(c, 1.0 / 2.4) - 0.055;
 }
 
-// linear sRGB as float (PFM order: the film's own rows) and the anchor keys
-__global__ void k_linear(const long long* __restrict__ film, size_t npix, double inv, double norm,
-                         float* __restrict__ lin, unsigned long long* __restrict__ keys) {
+// Linear sRGB as float (PFM order: the film's own rows): thread i computes channel i % 3 of
+// pixel i / 3, so that a wave stores contiguous floats (to pinned host memory).
+__global__ void __launch_bounds__(256) k_linear(const long long* __restrict__ film, size_t npix, double inv,
+                                                double norm, float* __restrict__ lin) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 3 * npix; i += stride) {
+        double c[3];
+        linearPixel(film, i / 3, inv, norm, c[0], c[1], c[2]);
+        const unsigned k = (unsigned)(i % 3);
+        lin[i] = (float)(k == 0 ? c[0] : (k == 1 ? c[1] : c[2]));
+    }
+}
+
+// Keys of the anchor.
+__global__ void __launch_bounds__(256) k_keys(const long long* __restrict__ film, size_t npix, double inv,
+                                              double norm, unsigned long long* __restrict__ keys) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < npix; i += stride) {
         double r, g, b;
         linearPixel(film, i, inv, norm, r, g, b);
-        if (lin) {
-            lin[3 * i + 0] = (float)r;
-            lin[3 * i + 1] = (float)g;
-            lin[3 * i + 2] = (float)b;
-        }
-        if (keys) {
-            double m = r > g ? r : g;
-            m = m > b ? m : b;
-            // every value <= 0 is the same key (+0.0), so -0.0 cannot sort last
-            keys[i] = m > 0.0 ? (unsigned long long)__double_as_longlong(m) : 0ull;
-        }
+        double m = r > g ? r : g;
+        m = m > b ? m : b;
+        // every value <= 0 is the same key (+0.0), so -0.0 cannot sort last
+        keys[i] = m > 0.0 ? (unsigned long long)__double_as_longlong(m) : 0ull;
     }
 }
 
 struct SelectState {
-    unsigned long long prefix;   // bytes chosen so far
-    unsigned long long mask;     // which bytes are chosen
+    unsigned long long prefix;   // bits chosen so far
+    unsigned long long mask;     // which bits are chosen
     unsigned long long k;        // rank still sought among keys matching the prefix
     unsigned long long pad;
 };
 
-__global__ void __launch_bounds__(256) k_select_hist(const unsigned long long* __restrict__ keys, size_t n,
-                                                     const SelectState* st, int shift,
-                                                     unsigned* __restrict__ hist) {
-    __shared__ unsigned h[256];
-    h[threadIdx.x] = 0;
+constexpr int kSelBits = 13, kSelBins = 1 << kSelBits, kSelPasses = 5;
+inline int selShift(int pass) { return std::max(0, 63 - kSelBits * (pass + 1)); }
+
+constexpr int kHistThreads = 512;
+__global__ void __launch_bounds__(kHistThreads) k_select_hist(const unsigned long long* __restrict__ keys, size_t n,
+                                                              const SelectState* st, int shift,
+                                                              unsigned* __restrict__ hist) {
+    __shared__ unsigned h[kSelBins];
+    for (int b = threadIdx.x; b < kSelBins; b += kHistThreads) h[b] = 0;
     __syncthreads();
     const unsigned long long prefix = st->prefix, mask = st->mask;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const unsigned long long key = keys[i];
-        if ((key & mask) == prefix) atomicAdd(&h[(key >> shift) & 255u], 1u);
+        // in the last pass the upper two of these bits are chosen already, the same in all
+        if ((key & mask) == prefix) atomicAdd(&h[(key >> shift) & (kSelBins - 1)], 1u);
     }
     __syncthreads();
-    if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
+    for (int b = threadIdx.x; b < kSelBins; b += kHistThreads)
+        if (h[b]) atomicAdd(&hist[b], h[b]);
 }
 
-// One workgroup of 256: find the bin holding rank k, narrow the prefix, clear hist.
-__global__ void __launch_bounds__(256) k_select_pick(SelectState* st, int shift, unsigned* hist) {
-    __shared__ unsigned long long scan[256];
+// One workgroup: find the bin holding rank k, narrow the prefix, clear hist.
+constexpr int kPickThreads = 1024;
+__global__ void __launch_bounds__(kPickThreads) k_select_pick(SelectState* st, int shift, unsigned* hist) {
+    constexpr int kPer = kSelBins / kPickThreads;
+    __shared__ unsigned long long scan[kPickThreads];
     const int t = threadIdx.x;
-    const unsigned c = hist[t];
-    scan[t] = c;
+    unsigned c[kPer];
+    unsigned long long sum = 0;
+    for (int k = 0; k < kPer; ++k) {
+        c[k] = hist[t * kPer + k];
+        hist[t * kPer + k] = 0;
+        sum += c[k];
+    }
+    scan[t] = sum;
     __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
+    for (int off = 1; off < kPickThreads; off <<= 1) {
         const unsigned long long v = t >= off ? scan[t - off] : 0ull;
         __syncthreads();
         scan[t] += v;
         __syncthreads();
     }
     const unsigned long long k = st->k;
-    const unsigned long long before = t > 0 ? scan[t - 1] : 0ull;
+    unsigned long long before = t > 0 ? scan[t - 1] : 0ull;
     __syncthreads();
-    if (c > 0 && before <= k && k < scan[t]) {
-        st->k = k - before;
-        st->prefix |= (unsigned long long)t << shift;
-        st->mask |= 255ull << shift;
+    for (int j = 0; j < kPer; ++j) {
+        if (c[j] > 0 && before <= k && k < before + c[j]) {
+            st->k = k - before;
+            st->prefix |= (unsigned long long)(t * kPer + j) << shift;
+            st->mask |= (unsigned long long)(kSelBins - 1) << shift;
+        }
+        before += c[j];
     }
-    hist[t] = 0;
 }
 
 // exposure from the anchor (main.cpp:10305-10338); out[0] = eAuto, out[1] = exposure
@@ -165,14 +191,9 @@ __global__ void k_rgb8(const long long* __restrict__ film, int W, int H, double 
 // than a host copy and memset, so the allocation-free entry point records only
 // kernels on the stream).
 __global__ void __launch_bounds__(256) k_select_init(SelectState* st, unsigned* hist, unsigned long long k) {
-    hist[threadIdx.x] = 0;
+    for (int b = threadIdx.x; b < kSelBins; b += blockDim.x) hist[b] = 0;
     if (threadIdx.x == 0) *st = SelectState{0, 0, k, 0};
 }
-
-struct DevMem {
-    void* p = nullptr;
-    ~DevMem() { if (p) hipFree(p); }
-};
 
 // Scratch memory of the allocation-free tone map (gp_film_tonemap_noalloc): the
 // select state, histogram and exposure, then the anchor keys (8 B per pixel) and the
@@ -180,10 +201,10 @@ struct DevMem {
 // holds its own copy for the life of the process; host code reaches it only through
 // the address hipGetSymbolAddress returns on that device (noAllocScratch).
 constexpr size_t kNoAllocMaxPixels = size_t(1) << 22;   // 2048 x 2048
-constexpr size_t kNoAllocHead = 4096;                   // SelectState, 256 bins, 2 doubles
+constexpr size_t kNoAllocHead = 65536;                  // SelectState, bins, 2 doubles
 constexpr size_t kNoAllocKeys = kNoAllocMaxPixels * sizeof(unsigned long long);
 constexpr size_t kNoAllocBytes = kNoAllocHead + kNoAllocKeys + kNoAllocMaxPixels * 3;
-static_assert(sizeof(SelectState) + 256 * sizeof(unsigned) + 2 * sizeof(double) <= kNoAllocHead, "head");
+static_assert(sizeof(SelectState) + kSelBins * sizeof(unsigned) + 2 * sizeof(double) <= kNoAllocHead, "head");
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
 constexpr int kNoAllocMaxDevices = 64;
@@ -237,6 +258,33 @@ int gridFor(size_t n) {
     return (int)(b < 4096 ? (b > 0 ? b : 1) : 4096);
 }
 
+// The tone map's kernels: select state, histogram and exposure in `head`, then keys and image.
+// Returns where the exposure (automatic, applied) is.
+const double* enqueueTonemap(const gp_film* film, double inv, double norm, double anchor, double expComp, int absolute,
+                             unsigned char* head, unsigned long long* keys, unsigned char* img, hipStream_t s) {
+    const int W = film->rx, H = film->ry;
+    const size_t npix = (size_t)W * H;
+    SelectState* st = (SelectState*)head;
+    unsigned* hist = (unsigned*)(head + sizeof(SelectState));
+    double* expo = (double*)((char*)hist + kSelBins * sizeof(unsigned));
+    const long long* d = (const long long*)film->d;
+    // the previous call's state may still be there: start the select afresh
+    hipLaunchKernelGGL(k_select_init, dim3(1), dim3(256), 0, s, st, hist,
+                       (unsigned long long)(size_t)(0.99 * (double)(npix - 1)));
+    if (!absolute && !(anchor > 0.0)) {
+        hipLaunchKernelGGL(k_keys, dim3(gridFor(npix)), dim3(256), 0, s, d, npix, inv, norm, keys);
+        const unsigned g = (unsigned)std::min<size_t>(512, (npix + kHistThreads - 1) / kHistThreads);
+        for (int pass = 0; pass < kSelPasses; ++pass) {
+            hipLaunchKernelGGL(k_select_hist, dim3(g), dim3(kHistThreads), 0, s, (const unsigned long long*)keys, npix,
+                               (const SelectState*)st, selShift(pass), hist);
+            hipLaunchKernelGGL(k_select_pick, dim3(1), dim3(kPickThreads), 0, s, st, selShift(pass), hist);
+        }
+    }
+    hipLaunchKernelGGL(k_exposure, dim3(1), dim3(64), 0, s, (const SelectState*)st, anchor, expComp, absolute, expo);
+    hipLaunchKernelGGL(k_rgb8, dim3(gridFor(npix)), dim3(256), 0, s, d, W, H, inv, norm, (const double*)expo, img);
+    return expo;
+}
+
 }  // namespace
 
 void launchFilmTotals(const unsigned long long* film, size_t n, double inv, double* xyz, double* hits, hipStream_t s) {
@@ -259,14 +307,16 @@ gp_status gp_film_to_linear(gp_film* film, int64_t n_photons, float* rgb) {
     if ((st = requireDevice()) != GP_OK) return st;
     const size_t npix = (size_t)film->rx * film->ry;
     hipStream_t s = device().stream;
-    DevMem lin;
-    GP_HIP(hipMalloc(&lin.p, npix * 3 * sizeof(float)));
-    hipLaunchKernelGGL(k_linear, dim3(gridFor(npix)), dim3(256), 0, s, (const long long*)film->d, npix, inv,
-                       norm, (float*)lin.p, (unsigned long long*)nullptr);
-    GP_HIP(hipGetLastError());
-    GP_HIP(hipMemcpyAsync(rgb, lin.p, npix * 3 * sizeof(float), hipMemcpyDeviceToHost, s));
-    GP_HIP(hipStreamSynchronize(s));
-    return GP_OK;
+    return stagedDown(
+        npix, 3 * sizeof(float), s,
+        [&](char* slot, size_t first, size_t n) {
+            hipLaunchKernelGGL(k_linear, dim3(std::min(1024, gridFor(3 * n))), dim3(256), 0, s,
+                               (const long long*)film->d + 4 * first, n, inv, norm, (float*)slot);
+            return hipGetLastError();
+        },
+        [&](const char* slot, size_t first, size_t n) {
+            std::memcpy(rgb + 3 * first, slot, n * 3 * sizeof(float));
+        });
 }
 
 gp_status gp_film_tonemap(gp_film* film, int64_t n_photons, double exposure_comp, int32_t absolute,
@@ -276,39 +326,24 @@ gp_status gp_film_tonemap(gp_film* film, int64_t n_photons, double exposure_comp
     if (st != GP_OK) return st;
     if (!rgb8) return fail(GP_ERR_INVALID, "null output");
     if ((st = requireDevice()) != GP_OK) return st;
-    const int W = film->rx, H = film->ry;
-    const size_t npix = (size_t)W * H;
+    const size_t npix = (size_t)film->rx * film->ry;
     hipStream_t s = device().stream;
-    const bool select = !absolute && !(anchor && *anchor > 0.0);
-    DevMem keys, scratch, img;
-    GP_HIP(hipMalloc(&scratch.p, sizeof(SelectState) + 256 * sizeof(unsigned) + 2 * sizeof(double)));
-    SelectState* dst = (SelectState*)scratch.p;
-    unsigned* hist = (unsigned*)((char*)scratch.p + sizeof(SelectState));
-    double* expo = (double*)((char*)hist + 256 * sizeof(unsigned));
-    SelectState h0{0, 0, (unsigned long long)(size_t)(0.99 * (double)(npix - 1)), 0};
-    GP_HIP(hipMemcpyAsync(dst, &h0, sizeof h0, hipMemcpyHostToDevice, s));
-    GP_HIP(hipMemsetAsync(hist, 0, 256 * sizeof(unsigned), s));
-    if (select) {
-        GP_HIP(hipMalloc(&keys.p, npix * sizeof(unsigned long long)));
-        hipLaunchKernelGGL(k_linear, dim3(gridFor(npix)), dim3(256), 0, s, (const long long*)film->d, npix,
-                           inv, norm, (float*)nullptr, (unsigned long long*)keys.p);
-        for (int pass = 0; pass < 8; ++pass) {
-            const int shift = 56 - 8 * pass;
-            hipLaunchKernelGGL(k_select_hist, dim3(gridFor(npix)), dim3(256), 0, s,
-                               (const unsigned long long*)keys.p, npix, (const SelectState*)dst, shift, hist);
-            hipLaunchKernelGGL(k_select_pick, dim3(1), dim3(256), 0, s, dst, shift, hist);
-        }
-    }
-    hipLaunchKernelGGL(k_exposure, dim3(1), dim3(64), 0, s, (const SelectState*)dst,
-                       anchor ? *anchor : 0.0, exposure_comp, (int)absolute, expo);
-    GP_HIP(hipMalloc(&img.p, npix * 3));
-    hipLaunchKernelGGL(k_rgb8, dim3(gridFor(npix)), dim3(256), 0, s, (const long long*)film->d, W, H, inv,
-                       norm, (const double*)expo, (unsigned char*)img.p);
+    Staging& g = staging();
+    std::lock_guard<std::mutex> lock(g.mu);
+    if ((st = g.ready()) != GP_OK) return st;
+    struct Trim {
+        Staging& g;
+        ~Trim() { g.trim(Staging::kScratch); }
+    } trim{g};
+    char* base = nullptr;
+    if ((st = g.scratchFor(kNoAllocHead + npix * (sizeof(unsigned long long) + 3), &base)) != GP_OK) return st;
+    unsigned char* img = (unsigned char*)base + kNoAllocHead + npix * sizeof(unsigned long long);
+    const double* expo = enqueueTonemap(film, inv, norm, anchor ? *anchor : 0.0, exposure_comp, (int)absolute,
+                                        (unsigned char*)base, (unsigned long long*)(base + kNoAllocHead), img, s);
     GP_HIP(hipGetLastError());
+    if ((st = copyDownLocked(g, rgb8, img, npix * 3, s)) != GP_OK) return st;
     double e[2];
-    GP_HIP(hipMemcpyAsync(rgb8, img.p, npix * 3, hipMemcpyDeviceToHost, s));
-    GP_HIP(hipMemcpyAsync(e, expo, sizeof e, hipMemcpyDeviceToHost, s));
-    GP_HIP(hipStreamSynchronize(s));
+    if ((st = copyDownLocked(g, e, expo, sizeof e, s)) != GP_OK) return st;
     if (anchor && !absolute && !(*anchor > 0.0)) *anchor = e[0];
     if (exposure_out) *exposure_out = e[1];
     return GP_OK;
@@ -328,30 +363,10 @@ gp_status gp_film_tonemap_noalloc(gp_film* film, int64_t n_photons, double expos
                                          " pixels exceeds its scratch limit of 4194304 (2048 x 2048)");
     unsigned char* base = nullptr;
     if ((st = noAllocScratch(device().id, &base)) != GP_OK) return st;
-    SelectState* dst = (SelectState*)base;
-    unsigned* hist = (unsigned*)(base + sizeof(SelectState));
-    double* expo = (double*)((char*)hist + 256 * sizeof(unsigned));
-    unsigned long long* keys = (unsigned long long*)(base + kNoAllocHead);
     unsigned char* img = base + kNoAllocHead + kNoAllocKeys;
     hipStream_t s = device().stream;
-    const bool select = !absolute && !(anchor && *anchor > 0.0);
-    // the previous call's state is still in scratch: start the select afresh
-    hipLaunchKernelGGL(k_select_init, dim3(1), dim3(256), 0, s, dst, hist,
-                       (unsigned long long)(size_t)(0.99 * (double)(npix - 1)));
-    if (select) {
-        hipLaunchKernelGGL(k_linear, dim3(gridFor(npix)), dim3(256), 0, s, (const long long*)film->d, npix,
-                           inv, norm, (float*)nullptr, keys);
-        for (int pass = 0; pass < 8; ++pass) {
-            const int shift = 56 - 8 * pass;
-            hipLaunchKernelGGL(k_select_hist, dim3(gridFor(npix)), dim3(256), 0, s,
-                               (const unsigned long long*)keys, npix, (const SelectState*)dst, shift, hist);
-            hipLaunchKernelGGL(k_select_pick, dim3(1), dim3(256), 0, s, dst, shift, hist);
-        }
-    }
-    hipLaunchKernelGGL(k_exposure, dim3(1), dim3(64), 0, s, (const SelectState*)dst,
-                       anchor ? *anchor : 0.0, exposure_comp, (int)absolute, expo);
-    hipLaunchKernelGGL(k_rgb8, dim3(gridFor(npix)), dim3(256), 0, s, (const long long*)film->d, W, H, inv,
-                       norm, (const double*)expo, img);
+    const double* expo = enqueueTonemap(film, inv, norm, anchor ? *anchor : 0.0, exposure_comp, (int)absolute, base,
+                                        (unsigned long long*)(base + kNoAllocHead), img, s);
     GP_HIP(hipGetLastError());
     double e[2];
     GP_HIP(hipMemcpyAsync(rgb8, img, npix * 3, hipMemcpyDeviceToHost, s));

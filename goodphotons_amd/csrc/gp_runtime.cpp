@@ -112,8 +112,15 @@ StagingUse::~StagingUse() {
 }
 
 gp_status copyDown(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    return stagedDown(
-        bytes, 1, s,
+    Staging& g = staging();
+    std::lock_guard<std::mutex> lock(g.mu);
+    const gp_status st = g.ready();
+    return st != GP_OK ? st : copyDownLocked(g, dst, src, bytes, s);
+}
+
+gp_status copyDownLocked(Staging& g, void* dst, const void* src, size_t bytes, hipStream_t s) {
+    return stagedDownLocked(
+        g, bytes, 1, s,
         [&](char* slot, size_t first, size_t n) {
             return hipMemcpyAsync(slot, (const char*)src + first, n, hipMemcpyDeviceToHost, s);
         },

@@ -138,12 +138,9 @@ gp_status requireDevice();
 // takes them on the host. Returns when all are drained. One thread drains: what is left of
 // a copy is its page faults in the caller's fresh array (9-14 GB/s), and four threads
 // brought 118 MB of frames from 12.6 to 10.9 ms only.
+// stagedDownLocked: for a caller that holds g.mu and has called g.ready().
 template <class Fill, class Drain>
-gp_status stagedDown(size_t items, size_t each, hipStream_t s, Fill&& fill, Drain&& drain) {
-    Staging& g = staging();
-    std::lock_guard<std::mutex> lock(g.mu);
-    gp_status st = g.ready();
-    if (st != GP_OK) return st;
+gp_status stagedDownLocked(Staging& g, size_t items, size_t each, hipStream_t s, Fill&& fill, Drain&& drain) {
     const size_t per = std::max<size_t>(1, Staging::kSlot / each), chunks = (items + per - 1) / per;
     hipError_t e = hipSuccess;
     if (chunks == 1) {   // an event would cost a small copy more than it orders
@@ -170,7 +167,15 @@ gp_status stagedDown(size_t items, size_t each, hipStream_t s, Fill&& fill, Drai
     }
     return GP_OK;
 }
+template <class Fill, class Drain>
+gp_status stagedDown(size_t items, size_t each, hipStream_t s, Fill&& fill, Drain&& drain) {
+    Staging& g = staging();
+    std::lock_guard<std::mutex> lock(g.mu);
+    const gp_status st = g.ready();
+    return st != GP_OK ? st : stagedDownLocked(g, items, each, s, fill, drain);
+}
 // Plain copy of device memory to a caller's array, after the work on s.
+gp_status copyDownLocked(Staging& g, void* dst, const void* src, size_t bytes, hipStream_t s);
 gp_status copyDown(void* dst, const void* src, size_t bytes, hipStream_t s);
 
 // Film words -> the doubles of gp_film_download: pixels [0, n) of `film` to xyz (3 n, may be
