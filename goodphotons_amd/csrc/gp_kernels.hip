@@ -841,9 +841,10 @@ __global__ void __launch_bounds__(kShadeThreads, 4) k_shade(Queues q, int cur) {
         unsigned* hist = keyHist[buf];
         const unsigned lk = localKey(bkey);
         const unsigned rank = alive ? atomicAdd(&hist[lk], 1u) : 0u;
-        if (threadIdx.x < kLocalKeys) keyHist[buf ^ 1u][threadIdx.x] = 0u;
         __syncthreads();
         if (threadIdx.x < kLocalKeys) {
+            // after the barrier: every wave has read the last round's ranks in it
+            keyHist[buf ^ 1u][threadIdx.x] = 0u;
             const unsigned lane = threadIdx.x & 63u, own = hist[threadIdx.x];
             unsigned sum = own;
             for (unsigned off = 1; off < 64; off <<= 1) {
