@@ -251,8 +251,8 @@ __device__ __forceinline__ bool makeConnection(const DevCamera& K, unsigned tagJ
 // a wave (k_emit) or workgroup (k_shade): same-address atomics take 12 ns each, and a wave's
 // append for every camera held up both. Six cameras: k_shade 1915 -> 1452 us, k_emit 646 ->
 // 408 us; one camera: k_shade 13.3 -> 12.9 ms on the glass scene, 1137 -> 1087 us on the box.
-// First the cameras the vertex connects to (bit k:
-// camera k; lanes without a vertex pass nCams = 0); called by all lanes of the wave.
+// First the cameras the vertex connects to (bit k: camera k; lanes without a vertex pass
+// nCams = 0); called by all lanes of the wave.
 __device__ __forceinline__ unsigned connectMask(const DevCamera* cams, int nCams, F3 p, F3 n) {
     unsigned mask = 0;
     for (int k = 0; __any(k < nCams); ++k) {

@@ -734,9 +734,12 @@ bool Engine::flies(uint64_t n, int cams) const {
 
 gp_status Engine::fly(unsigned n, int maxDepth) {
     const unsigned cus = (unsigned)std::max(1, device().cus);
-    // one wave per SIMD before a second photon joins a wave
-    unsigned lanes = 4;
-    while (lanes < 64 && (uint64_t)lanes * 4 * cus < n) lanes *= 2;
+    // Three waves per SIMD before a wave takes more photons: fewer lanes a wave shorten its
+    // longest path, more waves share a SIMD's issue slots. 5000 photons at one, two and four
+    // waves: box 316 / 287 / 263 us, six views 1097 / 909 / 799, 100K-triangle soup 618 / 631
+    // / 535; 131072 photons: box 391 / 395 / 436, six views 1985 / 1995 / 2149.
+    unsigned lanes = 1;
+    while (lanes < 64 && (uint64_t)lanes * 12 * cus < n) lanes *= 2;
     const unsigned most = std::min(kFlightWaves * cus, (unsigned)ls.extend);
     launchFlight(q, n, lanes, (int)std::min(most, (n + lanes - 1) / lanes), device().stream);
     GP_HIP(hipGetLastError());
