@@ -10,7 +10,7 @@
 //                          origin cell and direction octant into a third queue
 //   k_extend               closest hit for every live path (four-wide nodes, LDS stack)
 //   k_shade                material scatter, Russian roulette, camera connection,
-//                          survivors compacted into the other queue by wave ballot
+//                          survivors placed in the other queue sorted within the workgroup
 //   k_connect              any-hit for every connection; unoccluded ones splat into
 //                          the int64 fixed-point film with 64-bit atomics
 //   k_flight               (small traces, instead of all the others) whole paths in registers
