@@ -42,7 +42,8 @@ DeviceState& device() {
             return d;
         }
         if (hipSetDevice(0) != hipSuccess || hipStreamCreate(&d.stream) != hipSuccess ||
-            hipStreamCreate(&d.copyStream) != hipSuccess) {
+            hipStreamCreate(&d.copyStream) != hipSuccess ||
+            hipStreamCreateWithFlags(&d.captureStream, hipStreamNonBlocking) != hipSuccess) {
             d.why = "stream creation failed";
             return d;
         }
@@ -654,9 +655,8 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
 
 // One launch, timed with HIP events while gp_tuning.profile is set.
 template <class F>
-gp_status Engine::timed(int k, F&& launch) {
+gp_status Engine::timed(int k, hipStream_t s, F&& launch) {
     if (!tun.profile) { launch(); return GP_OK; }
-    hipStream_t s = device().stream;
     std::array<hipEvent_t, 2> ev;
     GP_HIP(hipEventCreate(&ev[0]));
     GP_HIP(hipEventCreate(&ev[1]));
@@ -667,26 +667,24 @@ gp_status Engine::timed(int k, F&& launch) {
     return GP_OK;
 }
 
-gp_status Engine::enqueueEmit(const LaunchShape& sh) {
-    hipStream_t s = device().stream;
-    return timed(1, [&] {
+gp_status Engine::enqueueEmit(const LaunchShape& sh, hipStream_t s) {
+    return timed(1, s, [&] {
         if (q.emitOrder) launchEmitOrder(q, s);
         launchEmit(q, parity, sh, s);
     });
 }
 
 // Closest hit, scatter and connections of the paths in queue `parity`.
-gp_status Engine::enqueueBounce(const LaunchShape& sh) {
-    hipStream_t s = device().stream;
+gp_status Engine::enqueueBounce(const LaunchShape& sh, hipStream_t s) {
     const int cur = parity;
     gp_status st;
     if (q.binned)
-        if ((st = timed(5, [&] { launchBin(q, cur, s); })) != GP_OK) return st;
-    if ((st = timed(2, [&] { launchExtend(q, cur, sh, s); })) != GP_OK) return st;
-    if ((st = timed(3, [&] { launchShade(q, cur, sh, s); })) != GP_OK) return st;
-    if ((st = timed(4, [&] { launchConnect(q, sh, s); })) != GP_OK) return st;
+        if ((st = timed(5, s, [&] { launchBin(q, cur, s); })) != GP_OK) return st;
+    if ((st = timed(2, s, [&] { launchExtend(q, cur, sh, s); })) != GP_OK) return st;
+    if ((st = timed(3, s, [&] { launchShade(q, cur, sh, s); })) != GP_OK) return st;
+    if ((st = timed(4, s, [&] { launchConnect(q, sh, s); })) != GP_OK) return st;
     if (mirrorActive && q.mv[0])
-        if ((st = timed(4, [&] { launchMirror(q, sh, s); })) != GP_OK) return st;
+        if ((st = timed(4, s, [&] { launchMirror(q, sh, s); })) != GP_OK) return st;
     parity ^= 1;
     return GP_OK;
 }
@@ -705,13 +703,14 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
     // the first iteration connects the emitted photons and the shaded vertices
     sh.connect = blocks(2 * (uint64_t)n * (uint64_t)cams, 256, ls.connect);
     sh.mirror = blocks(2 * (uint64_t)n, kFlightThreads, ls.mirror);
+    hipStream_t s = device().stream;
     gp_status st;
-    if ((st = enqueueEmit(sh)) != GP_OK) return st;
+    if ((st = enqueueEmit(sh, s)) != GP_OK) return st;
     for (int i = 0; i < maxDepth;) {
         const int stop = std::min(maxDepth, i + kOnceChunk);
         for (; i < stop; ++i) {
             q.resetCounts = i > 0 ? 1 : 0;
-            st = enqueueBounce(sh);
+            st = enqueueBounce(sh, s);
             q.resetCounts = 0;
             if (st != GP_OK) return st;
             sh.connect = blocks((uint64_t)n * (uint64_t)cams, 256, ls.connect);
@@ -747,13 +746,12 @@ gp_status Engine::fly(unsigned n, int maxDepth) {
     return readCtrl();
 }
 
-gp_status Engine::enqueueIterations(int n) {
-    hipStream_t s = device().stream;
+gp_status Engine::enqueueIterations(int n, hipStream_t s) {
     gp_status st;
     for (int i = 0; i < n; ++i) {
-        if ((st = timed(0, [&] { launchSchedule(q, parity, s); })) != GP_OK) return st;
-        if ((st = enqueueEmit(ls)) != GP_OK) return st;
-        if ((st = enqueueBounce(ls)) != GP_OK) return st;
+        if ((st = timed(0, s, [&] { launchSchedule(q, parity, s); })) != GP_OK) return st;
+        if ((st = enqueueEmit(ls, s)) != GP_OK) return st;
+        if ((st = enqueueBounce(ls, s)) != GP_OK) return st;
     }
     GP_HIP(hipGetLastError());
     return GP_OK;
@@ -786,15 +784,16 @@ gp_status Engine::collectProfile() {
 gp_status Engine::runIterations(int n) {
     hipStream_t s = device().stream;
     const int K = chunkIterations(tun);
-    if (!tun.use_graph || tun.profile || q.stats || parity != 0 || n < K) return enqueueIterations(n);
+    if (!tun.use_graph || tun.profile || q.stats || parity != 0 || n < K) return enqueueIterations(n, s);
     if (!graph || graphIters != K || graphLds != q.lds || graphMirror != mirrorActive || graphBinned != q.binned ||
         graphEmitOrder != q.emitOrder) {
         if (graph) { hipGraphExecDestroy(graph); graph = nullptr; }
         hipGraph_t g;
-        GP_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        hipStream_t cs = device().captureStream;
+        GP_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
         int saved = parity;
-        gp_status st = enqueueIterations(K);
-        hipError_t ce = hipStreamEndCapture(s, &g);
+        gp_status st = enqueueIterations(K, cs);
+        hipError_t ce = hipStreamEndCapture(cs, &g);
         parity = saved;
         if (st != GP_OK) return st;
         if (ce != hipSuccess) return fail(GP_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(ce));
@@ -812,7 +811,7 @@ gp_status Engine::runIterations(int n) {
         GP_HIP(hipGraphLaunch(graph, s));
         done += K;
     }
-    if (done < n) return enqueueIterations(n - done);
+    if (done < n) return enqueueIterations(n - done, s);
     return GP_OK;
 }
 

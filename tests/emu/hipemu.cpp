@@ -7,6 +7,7 @@
 #include <memory>
 #include <mutex>
 #include <semaphore>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -143,23 +144,43 @@ void runBlock(const std::function<void()>& fn, unsigned bx, unsigned nthreads) {
 }
 
 struct Rec {
+    std::string name;
     std::function<void()> fn;
     dim3 g, b;
 };
-bool gCapturing = false;
-std::vector<Rec> gCapture;
+
+// one launch at a time, whichever thread makes it (blockDim, shared memory)
+std::mutex gRun;
+// streams, events, counts
+std::mutex gState;
+std::map<std::string, long long> gLaunches;
+long long gStreamSyncs = 0;
+void (*gOnCapture)() = nullptr;
+
+bool async() {
+    static const bool on = getenv("EMU_ASYNC") && atoi(getenv("EMU_ASYNC")) != 0;
+    return on;
+}
 
 }  // namespace
 
-struct EmuGraph {
-    std::vector<Rec> recs;
-};
 struct EmuStream {
-    int id;
+    bool capturing = false, invalid = false;
+    std::vector<Rec> captured;
+    unsigned long long enqueued = 0, done = 0;   // pieces of work given and waited for
 };
 struct EmuEvent {
-    int id;
+    EmuStream* s = nullptr;
+    unsigned long long at = 0;
 };
+struct EmuGraph {
+    std::vector<Rec> recs;
+    EmuStream* s = nullptr;   // last launch
+    unsigned long long at = 0;
+};
+
+static EmuStream gNullStream;
+static EmuStream* streamOf(hipStream_t s) { return s ? s : &gNullStream; }
 
 unsigned long long emu_ballot(int pred, void* site) {
     Lane& L = *gLane;
@@ -197,11 +218,53 @@ int emu_sync_or(int pred, void* site) {
     return (int)L.result;
 }
 
-void emu_launch(std::function<void()> fn, dim3 g, dim3 b) {
-    if (gCapturing) { gCapture.push_back({fn, g, b}); return; }
-    gridDim = g;
-    blockDim = b;
-    for (unsigned bx = 0; bx < g.x; ++bx) runBlock(fn, bx, b.x);
+static void runRec(const Rec& r) {
+    std::lock_guard<std::mutex> run(gRun);
+    {
+        std::lock_guard<std::mutex> lock(gState);
+        ++gLaunches[r.name];
+    }
+    gridDim = r.g;
+    blockDim = r.b;
+    for (unsigned bx = 0; bx < r.g.x; ++bx) runBlock(r.fn, bx, r.b.x);
+}
+
+void emu_launch(const char* name, std::function<void()> fn, dim3 g, dim3 b, hipStream_t st) {
+    EmuStream* s = streamOf(st);
+    {
+        std::lock_guard<std::mutex> lock(gState);
+        if (s->capturing) {
+            s->captured.push_back({name, fn, g, b});
+            return;
+        }
+        ++s->enqueued;
+    }
+    runRec({name, fn, g, b});
+}
+
+// Work on a stream that cannot be recorded here (the library captures kernels only).
+static hipError_t enqueueOther(hipStream_t st) {
+    EmuStream* s = streamOf(st);
+    std::lock_guard<std::mutex> lock(gState);
+    if (s->capturing) {
+        s->invalid = true;
+        return hipErrorStreamCaptureUnsupported;
+    }
+    ++s->enqueued;
+    return hipSuccess;
+}
+
+void emu_on_capture(void (*cb)()) { gOnCapture = cb; }
+long long emu_launches(const char* part) {
+    std::lock_guard<std::mutex> lock(gState);
+    long long n = 0;
+    for (auto& kv : gLaunches)
+        if (kv.first.find(part) != std::string::npos) n += kv.second;
+    return n;
+}
+long long emu_stream_syncs() {
+    std::lock_guard<std::mutex> lock(gState);
+    return gStreamSyncs;
 }
 
 static int gEmuCus() {
@@ -248,42 +311,93 @@ hipError_t hipMemcpy2D(void* d, size_t dpitch, const void* s, size_t spitch, siz
         std::memmove((char*)d + r * dpitch, (const char*)s + r * spitch, width);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
-    if (gCapturing) { fprintf(stderr, "EMU: memcpy during capture\n"); abort(); }
-    return hipMemcpy(d, s, n, k);
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t st) {
+    const hipError_t e = enqueueOther(st);
+    return e != hipSuccess ? e : hipMemcpy(d, s, n, k);
 }
 hipError_t hipMemset(void* d, int v, size_t n) { std::memset(d, v, n); return hipSuccess; }
-hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
-    if (gCapturing) { fprintf(stderr, "EMU: memset during capture\n"); abort(); }
-    std::memset(d, v, n);
-    return hipSuccess;
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t st) {
+    const hipError_t e = enqueueOther(st);
+    if (e == hipSuccess) std::memset(d, v, n);
+    return e;
 }
-hipError_t hipStreamCreate(hipStream_t* s) { *s = new EmuStream{1}; return hipSuccess; }
+hipError_t hipStreamCreate(hipStream_t* s) { *s = new EmuStream(); return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return hipStreamCreate(s); }
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t st) {
+    EmuStream* s = streamOf(st);
+    std::lock_guard<std::mutex> lock(gState);
+    ++gStreamSyncs;
+    if (s->capturing) {
+        s->invalid = true;
+        return hipErrorStreamCaptureUnsupported;
+    }
+    s->done = s->enqueued;
+    return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipEventCreate(hipEvent_t* e) { *e = new EmuEvent{1}; return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { *e = new EmuEvent(); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
+    const hipError_t r = enqueueOther(st);
+    if (r != hipSuccess) return r;
+    std::lock_guard<std::mutex> lock(gState);
+    e->s = streamOf(st);
+    e->at = e->s->enqueued;
+    return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+    std::lock_guard<std::mutex> lock(gState);
+    if (e->s && e->s->done < e->at) e->s->done = e->at;
+    return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) {
+    std::lock_guard<std::mutex> lock(gState);
+    return async() && e->s && e->at > e->s->done ? hipErrorNotReady : hipSuccess;
+}
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0.f; return hipSuccess; }
-hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { gCapturing = true; gCapture.clear(); return hipSuccess; }
-hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
-    gCapturing = false;
-    *g = new EmuGraph{gCapture};
-    gCapture.clear();
+hipError_t hipStreamBeginCapture(hipStream_t st, hipStreamCaptureMode) {
+    EmuStream* s = streamOf(st);
+    {
+        std::lock_guard<std::mutex> lock(gState);
+        s->capturing = true;
+        s->invalid = false;
+        s->captured.clear();
+    }
+    if (void (*cb)() = gOnCapture) {
+        gOnCapture = nullptr;
+        cb();
+    }
+    return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t st, hipGraph_t* g) {
+    EmuStream* s = streamOf(st);
+    std::lock_guard<std::mutex> lock(gState);
+    s->capturing = false;
+    if (s->invalid) { *g = nullptr; return hipErrorStreamCaptureInvalidated; }
+    *g = new EmuGraph{s->captured};
+    s->captured.clear();
     return hipSuccess;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t) {
     *e = new EmuGraph{g->recs};
     return hipSuccess;
 }
-hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t) {
-    for (auto& r : e->recs) emu_launch(r.fn, r.g, r.b);
+hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t st) {
+    const hipError_t r = enqueueOther(st);
+    if (r != hipSuccess) return r;
+    e->s = streamOf(st);
+    e->at = e->s->enqueued;
+    for (auto& rec : e->recs) runRec(rec);
     return hipSuccess;
 }
 hipError_t hipGraphDestroy(hipGraph_t g) { delete g; return hipSuccess; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete e; return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) {
+    if (async() && e->s && e->at > e->s->done) {
+        fprintf(stderr, "EMU: graph destroyed while it runs\n");
+        abort();
+    }
+    delete e;
+    return hipSuccess;
+}

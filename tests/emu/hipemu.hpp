@@ -10,6 +10,13 @@
 // AddressSanitizer bounds-checks every kernel access. With EMU_PREEMPT=k a lane gives up
 // the baton at every k-th preemption point (each __float_as_int, which the traversal
 // loops call per node), so lanes of a block interleave inside loops as waves do.
+//
+// Streams run what they are given at once, but keep the GPU's rules where the library's
+// host code depends on them. A stream that is captured records its launches, whichever
+// thread makes them, and synchronising it ends the capture in an error. With EMU_ASYNC=1
+// work counts as running until its stream or an event behind it has been waited for
+// (hipEventQuery says not ready until then), and destroying a graph that is still running
+// aborts. emu_on_capture, emu_launches and emu_stream_syncs serve the tests.
 #pragma once
 #include <cmath>
 #include <cstddef>
@@ -112,7 +119,7 @@ template <class T> inline T max(T a, T b) { return a > b ? a : b; }
 // ---------------------------------------------------------------- runtime
 typedef enum hipError_t {
     hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorNotReady = 600,
-    hipErrorUnknown = 999
+    hipErrorStreamCaptureUnsupported = 900, hipErrorStreamCaptureInvalidated = 901, hipErrorUnknown = 999
 } hipError_t;
 typedef enum hipMemcpyKind {
     hipMemcpyHostToHost = 0, hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2,
@@ -129,6 +136,7 @@ typedef EmuGraph* hipGraph_t;
 typedef EmuGraph* hipGraphExec_t;
 typedef struct hipGraphNode* hipGraphNode_t;
 #define hipEventDisableTiming 2
+#define hipStreamNonBlocking 1
 struct hipDeviceProp_t {
     char name[256];
     char gcnArchName[256];
@@ -180,12 +188,21 @@ hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s);
 hipError_t hipGraphDestroy(hipGraph_t g);
 hipError_t hipGraphExecDestroy(hipGraphExec_t e);
 
-void emu_launch(std::function<void()> fn, dim3 g, dim3 b);
+void emu_launch(const char* name, std::function<void()> fn, dim3 g, dim3 b, hipStream_t s);
 
 template <class... P, class... A>
-void emu_launch_kernel(void (*k)(P...), dim3 g, dim3 b, A&&... a) {
+void emu_launch_kernel(const char* name, void (*k)(P...), dim3 g, dim3 b, hipStream_t s, A&&... a) {
     std::tuple<std::decay_t<P>...> args(static_cast<std::decay_t<P>>(std::forward<A>(a))...);
-    emu_launch([k, args]() { std::apply(k, args); }, g, b);
+    emu_launch(name, [k, args]() { std::apply(k, args); }, g, b, s);
 }
-#define hipLaunchKernelGGL(K, G, B, SH, ST, ...) emu_launch_kernel(K, dim3(G), dim3(B), ##__VA_ARGS__)
+#define hipLaunchKernelGGL(K, G, B, SH, ST, ...) emu_launch_kernel(#K, K, dim3(G), dim3(B), ST, ##__VA_ARGS__)
 #define HIP_SYMBOL(x) (&(x))
+
+extern "C" {
+// Calls cb once, inside the next hipStreamBeginCapture.
+void emu_on_capture(void (*cb)());
+// Launches (captured ones each time their graph runs) of kernels whose name contains `part`.
+long long emu_launches(const char* part);
+// hipStreamSynchronize calls.
+long long emu_stream_syncs();
+}

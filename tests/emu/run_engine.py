@@ -1,0 +1,72 @@
+"""Test infrastructure only: the engine's host code through the emulation build (child
+process, started with the AddressSanitizer runtime preloaded by
+tests/test_emulated_engine.py). argv: the scenario. Prints JSON on the last line."""
+import ctypes as C
+import json
+import os
+import sys
+import threading
+
+import numpy as np
+
+ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+sys.path.insert(0, ROOT)
+
+import goodphotons_amd as gp  # noqa: E402
+from goodphotons_amd import scenes  # noqa: E402
+
+lib = gp.Library(os.environ["EMU_LIB"])
+emu = lib.lib
+emu.emu_launches.restype = C.c_longlong
+emu.emu_launches.argtypes = [C.c_char_p]
+emu.emu_stream_syncs.restype = C.c_longlong
+KEYS = ("photons", "segments", "connections", "splats")
+
+
+def counts(st):
+    return [int(getattr(st, k)) for k in KEYS]
+
+
+def film_of(sd, n):
+    return gp.Film(sd.camera.res_x, sd.camera.res_y, max_photons=n, lib=lib)
+
+
+def capture():
+    """A film is downloaded and another seeded by a second thread while the first captures
+    the graph of a trace that is refilled."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
+    sd = scenes.cornell_c0(32)
+    gs = gp.GpuScene(sd, lib)
+    other = film_of(sd, 1000)
+    gp.trace(gs, sd.camera, other, 1000, max_depth=4)
+    xyz, hits = other.download()
+    seen = {}
+
+    def side():
+        try:
+            x, h = other.download()
+            fresh = film_of(sd, 1000)
+            fresh.seed(gs, sd.camera, 1000, xyz, hits, max_depth=4)
+            y, g = fresh.download()
+            seen["same"] = bool(np.array_equal(x, xyz) and np.array_equal(h, hits) and np.array_equal(g, hits))
+        except gp.GpError as e:
+            seen["error"] = str(e)
+
+    def during():
+        t = threading.Thread(target=side)
+        t.start()
+        t.join()
+
+    cb = C.CFUNCTYPE(None)(during)
+    emu.emu_on_capture(cb)
+    n = 5001
+    got = []
+    for _ in range(2):   # captured, then replayed
+        f = film_of(sd, n)
+        _, st = gp.trace(gs, sd.camera, f, n, max_depth=4)
+        got.append((f.raw()[0], counts(st)))
+    return {"seen": seen, "counts": got[0][1], "hits": got[0][0][:, 3].tolist(),
+            "same": bool(np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1])}
+
+
+print(json.dumps({"capture": capture}[sys.argv[1]]()))

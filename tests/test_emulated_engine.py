@@ -1,0 +1,63 @@
+"""The engine's host code and the kernels that the other emulated cases do not reach, on
+the CPU under AddressSanitizer (tests/emu): what the host may do to streams and graphs
+while work runs on them, and which kernels a call runs.
+
+Exact equality throughout, except where the oracle's film is compared.
+"""
+import json
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from goodphotons_amd import scenes
+from tests.emu import build as emu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+pytestmark = pytest.mark.skipif(not emu.available(), reason="clang++ with AddressSanitizer not found")
+
+
+def _run(scenario, lib, cus, preempt=0, run_async=0):
+    env = dict(os.environ)
+    env.update({"LD_PRELOAD": emu.asan_runtime(), "ASAN_OPTIONS": "detect_leaks=0", "EMU_CUS": str(cus),
+                "EMU_PREEMPT": str(preempt), "EMU_ASYNC": str(run_async), "EMU_LIB": lib})
+    return subprocess.Popen([sys.executable, os.path.join(ROOT, "tests", "emu", "run_engine.py"), scenario],
+                            stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, env=env)
+
+
+# Each scenario is a child process of its own; all are started at once.
+CASES = {
+    "capture": dict(cus=1),
+}
+
+
+@pytest.fixture(scope="module")
+def runs():
+    lib = emu.build()
+    procs = {k: _run(k, lib, **kw) for k, kw in CASES.items()}
+    yield procs
+    for p in procs.values():
+        if p.poll() is None:
+            p.kill()
+            p.wait()
+
+
+def _result(runs, key):
+    out, err = runs[key].communicate(timeout=900)
+    assert runs[key].returncode == 0, err[-3000:]
+    return json.loads(out.strip().splitlines()[-1])
+
+
+def test_film_calls_of_another_thread_stay_out_of_a_graph_capture(runs, orc):
+    # a download and a seed that fall into the capture of a trace's graph neither fail nor
+    # end up in the graph, and the trace holds the oracle's photons
+    out = _result(runs, "capture")
+    assert out["seen"] == {"same": True}
+    assert out["same"]
+    sd = scenes.cornell_c0(32)
+    _, h, _, st = orc.render(orc.scene(sd), sd.camera, 5001, hero_c=4, max_bounce=4, threads=8)
+    assert out["counts"] == [5001] + [st[k] for k in ("segments", "connections", "splats")]
+    assert np.array_equal(np.array(out["hits"]), h)
