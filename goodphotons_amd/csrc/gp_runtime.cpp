@@ -508,43 +508,53 @@ void addCounters(const unsigned long long* cv, gp_trace_stats& st) {
 
 bool binningFor(const gp_tuning& t) { return t.ray_sort == 1; }
 
-gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mirrors) {
-    if (!tunSet) { tun = defaultTuning(); tunSet = true; }
+Engine::Shape Engine::shapeFor(unsigned cap, int lds, int stackNeed, int cams, bool mirrors) const {
     DeviceState& d = device();
     const int cus = d.cus > 0 ? d.cus : 256;
     const int blocks = std::max(1, cus * tun.grid_waves_per_cu / 4);
-    ls.emit = ls.connect = blocks;
-    ls.mirror = blocks * (256 / kFlightThreads);
-    ls.shade = (blocks * 256 + kShadeThreads - 1) / kShadeThreads;
-    ls.extend = blocks * kExtendGridScale * (256 / kExtendThreads);
-    const size_t threads = (size_t)ls.extend * kExtendThreads;
+    Shape p;
+    p.ls.emit = p.ls.connect = blocks;
+    p.ls.mirror = blocks * (256 / kFlightThreads);
+    p.ls.shade = (blocks * 256 + kShadeThreads - 1) / kShadeThreads;
+    p.ls.extend = blocks * kExtendGridScale * (256 / kExtendThreads);
+    p.threads = (size_t)p.ls.extend * kExtendThreads;
     // k_emit appends connections and k_shade paths and connections, each over its own grid
-    const unsigned sc = std::max(segmentBound(cap, (unsigned)ls.emit, 256),
-                                 segmentBound(cap, (unsigned)ls.shade, kShadeThreads));
-    const int camsNeed = std::max(camCap, std::max(1, cams));
-    const bool needQueues = (cap != capacity) || sc != segCap || camsNeed != camCap || !dCtrl;
-    const bool wantMirror = mirrors || mirrorQueue;
-    const bool needMirrorAlloc = wantMirror && (needQueues || !q.mv[0]);
-    const int binned = binningFor(tun) ? 1 : 0;
-    const bool needBinAlloc = binned && (needQueues || !q.pb);
+    // (the bound is a loop over the queue's workgroups: kept while the grids are the same)
+    const bool kept = dCtrl && cap == capacity && p.ls.emit == ls.emit && p.ls.shade == ls.shade;
+    p.segCap = kept ? segCap : std::max(segmentBound(cap, (unsigned)p.ls.emit, 256),
+                                        segmentBound(cap, (unsigned)p.ls.shade, kShadeThreads));
+    p.cams = std::max(camCap, std::max(1, cams));
+    p.queues = (cap != capacity) || p.segCap != segCap || p.cams != camCap || !dCtrl;
+    p.mirrorAlloc = (mirrors || mirrorQueue) && (p.queues || !q.mv[0]);
+    p.binned = binningFor(tun) ? 1 : 0;
+    p.binAlloc = p.binned && (p.queues || !q.pb);
     // Entries beyond the LDS stack live in the spill area (stack index sp >= SD maps to
     // spill[sp - SD], and sp < stackNeed). k_connect keeps as many entries in LDS as the
     // closest-hit kernel, 8 for its 12 (4-byte entries: at 8, six waves per SIMD fit its
     // LDS; 12 or 16 leave room for five, 24 for four), and so does k_mirror. The spill area
     // covers the shallower of the two.
-    const int connLds = lds == 12 ? 8 : lds;
-    const int needSpill = std::max(0, stackNeed - std::min(lds, connLds));
-    const int connUseSpill = stackNeed > connLds ? 1 : 0;
-    const bool needSpillAlloc = needSpill > spillDepth || (needSpill > 0 && threads > spillThreads);
+    p.connLds = lds == 12 ? 8 : lds;
+    p.needSpill = std::max(0, stackNeed - std::min(lds, p.connLds));
+    p.connUseSpill = stackNeed > p.connLds ? 1 : 0;
+    p.spillAlloc = p.needSpill > spillDepth || (p.needSpill > 0 && p.threads > spillThreads);
     // The kernels without spill code keep the whole stack in LDS: they may only run
     // when every traced scene fits. A change of variant re-captures the graph.
-    const int useSpill = needSpill > 0 ? 1 : 0;
-    if (!needQueues && !needSpillAlloc && !needMirrorAlloc && !needBinAlloc && q.lds == lds &&
-        q.useSpill == useSpill && q.connLds == connLds && q.connUseSpill == connUseSpill &&
-        graphShape == ls.extend && q.binned == binned)
-        return GP_OK;
+    p.useSpill = p.needSpill > 0 ? 1 : 0;
+    p.same = !p.queues && !p.spillAlloc && !p.mirrorAlloc && !p.binAlloc && q.lds == lds &&
+             q.useSpill == p.useSpill && q.connLds == p.connLds && q.connUseSpill == p.connUseSpill &&
+             graphShape == p.ls.extend && q.binned == p.binned;
+    return p;
+}
+
+gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mirrors) {
+    if (!tunSet) { tun = defaultTuning(); tunSet = true; }
+    const Shape p = shapeFor(cap, lds, stackNeed, cams, mirrors);
+    ls = p.ls;
+    if (p.same) return GP_OK;
+    const unsigned sc = p.segCap;
+    const int cus = device().cus > 0 ? device().cus : 256;
     if (graph) { hipGraphExecDestroy(graph); graph = nullptr; }
-    if (needQueues) {
+    if (p.queues) {
         releaseQueues();
         auto alloc = [&](size_t bytes, void** out) -> gp_status {
             hipError_t e = hipMalloc(out, bytes);
@@ -565,7 +575,7 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
         // Connections per iteration and camera: one per emitted photon (direct view of
         // the light) plus at most one per live path; k_emit and k_shade run the same
         // grid, so a segment receives at most segCap of each per camera.
-        const size_t ccap = 2 * pcap * (size_t)camsNeed;
+        const size_t ccap = 2 * pcap * (size_t)p.cams;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.co)) != GP_OK) return st;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.cd)) != GP_OK) return st;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.cx)) != GP_OK) return st;
@@ -587,11 +597,11 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
         q.ctrl = dCtrl;
         q.jobs = dJobs;
         q.segCap = sc;
-        q.connSegCap = 2 * sc * (unsigned)camsNeed;
+        q.connSegCap = 2 * sc * (unsigned)p.cams;
         q.mirrorSegCap = 2 * sc;
-        camCap = camsNeed;
+        camCap = p.cams;
     }
-    if (needMirrorAlloc) {
+    if (p.mirrorAlloc) {
         // one vertex per emitted photon and per shaded path, like the connections of
         // one camera
         const size_t mcap = 2 * (size_t)kSegs * segCap;
@@ -609,44 +619,44 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
         }
         mirrorQueue = true;
     }
-    if (needBinAlloc) {
+    if (p.binAlloc) {
         // the binned path queue (same slots as the others, 80-byte records), the keys of
         // both path queues and the counting-sort tables
         const size_t pcap = (size_t)kSegs * segCap;
-        void* p[6] = {};
+        void* part[6] = {};
         const size_t bytes[6] = {pcap * 5 * sizeof(float4), pcap * sizeof(unsigned short),
                                  pcap * sizeof(unsigned short), (size_t)kBinCols * kBins * sizeof(unsigned),
                                  (size_t)kBinChunks * kBins * sizeof(unsigned), (size_t)kBins * sizeof(unsigned)};
         for (int k = 0; k < 6; ++k) {
-            hipError_t e = hipMalloc(&p[k], bytes[k]);
+            hipError_t e = hipMalloc(&part[k], bytes[k]);
             if (e != hipSuccess) {
-                for (int i = 0; i < k; ++i) hipFree(p[i]);
+                for (int i = 0; i < k; ++i) hipFree(part[i]);
                 return fail(GP_ERR_OOM, std::string("hipMalloc: ") + hipGetErrorString(e));
             }
         }
-        for (int k = 0; k < 6; ++k) bufs[nbufs++] = p[k];
-        q.pb = (float4*)p[0];
-        q.key[0] = (unsigned short*)p[1];
-        q.key[1] = (unsigned short*)p[2];
-        q.binHist = (unsigned*)p[3];
-        q.binChunk = (unsigned*)p[4];
-        q.binTotal = (unsigned*)p[5];
+        for (int k = 0; k < 6; ++k) bufs[nbufs++] = part[k];
+        q.pb = (float4*)part[0];
+        q.key[0] = (unsigned short*)part[1];
+        q.key[1] = (unsigned short*)part[2];
+        q.binHist = (unsigned*)part[3];
+        q.binChunk = (unsigned*)part[4];
+        q.binTotal = (unsigned*)part[5];
     }
-    if (needSpillAlloc) {
-        const int depthAlloc = std::max(needSpill, spillDepth);
+    if (p.spillAlloc) {
+        const int depthAlloc = std::max(p.needSpill, spillDepth);
         if (q.spill) hipFree(q.spill);
         q.spill = nullptr;
-        hipError_t e = hipMalloc(&q.spill, threads * (size_t)depthAlloc * sizeof(int2));
+        hipError_t e = hipMalloc(&q.spill, p.threads * (size_t)depthAlloc * sizeof(int2));
         if (e != hipSuccess) { spillDepth = 0; spillThreads = 0; return fail(GP_ERR_OOM, "spill stack allocation failed"); }
         spillDepth = depthAlloc;
-        spillThreads = threads;
+        spillThreads = p.threads;
     }
     q.spillDepth = spillDepth;
     q.lds = lds;
-    q.useSpill = useSpill;
-    q.connLds = connLds;
-    q.connUseSpill = connUseSpill;
-    q.binned = binned;
+    q.useSpill = p.useSpill;
+    q.connLds = p.connLds;
+    q.connUseSpill = p.connUseSpill;
+    q.binned = p.binned;
     q.binCols = std::min(kBinCols, std::max(kBinColStep, (cus * 4) / kBinColStep * kBinColStep));
     static_assert(kBinColStep % kBinChunks == 0 && kBinCols % kBinColStep == 0, "binning column shape");
     graphShape = ls.extend;

@@ -252,6 +252,18 @@ struct Engine {
     void resetProfile();
     gp_status collectProfile();
 
+    // What a call asks of the engine: launch grids, queue and spill sizes, kernel variants, and
+    // what of it has to be allocated. same: nothing changes; otherwise ensure() drops the
+    // graph and may re-allocate, so no chunk may be in flight.
+    struct Shape {
+        LaunchShape ls{};
+        unsigned segCap = 0;
+        int cams = 0;
+        size_t threads = 0;             // of the closest-hit kernel (spill rows)
+        int connLds = 0, needSpill = 0, useSpill = 0, connUseSpill = 0, binned = 0;
+        bool queues = false, mirrorAlloc = false, binAlloc = false, spillAlloc = false, same = false;
+    };
+    Shape shapeFor(unsigned cap, int lds, int stackNeed, int cams, bool mirrors) const;
     // stackNeed: traversal stack entries the traced scenes can need (gp_scene::stackNeed);
     // mirrors: allocate the mirror-vertex queue (kept from then on, like the camera count)
     gp_status ensure(unsigned cap, int lds, int stackNeed, int cams = 1, bool mirrors = false);

@@ -407,12 +407,10 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
     }
     const int lds = E.tun.lds_stack;
     if (srv->engineReady && !srv->inflight.empty()) {
-        // a change of engine shape would re-allocate under running chunks
-        const int need = std::max(0, maxStackNeed - lds);
-        const bool connSpill = maxStackNeed > std::max(lds, 24);
-        if (need > E.spillDepth || (need > 0) != (E.q.useSpill != 0) || connSpill != (E.q.connUseSpill != 0) ||
-            (mirrors && !E.q.mv[0]) || mirrors != E.mirrorActive || binningFor(E.tun) != (E.q.binned != 0) ||
-            E.wantsEmitOrder((uint64_t)maxPhotons) != (E.q.emitOrder != 0)) {
+        // a change of engine shape re-allocates, and one of the iteration's kernels drops the
+        // graph: neither may happen under running chunks
+        if (!E.shapeFor((unsigned)E.tun.queue_capacity, lds, maxStackNeed, 1, mirrors).same ||
+            mirrors != E.mirrorActive || E.wantsEmitOrder((uint64_t)maxPhotons) != (E.q.emitOrder != 0)) {
             while (!srv->inflight.empty())
                 if ((st = processOldest(E, srv)) != GP_OK) return st;
             GP_HIP(hipStreamSynchronize(device().stream));

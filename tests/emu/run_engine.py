@@ -69,4 +69,48 @@ def capture():
             "same": bool(np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1])}
 
 
-print(json.dumps({"capture": capture}[sys.argv[1]]()))
+def nest(n):
+    """n triangles, each half the size of the last, nested into a corner: a tree that grows
+    by about a level a triangle."""
+    sd = scenes.soup(n, 4, res=8)
+    corner = np.array([1, 0, 0, 1.2, 0.2, 0, 1, 0.2, 0.2])
+    v = np.array(sd.verts, np.float32).reshape(-1, 9)
+    v[:n] = corner[None] * (0.4 * 0.5 ** np.arange(n))[:, None] + 0.5
+    sd.verts = v.reshape(np.shape(sd.verts))
+    return sd
+
+
+def reshape():
+    """A server that is given a deeper tree at every step, with chunks in flight (EMU_ASYNC:
+    the emulator aborts if a graph is destroyed under one); then steps that change nothing."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2, lds_stack=12)
+    depths, same = [], True
+    sds = [nest(n) for n in (8, 12, 14, 16, 18, 20, 22, 24, 28, 32)]
+    gss = [gp.GpuScene(sd, lib, builder="device") for sd in sds]
+    srv = gp.Server(lib=lib)
+    ids = []
+    for sd, gs in zip(sds, gss):
+        depths.append(gs.info()["bvh_depth"])
+        ids.append(srv.submit(gs, sd.camera, 64, max_depth=3))
+        srv.step(max_iterations=2)
+    srv.step()
+    for sd, gs, j in zip(sds, gss, ids):
+        r, x, h = srv.take(j, 8, 8)
+        xa, ha, _, _ = gp.render_forward(gs, sd.camera, 64, max_depth=3)
+        same = same and r.status == 0 and bool(np.array_equal(x, xa) and np.array_equal(h, ha))
+    # steps of one scene whose stack needs 9..24 entries
+    waits = []
+    for k in (1, 5):
+        sd, gs = sds[k], gss[k]
+        j = srv.submit(gs, sd.camera, 64, max_depth=4)
+        srv.step(max_iterations=2)
+        before = emu.emu_stream_syncs()
+        srv.step(max_iterations=2)
+        waits.append(emu.emu_stream_syncs() - before)
+        srv.step()
+        srv.take(j, 8, 8)
+    srv.close()
+    return {"depths": depths, "same": same, "waits": waits}
+
+
+print(json.dumps({"capture": capture, "reshape": reshape}[sys.argv[1]]()))

@@ -31,6 +31,7 @@ def _run(scenario, lib, cus, preempt=0, run_async=0):
 # Each scenario is a child process of its own; all are started at once.
 CASES = {
     "capture": dict(cus=1),
+    "reshape": dict(cus=1, run_async=1),
 }
 
 
@@ -61,3 +62,13 @@ def test_film_calls_of_another_thread_stay_out_of_a_graph_capture(runs, orc):
     _, h, _, st = orc.render(orc.scene(sd), sd.camera, 5001, hero_c=4, max_bounce=4, threads=8)
     assert out["counts"] == [5001] + [st[k] for k in ("segments", "connections", "splats")]
     assert np.array_equal(np.array(out["hits"]), h)
+
+
+def test_a_server_waits_for_its_chunks_before_the_engine_changes_shape_and_only_then(runs):
+    # the emulator aborts where a graph is destroyed under a running chunk; a step that
+    # changes nothing synchronises no stream
+    out = _result(runs, "reshape")
+    need = [3 * ((d + 1) // 2) for d in out["depths"]]
+    assert need == sorted(need) and set(need) >= set(range(12, 37, 3))
+    assert out["same"]
+    assert out["waits"] == [0, 0]
