@@ -1163,8 +1163,10 @@ __global__ void __launch_bounds__(kFlightThreads, 4) k_flight(Queues q, unsigned
     __shared__ unsigned long long sKey[kFlightSlots];
     __shared__ unsigned long long sVal[kFlightSlots * 4];
     __shared__ unsigned long long sAcc[kAccRow];
+    __shared__ unsigned sLongest;   // segments of the longest path
     clearSplats<kFlightSlots>(sKey, sVal);
     if (threadIdx.x < kAccRow) sAcc[threadIdx.x] = 0ull;
+    if (threadIdx.x == 0) sLongest = 0u;
     __syncthreads();
     const DevJob& J = q.jobs[0];
     const unsigned gtid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1207,6 +1209,7 @@ __global__ void __launch_bounds__(kFlightThreads, 4) k_flight(Queues q, unsigned
                 d = nd;
                 ++bounce;
             }
+            if (!alive) atomicMax(&sLongest, (unsigned)bounce + (tri < 0 ? 1u : 0u));
         } else if (next < n && 4 * waiting >= live) {
             for (int k = 0; k < kMaxHero; ++k) { lam[k] = 0.f; beta[k] = 0.f; }
             photon = next;
@@ -1271,6 +1274,7 @@ __global__ void __launch_bounds__(kFlightThreads, 4) k_flight(Queues q, unsigned
     __syncthreads();
     if (threadIdx.x < kAccRow && sAcc[threadIdx.x])
         atomicAdd(J.acc + (size_t)(blockIdx.x % kSegs) * kAccRow + threadIdx.x, sAcc[threadIdx.x]);
+    if (threadIdx.x == 0) atomicMax(&q.ctrl->iter, sLongest);
     flushSplats<kFlightSlots>(q.jobs, sKey, sVal);
 }
 

@@ -716,8 +716,9 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
     hipStream_t s = device().stream;
     gp_status st;
     if ((st = enqueueEmit(sh, s)) != GP_OK) return st;
+    const int K = chunkIterations(tun);
     for (int i = 0; i < maxDepth;) {
-        const int stop = std::min(maxDepth, i + kOnceChunk);
+        const int stop = std::min(maxDepth, i + K);
         for (; i < stop; ++i) {
             q.resetCounts = i > 0 ? 1 : 0;
             st = enqueueBounce(sh, s);
@@ -752,8 +753,11 @@ gp_status Engine::fly(unsigned n, int maxDepth) {
     const unsigned most = std::min(kFlightWaves * cus, (unsigned)ls.extend);
     launchFlight(q, n, lanes, (int)std::min(most, (n + lanes - 1) / lanes), device().stream);
     GP_HIP(hipGetLastError());
-    onceIterations = maxDepth;
-    return readCtrl();
+    const gp_status st = readCtrl();
+    // as many as the wavefront would have run
+    const int K = chunkIterations(tun), longest = (int)hCtrl->iter;
+    onceIterations = std::min(maxDepth, (longest + K - 1) / K * K);
+    return st;
 }
 
 gp_status Engine::enqueueIterations(int n, hipStream_t s) {

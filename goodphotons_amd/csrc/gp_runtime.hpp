@@ -277,11 +277,10 @@ struct Engine {
     // Runs a trace whose n photons fit the path queue, from k_start_trace (once) to the
     // last path's end; reads the control block and slot 0's rows back. Every live path
     // advances one segment per iteration, so maxDepth iterations end it; the host looks
-    // for an earlier end every kOnceChunk. Grids are sized for n, and only the first
+    // for an earlier end every chunkIterations(). Grids are sized for n, and only the first
     // iteration schedules and emits: with five kernels an iteration on grids for the full
     // queue a 5000-photon render of the box spent 64 us an iteration on empty workgroups.
     gp_status traceOnce(unsigned n, int cams, int maxDepth);
-    static constexpr int kOnceChunk = 32;
     int onceIterations = 0;
     // Whether a trace of n photons runs as one k_flight launch, and that run. Mirror planes,
     // traversal statistics, kernel timing and ray binning belong to the wavefront's kernels.

@@ -203,7 +203,8 @@ typedef struct gp_trace_stats {
                                 light-side any hit and eye-side closest hit of each
                                 connection through a flat mirror                     */
     uint64_t splats;         /* connections that reached the film                    */
-    uint64_t iterations;     /* wavefront iterations run                             */
+    uint64_t iterations;     /* wavefront iterations run (a small trace that flies in one
+                                kernel: those that the wavefront would have run)     */
     double wall_ms;          /* host wall time of the trace loop                     */
     /* With gp_tuning.profile = 1: summed device time and launch count per kernel,
      * index 0 schedule, 1 emit, 2 extend (closest hit), 3 shade, 4 connect (and the
@@ -412,8 +413,7 @@ typedef struct gp_tuning {
                                 captured hipGraph: even, 2..64; 1..64 without graphs) */
     int32_t use_graph;       /* 1 = replay captured graphs, 0 = plain launches (a trace
                                 that fits the path queue always runs plain launches
-                                on grids of its own size, read back every 32
-                                iterations)                                          */
+                                on grids of its own size)                            */
     int32_t lds_stack;       /* traversal stack entries per lane held in LDS: 8, 12,
                                 16, 24 or 32 (default 12; deeper entries spill to
                                 global memory)                                       */

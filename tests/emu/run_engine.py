@@ -113,4 +113,27 @@ def reshape():
     return {"depths": depths, "same": same, "waits": waits}
 
 
-print(json.dumps({"capture": capture, "reshape": reshape}[sys.argv[1]]()))
+def deep():
+    """Paths that end long before the depth limit: iterations of a trace on the wavefront
+    (mirrors) and of one that flies, and what is still alive an iteration chunk earlier."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=4)
+    out = {}
+    for name, sd in (("mirror", scenes.mirror_box(8)), ("box", scenes.cornell_c0(8))):
+        gs = gp.GpuScene(sd, lib)
+
+        def run(depth):
+            f = film_of(sd, 64)
+            e, st = gp.trace(gs, sd.camera, f, 64, max_depth=depth)
+            return [int(st.iterations), float(e.residual), counts(st)]
+
+        flown = emu.emu_launches(b"k_flight")
+        whole = run(60)
+        out[name] = {"whole": whole, "before": run(whole[0] - 4) if whole[0] > 4 else None,
+                     "flown": emu.emu_launches(b"k_flight") - flown}
+        lib.set_tuning(profile=1)
+        out[name]["wavefront"] = run(60)
+        lib.set_tuning(profile=0)
+    return out
+
+
+print(json.dumps({"capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
