@@ -667,6 +667,13 @@ void gp_film_destroy(gp_film* f) { delete f; }
 // ------------------------------------------------------------------ trace
 gp_status gp_trace_shared(gp_scene* s, int32_t n_cams, const gp_camera_desc* cams, gp_film* const* films,
                           const gp_trace_params* p, gp_energy* energy, gp_trace_stats* stats) {
+    return traceShared(s, n_cams, cams, films, p, energy, stats, true);
+}
+
+}  // extern "C"
+
+gp_status gp::traceShared(gp_scene* s, int n_cams, const gp_camera_desc* cams, gp_film* const* films,
+                          const gp_trace_params* p, gp_energy* energy, gp_trace_stats* stats, bool mayFly) {
     if (!s || !cams || !films || !p) return fail(GP_ERR_INVALID, "null argument");
     if (n_cams < 1 || n_cams > kMaxCams) return fail(GP_ERR_INVALID, "n_cams must be 1..16");
     if (p->n_photons < 0) return fail(GP_ERR_INVALID, "negative photon count");
@@ -716,7 +723,7 @@ gp_status gp_trace_shared(gp_scene* s, int32_t n_cams, const gp_camera_desc* cam
         ts.capacity = E.capacity;
         ts.nCams = n_cams;
         ts.once = once ? 1 : 0;
-        const bool flies = E.flies((uint64_t)n, n_cams);
+        const bool flies = mayFly && E.flies((uint64_t)n, n_cams);
         launchStartTrace(E.q, ts, strm);
         GP_HIP(hipGetLastError());
         E.parity = 0;
@@ -766,6 +773,8 @@ gp_status gp_trace_shared(gp_scene* s, int32_t n_cams, const gp_camera_desc* cam
     if (stats) *stats = acc;
     return GP_OK;
 }
+
+extern "C" {
 
 gp_status gp_trace(gp_scene* s, const gp_camera_desc* cam, gp_film* film, const gp_trace_params* p,
                    gp_energy* energy, gp_trace_stats* stats) {

@@ -318,6 +318,9 @@ void addCounters(const unsigned long long* counters, gp_trace_stats& st);
 // records (to be placed at J.cams) are written to camsOut.
 gp_status fillJob(const gp_scene* s, const gp_camera_desc* cams, gp_film* const* films, int nCams,
                   const gp_trace_params& p, int slot, DevJob& J, DevCamera* camsOut);
+// gp_trace_shared; without mayFly a small trace runs the wavefront's kernels too.
+gp_status traceShared(gp_scene* s, int nCams, const gp_camera_desc* cams, gp_film* const* films,
+                      const gp_trace_params* p, gp_energy* energy, gp_trace_stats* stats, bool mayFly);
 gp_status prepareFilm(gp_film* film, const gp_scene* s, const CamBasis& cb,
                       const gp_trace_params& p);
 

@@ -581,8 +581,11 @@ gp_status gp_autotune(gp_scene* scene, const gp_camera_desc* cam, const gp_trace
         if ((s0 = gp_film_create(cam->res_x, cam->res_y, 2 * p.n_photons, &film)) != GP_OK) return s0;
         gp_energy e{};
         gp_trace_stats s{};
-        s0 = gp_trace(scene, cam, film, &p, &e, &s);        // warm (allocations, graph)
-        if (s0 == GP_OK) s0 = gp_trace(scene, cam, film, &p, &e, &s);
+        // a small budget would fly, and the settings are the wavefront's: on a flight they
+        // would be picked by noise, for every later trace
+        auto run = [&] { return traceShared(scene, 1, cam, &film, &p, &e, &s, false); };
+        s0 = run();                                          // warm (allocations, graph)
+        if (s0 == GP_OK) s0 = run();
         gp_film_destroy(film);
         if (s0 != GP_OK) return s0;
         const double rate = (double)s.segments / std::max(1e-6, s.wall_ms);

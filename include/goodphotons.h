@@ -417,7 +417,9 @@ typedef struct gp_tuning {
     int32_t lds_stack;       /* traversal stack entries per lane held in LDS: 8, 12,
                                 16, 24 or 32 (default 12; deeper entries spill to
                                 global memory)                                       */
-    int32_t profile;         /* 1 = time every kernel launch with HIP events (no graphs) */
+    int32_t profile;         /* 1 = time every kernel launch with HIP events (no graphs, and
+                                small traces run the wavefront's kernels instead of
+                                flying in one)                                       */
     int32_t ray_sort;        /* 1 = reorder each iteration's paths by origin cell
                                 (8 x 8 x 8 over the scene) and direction octant before
                                 the closest-hit kernel, a counting sort into a third
@@ -431,7 +433,8 @@ typedef struct gp_tuning {
 gp_status gp_get_tuning(gp_tuning* out);
 gp_status gp_set_tuning(const gp_tuning* in);
 /* Times candidate settings on `scene`/`cam` with a short trace and installs
- * the fastest. On failure the tuning in place before the call is restored. */
+ * the fastest. They are the wavefront's settings, so its kernels are timed also where a
+ * trace of so few photons would fly in one kernel. On failure the tuning in place before the call is restored. */
 gp_status gp_autotune(gp_scene* scene, const gp_camera_desc* cam,
                       const gp_trace_params* params, gp_tuning* best_out);
 

@@ -136,4 +136,20 @@ def deep():
     return out
 
 
-print(json.dumps({"capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def autotune():
+    """Kernels that gp_autotune times with a budget small enough to fly, and a trace of it."""
+    sd = scenes.cornell_c0(8)
+    gs = gp.GpuScene(sd, lib)
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4)
+    best = gp.abi.Tuning()
+    p = gp.trace_params(32, max_depth=1)
+    lib.check(emu.gp_autotune(gs.h, C.byref(sd.camera), C.byref(p), C.byref(best)))
+    out = {"flown": emu.emu_launches(b"k_flight"), "extended": emu.emu_launches(b"k_extend"),
+           "installed": lib.tuning().queue_capacity == best.queue_capacity}
+    lib.set_tuning(queue_capacity=4096)
+    gp.trace(gs, sd.camera, film_of(sd, 32), 32, max_depth=1)
+    out["trace_flown"] = emu.emu_launches(b"k_flight") - out["flown"]
+    return out
+
+
+print(json.dumps({"autotune": autotune, "capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

@@ -30,6 +30,7 @@ def _run(scenario, lib, cus, preempt=0, run_async=0):
 
 # Each scenario is a child process of its own; all are started at once.
 CASES = {
+    "autotune": dict(cus=1),
     "capture": dict(cus=1),
     "reshape": dict(cus=1, run_async=1),
     "deep": dict(cus=1),
@@ -90,3 +91,10 @@ def test_a_deep_trace_ends_with_the_chunk_that_ends_its_last_path(runs, name):
     assert 4 < iters < 60 and iters % 4 == 0 and residual == 0
     assert out["before"][1] > 0
     assert out["wavefront"] == out["whole"]
+
+
+def test_autotune_times_the_wavefronts_kernels_with_a_small_budget(runs):
+    # 18 shapes and the sorting modes, each warmed and timed
+    out = _result(runs, "autotune")
+    assert out["flown"] == 0 and out["extended"] >= 2 * 19 and out["installed"]
+    assert out["trace_flown"] == 1
