@@ -1126,6 +1126,15 @@ __global__ void __launch_bounds__(kTravThreads, 6) k_connect(Queues q) {
 // both: lanes of a wave may be in different traversals).
 constexpr int kFlightSlots = 64;
 
+// Keeps the LDS accesses of a wave's lanes on either side apart. The hardware runs them in
+// program order; the fence keeps the compiler to it also where the two sides use one array
+// under different types (stack entries, staged words), which it may otherwise take for
+// different memory. No instruction of its own.
+__device__ __forceinline__ void waveFence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Adds the splats of the lanes with `pending` to their films, four lanes per splat. The
 // records are staged in the stack array `stk` (no traversal is running: the whole wave is
 // here).
@@ -1133,6 +1142,7 @@ __device__ __forceinline__ void splatDirect(int2* stk, bool pending, unsigned lo
                                             unsigned long long Y, unsigned long long Z, unsigned long long H) {
     const unsigned long long mask = __ballot(pending);
     if (mask == 0ull) return;
+    waveFence();
     const unsigned lane = threadIdx.x;
     unsigned long long* col = (unsigned long long*)stk;
     const unsigned rank = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
@@ -1144,7 +1154,7 @@ __device__ __forceinline__ void splatDirect(int2* stk, bool pending, unsigned lo
         col[3 * kFlightThreads + rank] = H;
         col[4 * kFlightThreads + rank] = (unsigned long long)at;
     }
-    __builtin_amdgcn_wave_barrier();
+    waveFence();
     const unsigned count = (unsigned)__popcll(mask);
     for (unsigned b = 0; b < count; b += 16) {
         const unsigned r = b + (lane >> 2);
@@ -1153,7 +1163,7 @@ __device__ __forceinline__ void splatDirect(int2* stk, bool pending, unsigned lo
             if (v) atomicAdd((unsigned long long*)col[4 * kFlightThreads + r] + (lane & 3u), v);
         }
     }
-    __builtin_amdgcn_wave_barrier();
+    waveFence();
 }
 
 template <int SD, bool SPILL>

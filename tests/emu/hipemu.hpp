@@ -72,6 +72,7 @@ __attribute__((noinline)) inline void __syncthreads() { emu_sync(__builtin_retur
 // builtin only fences code motion): emulated as a wave collective.
 __attribute__((noinline)) inline void emu_wave_barrier() { (void)emu_ballot(1, __builtin_return_address(0)); }
 #define __builtin_amdgcn_wave_barrier() emu_wave_barrier()
+#define __builtin_amdgcn_fence(order, scope) ((void)0)   // lanes run one at a time
 __attribute__((noinline)) inline int __syncthreads_or(int p) { return emu_sync_or(p, __builtin_return_address(0)); }
 inline unsigned __lane_id() { return emu_lane(); }
 inline unsigned emu_mbcnt_lo(unsigned m, unsigned acc) {
