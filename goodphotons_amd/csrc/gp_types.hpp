@@ -64,14 +64,31 @@ constexpr int kBinCellsPerAxis = 8;
 // surface points they reach, with everything that starts there, stay close together.
 // Whole renders, index order -> sorted: 5.24M-triangle icosphere (2^28 photons, 1024^2)
 // 219.0 -> 204.0 ms, closest-hit kernel 147 -> 131; glass sphere and prism (2^26, 512^2)
-// 66.9 -> 62.7 ms; the box (2^22) 4.73 -> 4.64 ms. The four sorting kernels take about
-// 35 us an iteration, also one that emits nothing (8 us then), so traces of fewer than
-// kEmitOrderJobMin photons keep index order (2^20 photons: the glass scene 2.06 -> 2.12
-// ms, the box 1.33 -> 1.35), as do refills of fewer than kEmitOrderMin (a few photons to
-// each of the 4096 keys).
-constexpr int kEmitCols = 256;
-constexpr unsigned kEmitOrderMin = 1u << 16;
-constexpr uint64_t kEmitOrderJobMin = 1u << 19;
+// 66.9 -> 62.7 ms; the box (2^22) 4.73 -> 4.64 ms.
+// The four sorting kernels take about 35 us in an iteration that emits and 8 us in one that
+// does not, so the rule is on the photons of a trace (one refill: sorted once) or of a
+// server's largest job (every iteration). Index order -> sorted, ms:
+//   photons                   2^18           2^19           2^20           2^21
+//   trace: box                               1.00 -> 1.01   1.32 -> 1.29   1.97 -> 1.90
+//          glass, prism                      2.71 -> 2.44   2.87 -> 2.77   3.89 -> 3.57
+//          soup 100K tri.                    5.00 -> 4.91   5.83 -> 5.75   7.45 -> 7.19
+//          icosphere 1.3M                    3.04 -> 3.07   3.45 -> 3.37   4.11 -> 3.89
+//   4 jobs: box                              2.77 -> 2.81   4.11 -> 4.07   6.67 -> 6.57
+//          glass, prism                      4.91 -> 4.87   6.81 -> 6.46   10.6 -> 9.8
+//   16 jobs: box              14.4 -> 14.4   16.8 -> 16.6   22.6 -> 21.8   34.0 -> 32.3
+//          glass, prism       16.9 -> 16.7   21.0 -> 20.2   29.3 -> 27.2   45.7 -> 41.6
+// (the soup's and the icosphere's jobs gain 1-4% at 2^19 and 4-9% at 2^21). So from 2^19 on
+// it gains or, on the box, costs 1%; fewer photons fly where they are a trace. Refills of
+// fewer than kEmitOrderMin (a few photons to each of the 4096 keys) keep index order.
+// The macros let a CPU test sort a few thousand photons.
+#ifndef GP_EMIT_COLS
+#define GP_EMIT_COLS 256
+#define GP_EMIT_ORDER_MIN (1u << 16)
+#define GP_EMIT_ORDER_JOB_MIN (1u << 19)
+#endif
+constexpr int kEmitCols = GP_EMIT_COLS;
+constexpr unsigned kEmitOrderMin = GP_EMIT_ORDER_MIN;
+constexpr uint64_t kEmitOrderJobMin = GP_EMIT_ORDER_JOB_MIN;
 
 // A trace that the chip holds at once flies (k_flight) instead of running the wavefront.
 // kFlightWaves: resident waves of k_flight per CU. Per-trace times, wavefront -> flight, on
