@@ -31,13 +31,16 @@ def available() -> bool:
     return os.path.exists(CXX) and os.path.exists(asan_runtime())
 
 
-def build() -> str:
-    os.makedirs(OUT, exist_ok=True)
+def build(variant: str = "", defines: tuple = ()) -> str:
+    """Builds the library, or a variant of it with the given macros, and returns its path."""
+    out = os.path.join(OUT, variant)
+    lib = os.path.join(out, os.path.basename(LIB))
+    os.makedirs(out, exist_ok=True)
     flags = ["-std=c++20", "-O2", "-g", "-fPIC", "-fno-omit-frame-pointer", "-fsanitize=address",
              "-I", os.path.join(HERE, "fakehip"), "-I", HERE, "-I", os.path.join(ROOT, "include"),
-             "-I", CSRC, "-Wno-unused-result", "-Wno-ignored-attributes"]
-    jobs = [(os.path.join(CSRC, s), os.path.join(OUT, os.path.splitext(s)[0] + ".o"), True) for s in SOURCES]
-    jobs += [(os.path.join(HERE, "hipemu.cpp"), os.path.join(OUT, "hipemu.o"), False)]
+             "-I", CSRC, "-Wno-unused-result", "-Wno-ignored-attributes", *(f"-D{d}" for d in defines)]
+    jobs = [(os.path.join(CSRC, s), os.path.join(out, os.path.splitext(s)[0] + ".o"), True) for s in SOURCES]
+    jobs += [(os.path.join(HERE, "hipemu.cpp"), os.path.join(out, "hipemu.o"), False)]
 
     def one(job):
         src, obj, as_cxx = job
@@ -49,10 +52,10 @@ def build() -> str:
 
     with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 4)) as ex:
         objs = list(ex.map(one, jobs))
-    tmp = LIB + ".tmp"
+    tmp = lib + ".tmp"
     subprocess.run([CXX, "-shared", "-fsanitize=address", "-o", tmp, *objs, "-lpthread"], check=True)
-    os.replace(tmp, LIB)
-    return LIB
+    os.replace(tmp, lib)
+    return lib
 
 
 if __name__ == "__main__":

@@ -152,4 +152,64 @@ def autotune():
     return out
 
 
-print(json.dumps({"autotune": autotune, "capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def views(sd, count):
+    c = sd.camera
+    return [c] + [scenes.camera((c.eye[0] + 0.02 * k, c.eye[1], c.eye[2]), tuple(c.target), tuple(c.up),
+                                c.fov_y_deg, 9 + k, 11) for k in range(1, count)]
+
+
+def flight():
+    """Traces that fly, with the stack in LDS and spilling, one camera and three, against
+    the wavefront's kernels (kernel timing on) for the same photons."""
+    out = {}
+    for name, sd, n, cams, lds in (("c1_8", scenes.caustics_c1(32), 1500, 1, 8),
+                                   ("c1_12", scenes.caustics_c1(32), 1500, 1, 12),
+                                   ("c0_cams", scenes.cornell_c0(32), 900, 3, 12)):
+        gs, cs, got = gp.GpuScene(sd, lib), views(sd, cams), []
+        for profile in (0, 1):
+            lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, lds_stack=lds, profile=profile)
+            films = [gp.Film(c.res_x, c.res_y, max_photons=n, lib=lib) for c in cs]
+            before = emu.emu_launches(b"k_flight")
+            e, st = gp.trace_shared(gs, cs, films, n, max_depth=8)
+            got.append([[f.raw()[0].tolist() for f in films], e.as_dict(), counts(st)])
+            out.setdefault(name, {}).setdefault("flown", []).append(emu.emu_launches(b"k_flight") - before)
+        out[name].update(same=got[0] == got[1], counts=got[0][2], hits=[w[3] for w in got[0][0][0]])
+    return out
+
+
+def sort():
+    """Sorted emission (a build with low thresholds) of a trace with two lights, and of two
+    jobs on a server, against traces of the same photons that fly."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
+    sd = scenes.cornell_c0(16)
+    sd.emitters.append(scenes.quad_emitter((0.3, 0.9, 0.3), (0.2, 0, 0), (0, 0, 0.2), (0, -1, 0),
+                                           sd.emitters[0].spd, collimated=True, beam=(0, -1, 0)))
+    gs = gp.GpuScene(sd, lib)
+    n = 2003
+    whole, parts = film_of(sd, n), film_of(sd, n)
+    _, st = gp.trace(gs, sd.camera, whole, n, max_depth=4)
+    sorts = emu.emu_launches(b"k_emit_perm")
+    sums = np.zeros(len(KEYS), np.int64)
+    for at in range(0, n, 700):
+        _, sp = gp.trace(gs, sd.camera, parts, min(700, n - at), seed_base=at, max_depth=4)
+        sums += counts(sp)
+    out = {"sorts": sorts, "more_sorts": emu.emu_launches(b"k_emit_perm") - sorts, "counts": counts(st),
+           "trace": bool(np.array_equal(whole.raw()[0], parts.raw()[0]) and counts(st) == sums.tolist())}
+    srv = gp.Server(lib=lib)
+    jobs = [(gs, sd, 1203, 7), (gs, sd, 350, 9000)]
+    ids = [srv.submit(g, d.camera, k, seed_base=s, max_depth=2) for g, d, k, s in jobs]
+    srv.step()
+    same = True
+    for j, (g, d, k, s) in zip(ids, jobs):
+        r, x, h = srv.take(j, 16, 16)
+        f = film_of(d, k)
+        for at in range(0, k, 700):
+            gp.trace(g, d.camera, f, min(700, k - at), seed_base=s + at, max_depth=2)
+        hs = f.download_hits()
+        same = same and r.status == 0 and bool(np.array_equal(h, hs))
+    srv.close()
+    out["server"] = same
+    return out
+
+
+print(json.dumps({"flight": flight, "sort": sort, "autotune": autotune, "capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

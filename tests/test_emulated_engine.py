@@ -20,10 +20,10 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 pytestmark = pytest.mark.skipif(not emu.available(), reason="clang++ with AddressSanitizer not found")
 
 
-def _run(scenario, lib, cus, preempt=0, run_async=0):
+def _run(scenario, libs, cus, preempt=0, run_async=0, variant=""):
     env = dict(os.environ)
     env.update({"LD_PRELOAD": emu.asan_runtime(), "ASAN_OPTIONS": "detect_leaks=0", "EMU_CUS": str(cus),
-                "EMU_PREEMPT": str(preempt), "EMU_ASYNC": str(run_async), "EMU_LIB": lib})
+                "EMU_PREEMPT": str(preempt), "EMU_ASYNC": str(run_async), "EMU_LIB": libs[variant]})
     return subprocess.Popen([sys.executable, os.path.join(ROOT, "tests", "emu", "run_engine.py"), scenario],
                             stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, env=env)
 
@@ -34,13 +34,17 @@ CASES = {
     "capture": dict(cus=1),
     "reshape": dict(cus=1, run_async=1),
     "deep": dict(cus=1),
+    "flight": dict(cus=2, preempt=3),
+    "sort": dict(cus=1, variant="sort"),
 }
+# emission sorted from 64 photons on, in traces of 1000
+VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000")}
 
 
 @pytest.fixture(scope="module")
 def runs():
-    lib = emu.build()
-    procs = {k: _run(k, lib, **kw) for k, kw in CASES.items()}
+    libs = {v: emu.build(v, d) for v, d in VARIANTS.items()}
+    procs = {k: _run(k, libs, **kw) for k, kw in CASES.items()}
     yield procs
     for p in procs.values():
         if p.poll() is None:
@@ -98,3 +102,25 @@ def test_autotune_times_the_wavefronts_kernels_with_a_small_budget(runs):
     out = _result(runs, "autotune")
     assert out["flown"] == 0 and out["extended"] >= 2 * 19 and out["installed"]
     assert out["trace_flown"] == 1
+
+
+@pytest.mark.parametrize("name", ["c1_8", "c1_12", "c0_cams"])
+def test_flight_with_interleaved_lanes(runs, orc, name):
+    # every access of k_flight checked: the wavefront's words, ledger and counters, and the
+    # oracle's photons
+    out = _result(runs, "flight")[name]
+    assert out["flown"] == [1, 0] and out["same"]
+    sd = scenes.cornell_c0(32) if name == "c0_cams" else scenes.caustics_c1(32)
+    n = out["counts"][0]
+    _, h, _, st = orc.render(orc.scene(sd), sd.camera, n, hero_c=4, max_bounce=8, threads=8)
+    assert out["counts"][1] == st["segments"] and np.array_equal(np.array(out["hits"]), h)
+    if name != "c0_cams":
+        assert out["counts"][2:] == [st["connections"], st["splats"]]
+
+
+def test_sorted_emission(runs, orc):
+    # k_emit_keys, k_emit_perm and the ordered k_emit with every access checked: one sort of
+    # the trace's 2003 photons of two lights, then a server with two jobs in the order
+    out = _result(runs, "sort")
+    assert out["sorts"] == 1 and out["more_sorts"] == 0
+    assert out["trace"] and out["server"]
