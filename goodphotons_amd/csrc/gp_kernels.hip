@@ -1519,8 +1519,7 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_count(Queues q, int cur) {
     unsigned lo, hi;
     binRange(n, col, (unsigned)q.binCols, lo, hi);
     const unsigned short* __restrict__ keys = q.key[cur];
-    // keys are masked: paths queued before binning was switched on carry no key (both
-    // passes read the same words, so any value still gives a permutation)
+    // the mask bounds the LDS index (keys have 12 bits; both passes read the same words)
     for (unsigned li = lo + threadIdx.x; li < hi; li += blockDim.x) atomicAdd(&h[keys[sm.slot(li)] & (kBins - 1)], 1u);
     __syncthreads();
     unsigned* out = q.binHist + (size_t)col * kBins;
