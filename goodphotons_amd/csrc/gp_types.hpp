@@ -92,18 +92,25 @@ constexpr uint64_t kEmitOrderJobMin = GP_EMIT_ORDER_JOB_MIN;
 
 // A trace that the chip holds at once flies (k_flight) instead of running the wavefront.
 // kFlightWaves: resident waves of k_flight per CU. Per-trace times, wavefront -> flight, on
-// 256 CUs (262144 resident lanes):
-//   photons         4096          65536         262144        370816        524445
-//   box             552 -> 286    594 -> 365    729 -> 568    813 -> 787    929 -> 924 us
-//   glass, prism    1281 -> 427   1651 -> 684   1887 -> 938   1990 -> 1236  2118 -> 1486
-//   soup 100K tri.  2248 -> 646   3695 -> 1236  4187 -> 1508  4349 -> 2267  4502 -> 2622
-//   icosphere 1.3M  1651 -> 454   2672 -> 809   3195 -> 961   3298 -> 1366  3591 -> 1568
-// and 0.55-1.5x at 2^20: past about one and a half photons per lane a box loses. Six
-// cameras: 2068 -> 1745 us at 65536 photons, 2235 -> 2019 at 131080, 2332 -> 2480 at
-// 185386, so a camera more counts as a third of a photon.
-constexpr int kFlightWaves = 16;
+// 256 CUs (262144 resident lanes), us:
+//   photons         4096          65536         262144        393216        524445
+//   box             501 -> 231    550 -> 327    668 -> 461    768 -> 765    869 -> 903
+//   glass, prism    1288 -> 372   1644 -> 646   1856 -> 892   1962 -> 1262  2078 -> 1497
+//   soup 100K tri.  2509 -> 525   3659 -> 1103  4133 -> 1507  4245 -> 2251  4412 -> 2634
+//   icosphere 1.3M  2181 -> 515   3366 -> 907   3905 -> 1252  4070 -> 1838  4277 -> 1929
+// so a box loses past one and a half photons per lane. A lane traces its vertex to one camera
+// after the other, while the wavefront's k_connect gets them all at once: the limit falls with
+// cameras^1.5, and past six nothing flies (box, 8 segments deep):
+//   cameras, photons    3, 65536    4, 30000    6, 4096     6, 12000    6, 30000    16, 4096
+//                       618 -> 542  618 -> 550  601 -> 547  636 -> 617  669 -> 775  843 -> 1307
+// Over 1 to 6 cameras, 1 to 16 segments, 1000 to 393216 photons and six scenes no trace that
+// flies takes longer than the wavefront did when each camera's connections were appended by
+// an atomic of their own (0.98 at most); some of one to three segments take up to 1.36 times
+// what today's takes.
+constexpr int kFlightWaves = 16, kFlightCams = 6;
 inline bool flightFits(uint64_t photons, int cams, int cus) {
-    return 2 * photons * (uint64_t)(2 + cams) <= 9 * (uint64_t)cus * kFlightWaves * 64;
+    const uint64_t c = (uint64_t)cams, most = 3 * (uint64_t)cus * kFlightWaves * 64;   // twice 1.5 a lane
+    return cams <= kFlightCams && photons <= most && 4 * photons * photons * c * c * c <= most * most;
 }
 
 // Leaf links are negative: ~((first << 3) | (count - 1)).

@@ -164,7 +164,7 @@ def flight():
     out = {}
     for name, sd, n, cams, lds in (("c1_8", scenes.caustics_c1(32), 1500, 1, 8),
                                    ("c1_12", scenes.caustics_c1(32), 1500, 1, 12),
-                                   ("c0_cams", scenes.cornell_c0(32), 900, 3, 12)):
+                                   ("c0_cams", scenes.cornell_c0(32), 590, 3, 12)):
         gs, cs, got = gp.GpuScene(sd, lib), views(sd, cams), []
         for profile in (0, 1):
             lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, lds_stack=lds, profile=profile)
@@ -212,4 +212,18 @@ def sort():
     return out
 
 
-print(json.dumps({"flight": flight, "sort": sort, "autotune": autotune, "capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def route():
+    """Which traces fly, by cameras and photons (1024 resident lanes)."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4)
+    sd = scenes.cornell_c0(8)
+    gs, out = gp.GpuScene(sd, lib), []
+    for cams, n in ((1, 1536), (1, 1537), (2, 543), (2, 544), (6, 104), (6, 105), (7, 40), (16, 40)):
+        cs = views(sd, cams)
+        films = [gp.Film(c.res_x, c.res_y, max_photons=n, lib=lib) for c in cs]
+        before = emu.emu_launches(b"k_flight")
+        gp.trace_shared(gs, cs, films, n, max_depth=1)
+        out.append([cams, n, emu.emu_launches(b"k_flight") - before])
+    return out
+
+
+print(json.dumps({"route": route, "flight": flight, "sort": sort, "autotune": autotune, "capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

@@ -36,6 +36,7 @@ CASES = {
     "deep": dict(cus=1),
     "flight": dict(cus=2, preempt=3),
     "sort": dict(cus=1, variant="sort"),
+    "route": dict(cus=1),
 }
 # emission sorted from 64 photons on, in traces of 1000
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000")}
@@ -124,3 +125,9 @@ def test_sorted_emission(runs, orc):
     out = _result(runs, "sort")
     assert out["sorts"] == 1 and out["more_sorts"] == 0
     assert out["trace"] and out["server"]
+
+
+def test_traces_of_many_cameras_do_not_fly(runs):
+    # 1024 resident lanes: up to 1.5 photons a lane, less by cameras^1.5, and six cameras
+    for cams, n, flown in _result(runs, "route"):
+        assert flown == (1 if cams <= 6 and n * cams ** 1.5 <= 1536 else 0), (cams, n)
