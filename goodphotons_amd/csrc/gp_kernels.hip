@@ -24,6 +24,8 @@
 // (:499-577) and refractOrReflect (:2657-2694), in float32.
 #include <hip/hip_runtime.h>
 
+#include <tuple>
+
 #include "gp_device.hpp"
 #include "gp_kernels.hpp"
 
@@ -1791,15 +1793,40 @@ __global__ void k_fill64(unsigned long long* p, size_t n, unsigned long long v) 
 }
 
 // ------------------------------------------------------------------ launchers
-void launchSchedule(const Queues& q, int cur, hipStream_t s) {
-    hipLaunchKernelGGL(k_schedule, dim3(1), dim3(kMaxJobs), 0, s, q, cur);
+// Launches on the sink's stream, or appends the kernel to its graph. The arguments are
+// copied either way.
+template <class... P, class... A>
+static void enqueue(Sink& k, void (*kernel)(P...), dim3 grid, dim3 block, const A&... a) {
+    if (!k.graph) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, k.stream, a...);
+        return;
+    }
+    std::tuple<P...> args(a...);
+    hipKernelNodeParams n{};
+    n.func = (decltype(n.func))kernel;
+    n.gridDim = grid;
+    n.blockDim = block;
+    hipGraphNode_t node = nullptr;
+    const hipError_t e = std::apply(
+        [&](P&... x) {
+            void* at[] = {(void*)&x...};
+            n.kernelParams = at;
+            return hipGraphAddKernelNode(&node, k.graph, k.last ? &k.last : nullptr, k.last ? 1 : 0, &n);
+        },
+        args);
+    if (e != hipSuccess) k.error = e;
+    k.last = node;
 }
-void launchEmit(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s) {
-    hipLaunchKernelGGL(k_emit, dim3(ls.emit), dim3(256), 0, s, q, cur);
+
+void launchSchedule(const Queues& q, int cur, Sink& k) {
+    enqueue(k, k_schedule, dim3(1), dim3(kMaxJobs), q, cur);
 }
-void launchShade(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s) {
-    if (q.binned) hipLaunchKernelGGL(k_shade<true>, dim3(ls.shade), dim3(kShadeThreads), 0, s, q, cur);
-    else hipLaunchKernelGGL(k_shade<false>, dim3(ls.shade), dim3(kShadeThreads), 0, s, q, cur);
+void launchEmit(const Queues& q, int cur, const LaunchShape& ls, Sink& k) {
+    enqueue(k, k_emit, dim3(ls.emit), dim3(256), q, cur);
+}
+void launchShade(const Queues& q, int cur, const LaunchShape& ls, Sink& k) {
+    if (q.binned) enqueue(k, k_shade<true>, dim3(ls.shade), dim3(kShadeThreads), q, cur);
+    else enqueue(k, k_shade<false>, dim3(ls.shade), dim3(kShadeThreads), q, cur);
 }
 // Kernel instances by LDS stack depth and spill use.
 #define GP_BY_STACK(LDS, SPILL, CALL) \
@@ -1834,12 +1861,12 @@ void launchShade(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s)
         }                                  \
     } while (0)
 
-void launchExtend(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s) {
+void launchExtend(const Queues& q, int cur, const LaunchShape& ls, Sink& k) {
     const dim3 grid(ls.extend);
-#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, false, false>), grid, dim3(kExtendThreads), 0, s, q, cur)
-#define GP_CALLS(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, true, false>), grid, dim3(kExtendThreads), 0, s, q, cur)
-#define GP_CALLB(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, false, true>), grid, dim3(kExtendThreads), 0, s, q, cur)
-#define GP_CALLSB(SD, SP) hipLaunchKernelGGL((k_extend<SD, SP, true, true>), grid, dim3(kExtendThreads), 0, s, q, cur)
+#define GP_CALL(SD, SP) enqueue(k, k_extend<SD, SP, false, false>, grid, dim3(kExtendThreads), q, cur)
+#define GP_CALLS(SD, SP) enqueue(k, k_extend<SD, SP, true, false>, grid, dim3(kExtendThreads), q, cur)
+#define GP_CALLB(SD, SP) enqueue(k, k_extend<SD, SP, false, true>, grid, dim3(kExtendThreads), q, cur)
+#define GP_CALLSB(SD, SP) enqueue(k, k_extend<SD, SP, true, true>, grid, dim3(kExtendThreads), q, cur)
     if (q.binned) {
         if (q.stats) GP_BY_STACK_EXT(q.lds, q.useSpill, GP_CALLSB);
         else GP_BY_STACK_EXT(q.lds, q.useSpill, GP_CALLB);
@@ -1852,24 +1879,24 @@ void launchExtend(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s
 #undef GP_CALLS
 #undef GP_CALL
 }
-void launchEmitOrder(const Queues& q, hipStream_t s) {
+void launchEmitOrder(const Queues& q, Sink& k) {
     static_assert(kEmitCols % kBinChunks == 0, "emission columns split into the scan's chunks");
     const BinTables bt{q.emitHist, q.emitChunk, q.emitTotal, kEmitCols};
-    hipLaunchKernelGGL(k_emit_keys, dim3(kEmitCols), dim3(kBinThreads), 0, s, q);
-    hipLaunchKernelGGL(k_bin_chunks, dim3(kBins / 32), dim3(kBinChunks * 32), 0, s, bt);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kBinScanThreads), 0, s, bt);
-    hipLaunchKernelGGL(k_emit_perm, dim3(kEmitCols), dim3(kBinThreads), 0, s, q);
+    enqueue(k, k_emit_keys, dim3(kEmitCols), dim3(kBinThreads), q);
+    enqueue(k, k_bin_chunks, dim3(kBins / 32), dim3(kBinChunks * 32), bt);
+    enqueue(k, k_bin_scan, dim3(1), dim3(kBinScanThreads), bt);
+    enqueue(k, k_emit_perm, dim3(kEmitCols), dim3(kBinThreads), q);
 }
-void launchBin(const Queues& q, int cur, hipStream_t s) {
-    hipLaunchKernelGGL(k_bin_count, dim3(q.binCols), dim3(kBinThreads), 0, s, q, cur);
+void launchBin(const Queues& q, int cur, Sink& k) {
+    enqueue(k, k_bin_count, dim3(q.binCols), dim3(kBinThreads), q, cur);
     const BinTables bt{q.binHist, q.binChunk, q.binTotal, q.binCols};
-    hipLaunchKernelGGL(k_bin_chunks, dim3(std::min(kBins / 32, q.binCols)), dim3(kBinChunks * 32), 0, s, bt);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(kBinScanThreads), 0, s, bt);
-    hipLaunchKernelGGL(k_bin_scatter, dim3(q.binCols), dim3(kBinThreads), 0, s, q, cur);
+    enqueue(k, k_bin_chunks, dim3(std::min(kBins / 32, q.binCols)), dim3(kBinChunks * 32), bt);
+    enqueue(k, k_bin_scan, dim3(1), dim3(kBinScanThreads), bt);
+    enqueue(k, k_bin_scatter, dim3(q.binCols), dim3(kBinThreads), q, cur);
 }
-void launchConnect(const Queues& q, const LaunchShape& ls, hipStream_t s) {
-#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_connect<SD, SP, false>), dim3(ls.connect), dim3(kTravThreads), 0, s, q)
-#define GP_CALLS(SD, SP) hipLaunchKernelGGL((k_connect<SD, SP, true>), dim3(ls.connect), dim3(kTravThreads), 0, s, q)
+void launchConnect(const Queues& q, const LaunchShape& ls, Sink& k) {
+#define GP_CALL(SD, SP) enqueue(k, k_connect<SD, SP, false>, dim3(ls.connect), dim3(kTravThreads), q)
+#define GP_CALLS(SD, SP) enqueue(k, k_connect<SD, SP, true>, dim3(ls.connect), dim3(kTravThreads), q)
     if (q.stats) GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALLS);
     else GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALL);
 #undef GP_CALLS
@@ -1880,8 +1907,8 @@ void launchFlight(const Queues& q, unsigned n, unsigned lanes, int blocks, hipSt
     GP_BY_STACK_EXT(q.lds, q.useSpill, GP_CALL);
 #undef GP_CALL
 }
-void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s) {
-#define GP_CALL(SD, SP) hipLaunchKernelGGL((k_mirror<SD, SP>), dim3(ls.mirror), dim3(kFlightThreads), 0, s, q)
+void launchMirror(const Queues& q, const LaunchShape& ls, Sink& k) {
+#define GP_CALL(SD, SP) enqueue(k, k_mirror<SD, SP>, dim3(ls.mirror), dim3(kFlightThreads), q)
     GP_BY_STACK(q.connLds, q.connUseSpill, GP_CALL);
 #undef GP_CALL
 }

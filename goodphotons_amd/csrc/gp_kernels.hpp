@@ -80,20 +80,31 @@ struct LaunchShape {
     int emit, extend, shade, connect, mirror;
 };
 
-void launchSchedule(const Queues& q, int cur, hipStream_t s);
+// Where the wavefront's kernels go: onto a stream, or to the end of a graph's chain of nodes.
+// Graphs are built node by node and not by capturing a stream: what other threads enqueue
+// meanwhile cannot become part of them, and a synchronous copy of another thread (of this
+// library's or of the program's own) ends a capture in an error on any stream.
+struct Sink {
+    hipStream_t stream = nullptr;
+    hipGraph_t graph = nullptr;
+    hipGraphNode_t last = nullptr;
+    hipError_t error = hipSuccess;   // of the last node that could not be added
+};
+
+void launchSchedule(const Queues& q, int cur, Sink& k);
 // Sorts the iteration's emission slots (four kernels; only with q.emitOrder).
-void launchEmitOrder(const Queues& q, hipStream_t s);
-void launchEmit(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s);
-void launchExtend(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s);
-void launchShade(const Queues& q, int cur, const LaunchShape& ls, hipStream_t s);
-void launchConnect(const Queues& q, const LaunchShape& ls, hipStream_t s);
+void launchEmitOrder(const Queues& q, Sink& k);
+void launchEmit(const Queues& q, int cur, const LaunchShape& ls, Sink& k);
+void launchExtend(const Queues& q, int cur, const LaunchShape& ls, Sink& k);
+void launchShade(const Queues& q, int cur, const LaunchShape& ls, Sink& k);
+void launchConnect(const Queues& q, const LaunchShape& ls, Sink& k);
 // Ray binning of queue `cur` into queue 2 (four kernels: count, chunk sums, bin scan,
 // scatter).
-void launchBin(const Queues& q, int cur, hipStream_t s);
+void launchBin(const Queues& q, int cur, Sink& k);
 // A whole trace of n photons of job 0, `lanes` of each wave carrying photons; at most
 // the closest-hit kernel's threads (its spill area is sized for those).
 void launchFlight(const Queues& q, unsigned n, unsigned lanes, int blocks, hipStream_t s);
-void launchMirror(const Queues& q, const LaunchShape& ls, hipStream_t s);
+void launchMirror(const Queues& q, const LaunchShape& ls, Sink& k);
 
 // Batch probes of n rays (device or pinned host memory), `blocks` one-wave workgroups with
 // spillDepth spill entries per thread.

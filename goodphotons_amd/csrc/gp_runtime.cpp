@@ -42,8 +42,7 @@ DeviceState& device() {
             return d;
         }
         if (hipSetDevice(0) != hipSuccess || hipStreamCreate(&d.stream) != hipSuccess ||
-            hipStreamCreate(&d.copyStream) != hipSuccess ||
-            hipStreamCreateWithFlags(&d.captureStream, hipStreamNonBlocking) != hipSuccess) {
+            hipStreamCreate(&d.copyStream) != hipSuccess) {
             d.why = "stream creation failed";
             return d;
         }
@@ -665,8 +664,9 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
 
 // One launch, timed with HIP events while gp_tuning.profile is set.
 template <class F>
-gp_status Engine::timed(int k, hipStream_t s, F&& launch) {
+gp_status Engine::timed(int k, const Sink& sink, F&& launch) {
     if (!tun.profile) { launch(); return GP_OK; }
+    hipStream_t s = sink.stream;   // timed iterations are never part of a graph
     std::array<hipEvent_t, 2> ev;
     GP_HIP(hipEventCreate(&ev[0]));
     GP_HIP(hipEventCreate(&ev[1]));
@@ -677,7 +677,7 @@ gp_status Engine::timed(int k, hipStream_t s, F&& launch) {
     return GP_OK;
 }
 
-gp_status Engine::enqueueEmit(const LaunchShape& sh, hipStream_t s) {
+gp_status Engine::enqueueEmit(const LaunchShape& sh, Sink& s) {
     return timed(1, s, [&] {
         if (q.emitOrder) launchEmitOrder(q, s);
         launchEmit(q, parity, sh, s);
@@ -685,7 +685,7 @@ gp_status Engine::enqueueEmit(const LaunchShape& sh, hipStream_t s) {
 }
 
 // Closest hit, scatter and connections of the paths in queue `parity`.
-gp_status Engine::enqueueBounce(const LaunchShape& sh, hipStream_t s) {
+gp_status Engine::enqueueBounce(const LaunchShape& sh, Sink& s) {
     const int cur = parity;
     gp_status st;
     if (q.binned)
@@ -713,7 +713,7 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
     // the first iteration connects the emitted photons and the shaded vertices
     sh.connect = blocks(2 * (uint64_t)n * (uint64_t)cams, 256, ls.connect);
     sh.mirror = blocks(2 * (uint64_t)n, kFlightThreads, ls.mirror);
-    hipStream_t s = device().stream;
+    Sink s{device().stream};
     gp_status st;
     if ((st = enqueueEmit(sh, s)) != GP_OK) return st;
     const int K = chunkIterations(tun);
@@ -760,7 +760,7 @@ gp_status Engine::fly(unsigned n, int maxDepth) {
     return st;
 }
 
-gp_status Engine::enqueueIterations(int n, hipStream_t s) {
+gp_status Engine::enqueueIterations(int n, Sink& s) {
     gp_status st;
     for (int i = 0; i < n; ++i) {
         if ((st = timed(0, s, [&] { launchSchedule(q, parity, s); })) != GP_OK) return st;
@@ -797,23 +797,23 @@ gp_status Engine::collectProfile() {
 
 gp_status Engine::runIterations(int n) {
     hipStream_t s = device().stream;
+    Sink direct{s};
     const int K = chunkIterations(tun);
-    if (!tun.use_graph || tun.profile || q.stats || parity != 0 || n < K) return enqueueIterations(n, s);
+    if (!tun.use_graph || tun.profile || q.stats || parity != 0 || n < K) return enqueueIterations(n, direct);
     if (!graph || graphIters != K || graphLds != q.lds || graphMirror != mirrorActive || graphBinned != q.binned ||
         graphEmitOrder != q.emitOrder) {
         if (graph) { hipGraphExecDestroy(graph); graph = nullptr; }
-        hipGraph_t g;
-        hipStream_t cs = device().captureStream;
-        GP_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+        Sink nodes;
+        GP_HIP(hipGraphCreate(&nodes.graph, 0));
         int saved = parity;
-        gp_status st = enqueueIterations(K, cs);
-        hipError_t ce = hipStreamEndCapture(cs, &g);
+        gp_status st = enqueueIterations(K, nodes);
         parity = saved;
+        hipError_t e = nodes.error;
+        if (st == GP_OK && e == hipSuccess && (e = hipGraphInstantiate(&graph, nodes.graph, nullptr, nullptr, 0)) != hipSuccess)
+            graph = nullptr;
+        hipGraphDestroy(nodes.graph);
         if (st != GP_OK) return st;
-        if (ce != hipSuccess) return fail(GP_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(ce));
-        hipError_t ie = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
-        hipGraphDestroy(g);
-        if (ie != hipSuccess) { graph = nullptr; return fail(GP_ERR_HIP, "hipGraphInstantiate failed"); }
+        if (e != hipSuccess) return fail(GP_ERR_HIP, std::string("iteration graph: ") + hipGetErrorString(e));
         graphIters = K;
         graphLds = q.lds;
         graphMirror = mirrorActive;
@@ -825,7 +825,7 @@ gp_status Engine::runIterations(int n) {
         GP_HIP(hipGraphLaunch(graph, s));
         done += K;
     }
-    if (done < n) return enqueueIterations(n - done, s);
+    if (done < n) return enqueueIterations(n - done, direct);
     return GP_OK;
 }
 

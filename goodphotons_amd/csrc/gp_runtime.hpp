@@ -129,11 +129,6 @@ struct DeviceState {
     std::string name, arch;
     hipStream_t stream = nullptr;       // engine work
     hipStream_t copyStream = nullptr;   // result downloads that overlap engine work
-    // Graphs are captured here and launched on `stream`. Nothing else uses it: film calls of
-    // other threads launch and synchronise on `stream` without the engine's lock, and what
-    // enters a stream while it is captured becomes part of the graph or ends the capture.
-    // Non-blocking, so that work on the null stream does not touch the capture either.
-    hipStream_t captureStream = nullptr;
 };
 DeviceState& device();
 gp_status requireDevice();
@@ -271,9 +266,9 @@ struct Engine {
     void releaseQueues();
     void releaseSpill();
     template <class F>
-    gp_status timed(int k, hipStream_t s, F&& launch);
-    gp_status enqueueEmit(const LaunchShape& sh, hipStream_t s);
-    gp_status enqueueBounce(const LaunchShape& sh, hipStream_t s);
+    gp_status timed(int k, const Sink& s, F&& launch);
+    gp_status enqueueEmit(const LaunchShape& sh, Sink& s);
+    gp_status enqueueBounce(const LaunchShape& sh, Sink& s);
     // Runs a trace whose n photons fit the path queue, from k_start_trace (once) to the
     // last path's end; reads the control block and slot 0's rows back. Every live path
     // advances one segment per iteration, so maxDepth iterations end it; the host looks
@@ -286,7 +281,7 @@ struct Engine {
     // traversal statistics, kernel timing and ray binning belong to the wavefront's kernels.
     bool flies(uint64_t n, int cams) const;
     gp_status fly(unsigned n, int maxDepth);
-    gp_status enqueueIterations(int n, hipStream_t s);   // plain launches, tracks parity
+    gp_status enqueueIterations(int n, Sink& s);    // tracks parity
     gp_status runIterations(int n);           // graph replay when possible
     // Whether new photons are emitted in sorted order (set by the caller before
     // runIterations, from the most photons one job of the wavefront emits).

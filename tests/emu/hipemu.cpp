@@ -155,7 +155,7 @@ std::mutex gRun;
 std::mutex gState;
 std::map<std::string, long long> gLaunches;
 long long gStreamSyncs = 0;
-void (*gOnCapture)() = nullptr;
+void (*gOnGraph)() = nullptr;
 
 bool async() {
     static const bool on = getenv("EMU_ASYNC") && atoi(getenv("EMU_ASYNC")) != 0;
@@ -181,6 +181,13 @@ struct EmuGraph {
 
 static EmuStream gNullStream;
 static EmuStream* streamOf(hipStream_t s) { return s ? s : &gNullStream; }
+static EmuStream* gCapturing = nullptr;   // the stream under capture, if any
+
+// A synchronous call: ends a capture in an error, whichever stream is captured.
+static void synchronous() {
+    std::lock_guard<std::mutex> lock(gState);
+    if (gCapturing) gCapturing->invalid = true;
+}
 
 unsigned long long emu_ballot(int pred, void* site) {
     Lane& L = *gLane;
@@ -229,8 +236,15 @@ static void runRec(const Rec& r) {
     for (unsigned bx = 0; bx < r.g.x; ++bx) runBlock(r.fn, bx, r.b.x);
 }
 
-void emu_launch(const char* name, std::function<void()> fn, dim3 g, dim3 b, hipStream_t st) {
+// The kernel's symbol where it has one (launchers pass kernels on under other names).
+static std::string kernelName(const char* given, void* kernel) {
+    Dl_info info;
+    return dladdr(kernel, &info) && info.dli_sname && info.dli_saddr == kernel ? info.dli_sname : given;
+}
+
+void emu_launch(const char* given, void* kernel, std::function<void()> fn, dim3 g, dim3 b, hipStream_t st) {
     EmuStream* s = streamOf(st);
+    const std::string name = kernelName(given, kernel);
     {
         std::lock_guard<std::mutex> lock(gState);
         if (s->capturing) {
@@ -254,7 +268,7 @@ static hipError_t enqueueOther(hipStream_t st) {
     return hipSuccess;
 }
 
-void emu_on_capture(void (*cb)()) { gOnCapture = cb; }
+void emu_on_graph(void (*cb)()) { gOnGraph = cb; }
 long long emu_launches(const char* part) {
     std::lock_guard<std::mutex> lock(gState);
     long long n = 0;
@@ -303,7 +317,8 @@ hipError_t hipFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipFreeAsync(void* p, hipStream_t) { free(p); return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
 hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
-hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { if (n) std::memmove(d, s, n); return hipSuccess; }
+static hipError_t copyNow(void* d, const void* s, size_t n) { if (n) std::memmove(d, s, n); return hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { synchronous(); return copyNow(d, s, n); }
 hipError_t hipMemcpy2D(void* d, size_t dpitch, const void* s, size_t spitch, size_t width, size_t height,
                        hipMemcpyKind) {
     if (width > dpitch || width > spitch) return hipErrorInvalidValue;
@@ -311,11 +326,11 @@ hipError_t hipMemcpy2D(void* d, size_t dpitch, const void* s, size_t spitch, siz
         std::memmove((char*)d + r * dpitch, (const char*)s + r * spitch, width);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t st) {
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
     const hipError_t e = enqueueOther(st);
-    return e != hipSuccess ? e : hipMemcpy(d, s, n, k);
+    return e != hipSuccess ? e : copyNow(d, s, n);
 }
-hipError_t hipMemset(void* d, int v, size_t n) { std::memset(d, v, n); return hipSuccess; }
+hipError_t hipMemset(void* d, int v, size_t n) { synchronous(); std::memset(d, v, n); return hipSuccess; }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t st) {
     const hipError_t e = enqueueOther(st);
     if (e == hipSuccess) std::memset(d, v, n);
@@ -357,6 +372,12 @@ hipError_t hipEventQuery(hipEvent_t e) {
     return async() && e->s && e->at > e->s->done ? hipErrorNotReady : hipSuccess;
 }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0.f; return hipSuccess; }
+static void onGraph() {
+    if (void (*cb)() = gOnGraph) {
+        gOnGraph = nullptr;
+        cb();
+    }
+}
 hipError_t hipStreamBeginCapture(hipStream_t st, hipStreamCaptureMode) {
     EmuStream* s = streamOf(st);
     {
@@ -364,17 +385,30 @@ hipError_t hipStreamBeginCapture(hipStream_t st, hipStreamCaptureMode) {
         s->capturing = true;
         s->invalid = false;
         s->captured.clear();
+        gCapturing = s;
     }
-    if (void (*cb)() = gOnCapture) {
-        gOnCapture = nullptr;
-        cb();
-    }
+    onGraph();
+    return hipSuccess;
+}
+hipError_t hipGraphCreate(hipGraph_t* g, unsigned) {
+    *g = new EmuGraph();
+    onGraph();
+    return hipSuccess;
+}
+hipError_t hipGraphAddKernelNode(hipGraphNode_t* node, hipGraph_t g, const hipGraphNode_t* deps, size_t n,
+                                 const hipKernelNodeParams* p) {
+    // nodes are numbered from 1 in the order of addition
+    const size_t last = g->recs.size();
+    if ((last == 0) != (n == 0) || n > 1 || (n == 1 && (size_t)deps[0] != last)) return hipErrorInvalidValue;
+    g->recs.push_back({kernelName("node", p->func.at), p->func.bind(p->kernelParams), p->gridDim, p->blockDim});
+    *node = (hipGraphNode_t)(last + 1);
     return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t st, hipGraph_t* g) {
     EmuStream* s = streamOf(st);
     std::lock_guard<std::mutex> lock(gState);
     s->capturing = false;
+    gCapturing = nullptr;
     if (s->invalid) { *g = nullptr; return hipErrorStreamCaptureInvalidated; }
     *g = new EmuGraph{s->captured};
     s->captured.clear();

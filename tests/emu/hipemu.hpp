@@ -13,7 +13,8 @@
 //
 // Streams run what they are given at once, but keep the GPU's rules where the library's
 // host code depends on them. A stream that is captured records its launches, whichever
-// thread makes them, and synchronising it ends the capture in an error. With EMU_ASYNC=1
+// thread makes them; synchronising it, or a synchronous copy on any thread, ends the
+// capture in an error. With EMU_ASYNC=1
 // work counts as running until its stream or an event behind it has been waited for
 // (hipEventQuery says not ready until then), and destroying a graph that is still running
 // aborts. emu_on_capture, emu_launches and emu_stream_syncs serve the tests.
@@ -137,7 +138,6 @@ typedef EmuGraph* hipGraph_t;
 typedef EmuGraph* hipGraphExec_t;
 typedef struct hipGraphNode* hipGraphNode_t;
 #define hipEventDisableTiming 2
-#define hipStreamNonBlocking 1
 struct hipDeviceProp_t {
     char name[256];
     char gcnArchName[256];
@@ -184,24 +184,49 @@ hipError_t hipEventQuery(hipEvent_t e);
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b);
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode m);
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g);
+// A kernel of any signature, called with pointers to its arguments.
+struct EmuKernel {
+    void* at = nullptr;
+    std::function<std::function<void()>(void**)> bind;
+    EmuKernel() = default;
+    template <class... P>
+    EmuKernel(void (*k)(P...))
+        : at((void*)k), bind([k](void** a) -> std::function<void()> {
+              return [&]<size_t... I>(std::index_sequence<I...>) -> std::function<void()> {
+                  std::tuple<std::decay_t<P>...> args(*(std::decay_t<P>*)a[I]...);
+                  return [k, args]() { std::apply(k, args); };
+              }(std::index_sequence_for<P...>());
+          }) {}
+};
+struct hipKernelNodeParams {
+    EmuKernel func;
+    dim3 gridDim, blockDim;
+    unsigned sharedMemBytes = 0;
+    void** kernelParams = nullptr;
+    void** extra = nullptr;
+};
+hipError_t hipGraphCreate(hipGraph_t* g, unsigned flags);
+// Nodes run in the order in which they are added: each must depend on the one before it.
+hipError_t hipGraphAddKernelNode(hipGraphNode_t* node, hipGraph_t g, const hipGraphNode_t* deps, size_t n,
+                                 const hipKernelNodeParams* p);
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t* n, char* log, size_t sz);
 hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s);
 hipError_t hipGraphDestroy(hipGraph_t g);
 hipError_t hipGraphExecDestroy(hipGraphExec_t e);
 
-void emu_launch(const char* name, std::function<void()> fn, dim3 g, dim3 b, hipStream_t s);
+void emu_launch(const char* name, void* kernel, std::function<void()> fn, dim3 g, dim3 b, hipStream_t s);
 
 template <class... P, class... A>
 void emu_launch_kernel(const char* name, void (*k)(P...), dim3 g, dim3 b, hipStream_t s, A&&... a) {
     std::tuple<std::decay_t<P>...> args(static_cast<std::decay_t<P>>(std::forward<A>(a))...);
-    emu_launch(name, [k, args]() { std::apply(k, args); }, g, b, s);
+    emu_launch(name, (void*)k, [k, args]() { std::apply(k, args); }, g, b, s);
 }
 #define hipLaunchKernelGGL(K, G, B, SH, ST, ...) emu_launch_kernel(#K, K, dim3(G), dim3(B), ST, ##__VA_ARGS__)
 #define HIP_SYMBOL(x) (&(x))
 
 extern "C" {
-// Calls cb once, inside the next hipStreamBeginCapture.
-void emu_on_capture(void (*cb)());
+// Calls cb once, inside the next hipStreamBeginCapture or hipGraphCreate.
+void emu_on_graph(void (*cb)());
 // Launches (captured ones each time their graph runs) of kernels whose name contains `part`.
 long long emu_launches(const char* part);
 // hipStreamSynchronize calls.

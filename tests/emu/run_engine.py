@@ -5,6 +5,7 @@ import ctypes as C
 import json
 import os
 import sys
+import tempfile
 import threading
 
 import numpy as np
@@ -31,9 +32,9 @@ def film_of(sd, n):
     return gp.Film(sd.camera.res_x, sd.camera.res_y, max_photons=n, lib=lib)
 
 
-def capture():
-    """A film is downloaded and another seeded by a second thread while the first captures
-    the graph of a trace that is refilled."""
+def graph():
+    """A film is downloaded and saved, another seeded and a scene created by a second thread
+    while the first makes the graph of a trace that is refilled."""
     lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
     sd = scenes.cornell_c0(32)
     gs = gp.GpuScene(sd, lib)
@@ -48,6 +49,9 @@ def capture():
             fresh = film_of(sd, 1000)
             fresh.seed(gs, sd.camera, 1000, xyz, hits, max_depth=4)
             y, g = fresh.download()
+            gp.GpuScene(sd, lib).close()
+            with tempfile.TemporaryDirectory() as d:
+                other.save_checkpoint(os.path.join(d, "film"), 1000)
             seen["same"] = bool(np.array_equal(x, xyz) and np.array_equal(h, hits) and np.array_equal(g, hits))
         except gp.GpError as e:
             seen["error"] = str(e)
@@ -58,10 +62,10 @@ def capture():
         t.join()
 
     cb = C.CFUNCTYPE(None)(during)
-    emu.emu_on_capture(cb)
+    emu.emu_on_graph(cb)
     n = 5001
     got = []
-    for _ in range(2):   # captured, then replayed
+    for _ in range(2):   # made, then replayed
         f = film_of(sd, n)
         _, st = gp.trace(gs, sd.camera, f, n, max_depth=4)
         got.append((f.raw()[0], counts(st)))
@@ -226,4 +230,4 @@ def route():
     return out
 
 
-print(json.dumps({"route": route, "flight": flight, "sort": sort, "autotune": autotune, "capture": capture, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+print(json.dumps({"route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

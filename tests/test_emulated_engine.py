@@ -31,7 +31,7 @@ def _run(scenario, libs, cus, preempt=0, run_async=0, variant=""):
 # Each scenario is a child process of its own; all are started at once.
 CASES = {
     "autotune": dict(cus=1),
-    "capture": dict(cus=1),
+    "graph": dict(cus=1),
     "reshape": dict(cus=1, run_async=1),
     "deep": dict(cus=1),
     "flight": dict(cus=2, preempt=3),
@@ -64,10 +64,11 @@ def _result(runs, key):
     return _done[key]
 
 
-def test_film_calls_of_another_thread_stay_out_of_a_graph_capture(runs, orc):
-    # a download and a seed that fall into the capture of a trace's graph neither fail nor
-    # end up in the graph, and the trace holds the oracle's photons
-    out = _result(runs, "capture")
+def test_calls_of_another_thread_stay_out_of_a_graph(runs, orc):
+    # film calls, synchronous ones among them, and a new scene that fall into the making of a
+    # trace's graph neither fail nor end up in the graph, and the trace holds the oracle's
+    # photons
+    out = _result(runs, "graph")
     assert out["seen"] == {"same": True}
     assert out["same"]
     sd = scenes.cornell_c0(32)

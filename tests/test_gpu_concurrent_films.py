@@ -1,11 +1,13 @@
-"""Film calls of other threads while one thread traces: downloads, seeding and the image
-calls use the engine's stream without its lock, and the tracing thread captures a graph
-anew for every trace here (setting the tuning drops the last one). Every result equals the
-one the same call gives alone. Exact equality: no tolerance."""
+"""Calls of other threads while one thread traces: film downloads, seeding and the image
+calls use the engine's stream without its lock; checkpoints, new scenes and the program's
+own transfers make synchronous copies. The tracing thread makes a new graph for every trace
+here (setting the tuning drops the last one). Every result equals the one the same call
+gives alone. Exact equality: no tolerance."""
 import threading
 
 import numpy as np
 import pytest
+import torch
 
 import goodphotons_amd as gp
 from goodphotons_amd import abi, scenes
@@ -13,7 +15,7 @@ from goodphotons_amd import abi, scenes
 pytestmark = pytest.mark.gpu
 
 
-def test_film_calls_beside_graph_captures(gplib):
+def test_calls_beside_the_making_of_graphs(gplib, tmp_path):
     sd = scenes.cornell_c0(96)
     gs = gp.GpuScene(sd, gplib)
     saved = gplib.tuning()
@@ -42,6 +44,9 @@ def test_film_calls_beside_graph_captures(gplib):
                 while not done.is_set():
                     x, h = films[k].download()
                     ok = np.array_equal(x, alone[k][0]) and np.array_equal(h, alone[k][1])
+                    films[k].save_checkpoint(str(tmp_path / f"film{k}"), n)
+                    gp.GpuScene(sd, gplib, builder=("host", "device")[k & 1]).close()
+                    ok = ok and np.array_equal(torch.from_numpy(x).cuda().cpu().numpy(), x)
                     if k == 0:
                         f = gp.Film(96, 96, max_photons=4 * n, lib=gplib)
                         f.seed(gs, sd.camera, n, x, h, max_depth=6)
