@@ -154,7 +154,7 @@ std::mutex gRun;
 // streams, events, counts
 std::mutex gState;
 std::map<std::string, long long> gLaunches;
-long long gStreamSyncs = 0;
+long long gStreamSyncs = 0, gEventRecords = 0;
 void (*gOnGraph)() = nullptr;
 
 bool async() {
@@ -280,6 +280,10 @@ long long emu_stream_syncs() {
     std::lock_guard<std::mutex> lock(gState);
     return gStreamSyncs;
 }
+long long emu_event_records() {
+    std::lock_guard<std::mutex> lock(gState);
+    return gEventRecords;
+}
 
 static int gEmuCus() {
     const char* e = getenv("EMU_CUS");
@@ -358,6 +362,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
     const hipError_t r = enqueueOther(st);
     if (r != hipSuccess) return r;
     std::lock_guard<std::mutex> lock(gState);
+    ++gEventRecords;
     e->s = streamOf(st);
     e->at = e->s->enqueued;
     return hipSuccess;

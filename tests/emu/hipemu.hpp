@@ -17,7 +17,7 @@
 // capture in an error. With EMU_ASYNC=1
 // work counts as running until its stream or an event behind it has been waited for
 // (hipEventQuery says not ready until then), and destroying a graph that is still running
-// aborts. emu_on_capture, emu_launches and emu_stream_syncs serve the tests.
+// aborts. The emu_ functions at the end serve the tests.
 #pragma once
 #include <cmath>
 #include <cstddef>
@@ -229,6 +229,7 @@ extern "C" {
 void emu_on_graph(void (*cb)());
 // Launches (captured ones each time their graph runs) of kernels whose name contains `part`.
 long long emu_launches(const char* part);
-// hipStreamSynchronize calls.
+// hipStreamSynchronize and hipEventRecord calls.
 long long emu_stream_syncs();
+long long emu_event_records();
 }

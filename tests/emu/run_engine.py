@@ -21,6 +21,7 @@ emu = lib.lib
 emu.emu_launches.restype = C.c_longlong
 emu.emu_launches.argtypes = [C.c_char_p]
 emu.emu_stream_syncs.restype = C.c_longlong
+emu.emu_event_records.restype = C.c_longlong
 KEYS = ("photons", "segments", "connections", "splats")
 
 
@@ -230,4 +231,25 @@ def route():
     return out
 
 
-print(json.dumps({"route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def seeding():
+    """Events that seeding a film records (65536 pixels fill a staging slot), and whether its
+    words are the rounded doubles."""
+    sd0, out = scenes.cornell_c0(8), []
+    gs = gp.GpuScene(sd0, lib)
+    for rx, ry in ((1, 1), (16, 16), (1024, 64), (4099, 16)):
+        cam = sd0.with_camera_res(rx, ry).camera
+        rng = np.random.default_rng(rx)
+        h = np.floor(rng.uniform(0, 50, rx * ry))
+        x = rng.uniform(0, 1e12, (rx * ry, 3))
+        f = gp.Film(rx, ry, max_photons=1000, lib=lib)
+        before = emu.emu_event_records()
+        f.seed(gs, cam, 1000, x, h, max_depth=4)
+        events = emu.emu_event_records() - before
+        w, scale = f.raw()
+        out.append([rx * ry, events, bool(np.array_equal(w[:, :3], np.rint(x * scale).astype(np.int64))
+                                          and np.array_equal(w[:, 3], h) and w[:, :3].any())])
+        f.close()
+    return out
+
+
+print(json.dumps({"seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

@@ -37,6 +37,7 @@ CASES = {
     "flight": dict(cus=2, preempt=3),
     "sort": dict(cus=1, variant="sort"),
     "route": dict(cus=1),
+    "seeding": dict(cus=1),
 }
 # emission sorted from 64 photons on, in traces of 1000
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000")}
@@ -132,3 +133,11 @@ def test_traces_of_many_cameras_do_not_fly(runs):
     # 1024 resident lanes: up to 1.5 photons a lane, less by cameras^1.5, and six cameras
     for cams, n, flown in _result(runs, "route"):
         assert flown == (1 if cams <= 6 and n * cams ** 1.5 <= 1536 else 0), (cams, n)
+
+
+def test_seeding_a_film_of_up_to_a_slot_is_one_synchronous_copy(runs):
+    # no event and no staging ring; the words are the rounded doubles on either side of a slot
+    out = _result(runs, "seeding")
+    assert [npx for npx, *_ in out] == [1, 256, 65536, 65584]
+    assert all(same for *_, same in out)
+    assert [events > 0 for _, events, _ in out] == [False, False, False, True]
