@@ -131,6 +131,19 @@ gp_status downloadTotals(const gp_film& f, double* xyz, double* hits, hipStream_
     const size_t each = (xyz ? 24 : 0) + (hits ? 8 : 0);
     if (each == 0) return GP_OK;
     const double inv = f.scale > 0 ? 1.0 / f.scale : 0.0;
+    if ((size_t)f.rx * f.ry <= kHostTotals)
+        return stagedDown(
+            (size_t)f.rx * f.ry, 32, s,
+            [&](char* slot, size_t, size_t n) {
+                return hipMemcpyAsync(slot, f.d, n * 32, hipMemcpyDeviceToHost, s);
+            },
+            [&](const char* slot, size_t, size_t n) {
+                const long long* w = (const long long*)slot;
+                for (size_t i = 0; i < n; ++i) {
+                    for (int c = 0; c < 3 && xyz; ++c) xyz[3 * i + c] = (double)w[4 * i + c] * inv;
+                    if (hits) hits[i] = (double)w[4 * i + 3];
+                }
+            });
     return stagedDown(
         (size_t)f.rx * f.ry, each, s,
         [&](char* slot, size_t first, size_t n) {

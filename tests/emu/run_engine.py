@@ -252,4 +252,21 @@ def seeding():
     return out
 
 
-print(json.dumps({"seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def totals():
+    """Launches of the conversion kernel by film size, and whether the doubles are the words."""
+    sd0, out = scenes.cornell_c0(8), []
+    gs = gp.GpuScene(sd0, lib)
+    for rx, ry in ((1, 1), (32, 32), (64, 48), (439, 7)):
+        f = gp.Film(rx, ry, max_photons=200, lib=lib)
+        gp.trace(gs, sd0.with_camera_res(rx, ry).camera, f, 200, max_depth=2)
+        w, scale = f.raw()
+        before = emu.emu_launches(b"k_film_totals")
+        x, h = f.download()
+        only = f.download_hits()
+        out.append([rx * ry, emu.emu_launches(b"k_film_totals") - before,
+                    bool(np.array_equal(x, w[:, :3] * (1.0 / scale)) and np.array_equal(h, w[:, 3])
+                         and np.array_equal(only, h) and h.any())])
+    return out
+
+
+print(json.dumps({"totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

@@ -38,6 +38,7 @@ CASES = {
     "sort": dict(cus=1, variant="sort"),
     "route": dict(cus=1),
     "seeding": dict(cus=1),
+    "totals": dict(cus=1),
 }
 # emission sorted from 64 photons on, in traces of 1000
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000")}
@@ -141,3 +142,10 @@ def test_seeding_a_film_of_up_to_a_slot_is_one_synchronous_copy(runs):
     assert [npx for npx, *_ in out] == [1, 256, 65536, 65584]
     assert all(same for *_, same in out)
     assert [events > 0 for _, events, _ in out] == [False, False, False, True]
+
+
+def test_small_downloads_are_converted_on_the_host(runs):
+    # the same doubles on either side of the limit
+    out = _result(runs, "totals")
+    assert all(same for *_, same in out)
+    assert [launches for _, launches, _ in out] == [0, 0, 0, 2]   # 3073 pixels: both calls
