@@ -127,6 +127,13 @@ gp_status copyDownLocked(Staging& g, void* dst, const void* src, size_t bytes, h
         [&](const char* slot, size_t first, size_t n) { std::memcpy((char*)dst + first, slot, n); });
 }
 
+void wordsToTotals(const long long* words, size_t n, double inv, double* xyz, double* hits) {
+    for (size_t i = 0; i < n; ++i) {
+        for (int c = 0; c < 3 && xyz; ++c) xyz[3 * i + c] = (double)words[4 * i + c] * inv;
+        if (hits) hits[i] = (double)words[4 * i + 3];
+    }
+}
+
 gp_status downloadTotals(const gp_film& f, double* xyz, double* hits, hipStream_t s) {
     const size_t each = (xyz ? 24 : 0) + (hits ? 8 : 0);
     if (each == 0) return GP_OK;
@@ -137,13 +144,7 @@ gp_status downloadTotals(const gp_film& f, double* xyz, double* hits, hipStream_
             [&](char* slot, size_t, size_t n) {
                 return hipMemcpyAsync(slot, f.d, n * 32, hipMemcpyDeviceToHost, s);
             },
-            [&](const char* slot, size_t, size_t n) {
-                const long long* w = (const long long*)slot;
-                for (size_t i = 0; i < n; ++i) {
-                    for (int c = 0; c < 3 && xyz; ++c) xyz[3 * i + c] = (double)w[4 * i + c] * inv;
-                    if (hits) hits[i] = (double)w[4 * i + 3];
-                }
-            });
+            [&](const char* slot, size_t, size_t n) { wordsToTotals((const long long*)slot, n, inv, xyz, hits); });
     return stagedDown(
         (size_t)f.rx * f.ry, each, s,
         [&](char* slot, size_t first, size_t n) {

@@ -181,6 +181,8 @@ gp_status copyDown(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Film words -> the doubles of gp_film_download: pixels [0, n) of `film` to xyz (3 n, may be
 // null) and hits (n, may be null), word * inv and word.
 void launchFilmTotals(const unsigned long long* film, size_t n, double inv, double* xyz, double* hits, hipStream_t s);
+// The same on the host.
+void wordsToTotals(const long long* words, size_t n, double inv, double* xyz, double* hits);
 // Those doubles into a caller's arrays (either may be null), after the work on s. Up to
 // kHostTotals pixels the host converts a copy of the words: a kernel that writes to pinned
 // memory takes longer than so small a copy (kernel -> host, whole calls: 1024 pixels 16.8 ->

@@ -440,7 +440,9 @@ gp_status gp_autotune(gp_scene* scene, const gp_camera_desc* cam,
 
 /* ---- serving: many jobs in one wavefront -------------------------------- */
 typedef struct gp_server_config {
-    int64_t hbm_budget_bytes; /* admission limit for films + queues of live jobs   */
+    int64_t hbm_budget_bytes; /* admission limit for films + queues of live jobs (scratch
+                                 as large as the largest film comes on top while
+                                 memory lasts)                                      */
     int32_t max_live_jobs;    /* job slots in the device job table (<= 256)        */
     int32_t order_policy;     /* GP_ORDER_SHORTEST_FIRST (0) or GP_ORDER_ADMISSION */
 } gp_server_config;

@@ -316,7 +316,13 @@ hipError_t hipMalloc(void** p, size_t n) {
     std::memset(*p, f ? atoi(f) : 0xA5, n);
     return hipSuccess;
 }
-hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) { return hipMalloc(p, n); }
+static long long gAsyncAllowed = -1;
+void emu_fail_async_allocations(long long allowed) { gAsyncAllowed = allowed; }
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) {
+    if (gAsyncAllowed == 0) return hipErrorOutOfMemory;
+    if (gAsyncAllowed > 0) --gAsyncAllowed;
+    return hipMalloc(p, n);
+}
 hipError_t hipFree(void* p) { free(p); return hipSuccess; }
 hipError_t hipFreeAsync(void* p, hipStream_t) { free(p); return hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }

@@ -232,4 +232,6 @@ long long emu_launches(const char* part);
 // hipStreamSynchronize and hipEventRecord calls.
 long long emu_stream_syncs();
 long long emu_event_records();
+// After `allowed` more calls hipMallocAsync fails (a negative number: never).
+void emu_fail_async_allocations(long long allowed);
 }

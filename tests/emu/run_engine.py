@@ -269,4 +269,30 @@ def totals():
     return out
 
 
-print(json.dumps({"totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def films():
+    """Films of a server's jobs of several sizes, with scratch to convert them in and without
+    (allocations fail after those of the films), against the same traces."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
+    sd0, out = scenes.cornell_c0(8), []
+    gs = gp.GpuScene(sd0, lib)
+    cams = [sd0.with_camera_res(*r).camera for r in ((9, 5), (40, 30), (33, 7))]
+    emu.emu_fail_async_allocations.argtypes = [C.c_longlong]
+    for allowed in (-1, len(cams)):
+        srv = gp.Server(lib=lib)
+        emu.emu_fail_async_allocations(allowed)
+        before = emu.emu_launches(b"k_film_totals")
+        ids = [srv.submit(gs, c, 64, seed_base=7 * k, max_depth=2) for k, c in enumerate(cams)]
+        srv.step()
+        converted = emu.emu_launches(b"k_film_totals") - before
+        emu.emu_fail_async_allocations(-1)
+        same = True
+        for k, (j, c) in enumerate(zip(ids, cams)):
+            r, x, h = srv.take(j, c.res_x, c.res_y)
+            xa, ha, _, _ = gp.render_forward(gs, c, 64, seed_base=7 * k, max_depth=2)
+            same = same and r.status == 0 and bool(np.array_equal(x, xa) and np.array_equal(h, ha))
+        srv.close()
+        out.append([converted, same])
+    return out
+
+
+print(json.dumps({"films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

@@ -39,6 +39,7 @@ CASES = {
     "route": dict(cus=1),
     "seeding": dict(cus=1),
     "totals": dict(cus=1),
+    "films": dict(cus=1),
 }
 # emission sorted from 64 photons on, in traces of 1000
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000")}
@@ -149,3 +150,7 @@ def test_small_downloads_are_converted_on_the_host(runs):
     out = _result(runs, "totals")
     assert all(same for *_, same in out)
     assert [launches for _, launches, _ in out] == [0, 0, 0, 2]   # 3073 pixels: both calls
+
+
+def test_a_servers_films_with_and_without_scratch_to_convert_them_in(runs):
+    assert _result(runs, "films") == [[3, True], [0, True]]
