@@ -130,7 +130,7 @@ struct Ring {
         if (!busy[k]) return hipSuccess;
         busy[k] = false;
         const hipError_t e = hipEventSynchronize(g.ev[k]);
-        if (e == hipSuccess && dst[k]) std::memcpy(dst[k], g.host + k * Staging::kSlot, bytes[k]);
+        if (e == hipSuccess && dst[k]) copyOut(dst[k], g.host + k * Staging::kSlot, bytes[k]);
         return e;
     }
     hipError_t acquire(int& k) {

@@ -315,7 +315,7 @@ gp_status gp_film_to_linear(gp_film* film, int64_t n_photons, float* rgb) {
             return hipGetLastError();
         },
         [&](const char* slot, size_t first, size_t n) {
-            std::memcpy(rgb + 3 * first, slot, n * 3 * sizeof(float));
+            copyOut(rgb + 3 * first, slot, n * 3 * sizeof(float));
         });
 }
 

@@ -124,7 +124,7 @@ gp_status copyDownLocked(Staging& g, void* dst, const void* src, size_t bytes, h
         [&](char* slot, size_t first, size_t n) {
             return hipMemcpyAsync(slot, (const char*)src + first, n, hipMemcpyDeviceToHost, s);
         },
-        [&](const char* slot, size_t first, size_t n) { std::memcpy((char*)dst + first, slot, n); });
+        [&](const char* slot, size_t first, size_t n) { copyOut((char*)dst + first, slot, n); });
 }
 
 void wordsToTotals(const long long* words, size_t n, double inv, double* xyz, double* hits) {
@@ -154,8 +154,8 @@ gp_status downloadTotals(const gp_film& f, double* xyz, double* hits, hipStream_
         },
         [&](const char* slot, size_t first, size_t n) {
             const double* x = (const double*)slot;
-            if (xyz) std::memcpy(xyz + 3 * first, x, n * 24);
-            if (hits) std::memcpy(hits + first, x + (xyz ? 3 * n : 0), n * 8);
+            if (xyz) copyOut(xyz + 3 * first, x, n * 24);
+            if (hits) copyOut(hits + first, x + (xyz ? 3 * n : 0), n * 8);
         });
 }
 

@@ -133,6 +133,15 @@ struct DeviceState {
 DeviceState& device();
 gp_status requireDevice();
 
+// memcpy of results into a caller's array, in pieces: one of megabytes goes past the caches,
+// and into fresh pages, which the kernel has just cleared there, that takes half as long again
+// (5.5 MB 157 -> 105 us, 34 MB 1.70 -> 1.13 ms).
+inline void copyOut(void* dst, const void* src, size_t bytes) {
+    constexpr size_t kPiece = size_t(256) << 10;
+    for (size_t at = 0; at < bytes; at += kPiece)
+        std::memcpy((char*)dst + at, (const char*)src + at, std::min(kPiece, bytes - at));
+}
+
 // Moves `items` items of `each` bytes from the device: fill(slot, first, count) enqueues on
 // s what writes items [first, first + count) to the pinned slot, drain(slot, first, count)
 // takes them on the host. Returns when all are drained. One thread drains: what is left of

@@ -515,8 +515,8 @@ gp_status gp_server_take_result(gp_server* srv, int64_t jobId, gp_job_result* re
             if (J.filmWords) {
                 wordsToTotals((const long long*)J.filmHost, np, J.film->scale > 0 ? 1.0 / J.film->scale : 0.0, xyz, hits);
             } else {
-                if (xyz) std::memcpy(xyz, J.filmHost, np * 3 * sizeof(double));
-                if (hits) std::memcpy(hits, J.filmHost + 3 * np, np * sizeof(double));
+                if (xyz) copyOut(xyz, J.filmHost, np * 3 * sizeof(double));
+                if (hits) copyOut(hits, J.filmHost + 3 * np, np * sizeof(double));
             }
         }
         srv->pool.put(J.filmHost);
