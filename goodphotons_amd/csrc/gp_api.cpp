@@ -715,7 +715,7 @@ gp_status gp::traceShared(gp_scene* s, int n_cams, const gp_camera_desc* cams, g
     if ((st = E.ensure((unsigned)E.tun.queue_capacity, lds, s->stackNeed, n_cams, s->nMirrors > 0)) != GP_OK)
         return st;
     E.mirrorActive = s->nMirrors > 0;
-    E.setEmitOrder((uint64_t)p->n_photons);
+    E.setEmitOrder(E.wantsEmitOrder((uint64_t)p->n_photons));
     // the statistics variants run for this call only (plain launches, no graph); set
     // after ensure(), which may rebuild the queue descriptor
     struct StatsScope {

@@ -298,10 +298,13 @@ struct Engine {
     gp_status fly(unsigned n, int maxDepth);
     gp_status enqueueIterations(int n, Sink& s);    // tracks parity
     gp_status runIterations(int n);           // graph replay when possible
-    // Whether new photons are emitted in sorted order (set by the caller before
-    // runIterations, from the most photons one job of the wavefront emits).
+    // Whether new photons of a trace, or of a server's jobs (the largest and all of them), are
+    // emitted in sorted order (set by the caller before runIterations).
     bool wantsEmitOrder(uint64_t photons) const { return photons >= kEmitOrderJobMin && capacity >= kEmitOrderMin; }
-    void setEmitOrder(uint64_t photons) { q.emitOrder = wantsEmitOrder(photons) ? 1 : 0; }
+    bool wantsEmitOrder(uint64_t largest, uint64_t all) const {
+        return all >= kEmitOrderServerMin && wantsEmitOrder(largest);
+    }
+    void setEmitOrder(bool on) { q.emitOrder = on ? 1 : 0; }
     gp_status readCtrl();                     // synchronous copy of the control block and slot 0's rows
 };
 Engine& engine();

@@ -422,10 +422,12 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
     gp_status st;
     int maxStackNeed = 0;
     bool mirrors = false;
-    int64_t maxPhotons = 0;
+    uint64_t maxPhotons = 0, allPhotons = 0;
     for (auto& kv : srv->jobs) {
         if (kv.second.state == JobState::Finished) continue;   // its scene is no longer used
-        maxPhotons = std::max<int64_t>(maxPhotons, kv.second.desc.params.n_photons);
+        const uint64_t photons = (uint64_t)kv.second.desc.params.n_photons;
+        maxPhotons = std::max(maxPhotons, photons);
+        allPhotons += photons;
         maxStackNeed = std::max(maxStackNeed, kv.second.desc.scene->stackNeed);
         mirrors = mirrors || kv.second.desc.scene->nMirrors > 0;
     }
@@ -434,7 +436,7 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
         // a change of engine shape re-allocates, and one of the iteration's kernels drops the
         // graph: neither may happen under running chunks
         if (!E.shapeFor((unsigned)E.tun.queue_capacity, lds, maxStackNeed, 1, mirrors).same ||
-            mirrors != E.mirrorActive || E.wantsEmitOrder((uint64_t)maxPhotons) != (E.q.emitOrder != 0)) {
+            mirrors != E.mirrorActive || E.wantsEmitOrder(maxPhotons, allPhotons) != (E.q.emitOrder != 0)) {
             while (!srv->inflight.empty())
                 if ((st = processOldest(E, srv)) != GP_OK) return st;
             GP_HIP(hipStreamSynchronize(device().stream));
@@ -443,7 +445,7 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
     const unsigned oldCap = E.capacity, oldSeg = E.segCap;
     if ((st = E.ensure((unsigned)E.tun.queue_capacity, lds, maxStackNeed, 1, mirrors)) != GP_OK) return st;
     E.mirrorActive = mirrors;
-    E.setEmitOrder((uint64_t)maxPhotons);
+    E.setEmitOrder(E.wantsEmitOrder(maxPhotons, allPhotons));
     const bool fresh = !srv->engineReady || E.capacity != oldCap || E.segCap != oldSeg || srv->epoch != E.epoch;
     if (fresh) {
         if (!srv->order.empty() || !srv->inflight.empty())

@@ -65,30 +65,33 @@ constexpr int kBinCellsPerAxis = 8;
 // Whole renders, index order -> sorted: 5.24M-triangle icosphere (2^28 photons, 1024^2)
 // 219.0 -> 204.0 ms, closest-hit kernel 147 -> 131; glass sphere and prism (2^26, 512^2)
 // 66.9 -> 62.7 ms; the box (2^22) 4.73 -> 4.64 ms.
-// The four sorting kernels take about 35 us in an iteration that emits and 8 us in one that
-// does not, so the rule is on the photons of a trace (one refill: sorted once) or of a
-// server's largest job (every iteration). Index order -> sorted, ms:
-//   photons                   2^18           2^19           2^20           2^21
-//   trace: box                               1.00 -> 1.01   1.32 -> 1.29   1.97 -> 1.90
-//          glass, prism                      2.71 -> 2.44   2.87 -> 2.77   3.89 -> 3.57
-//          soup 100K tri.                    5.00 -> 4.91   5.83 -> 5.75   7.45 -> 7.19
-//          icosphere 1.3M                    3.04 -> 3.07   3.45 -> 3.37   4.11 -> 3.89
-//   4 jobs: box                              2.77 -> 2.81   4.11 -> 4.07   6.67 -> 6.57
-//          glass, prism                      4.91 -> 4.87   6.81 -> 6.46   10.6 -> 9.8
-//   16 jobs: box              14.4 -> 14.4   16.8 -> 16.6   22.6 -> 21.8   34.0 -> 32.3
-//          glass, prism       16.9 -> 16.7   21.0 -> 20.2   29.3 -> 27.2   45.7 -> 41.6
-// (the soup's and the icosphere's jobs gain 1-4% at 2^19 and 4-9% at 2^21). So from 2^19 on
-// it gains or, on the box, costs 1%; fewer photons fly where they are a trace. Refills of
-// fewer than kEmitOrderMin (a few photons to each of the 4096 keys) keep index order.
-// The macros let a CPU test sort a few thousand photons.
+// The four sorting kernels take about 35 us in an iteration that emits and 12 us in one that
+// does not. A trace of one refill is sorted once: from kEmitOrderJobMin photons on it gains
+// or, on the box, costs 1%; fewer photons fly. Index order -> sorted, ms:
+//   photons              2^19           2^20           2^21           2^22
+//   box                  1.00 -> 1.01   1.32 -> 1.29   1.97 -> 1.90   3.38 -> 3.23
+//   glass, prism         2.71 -> 2.44   2.87 -> 2.77   3.89 -> 3.57   5.73 -> 5.08
+//   soup 100K tri.       5.00 -> 4.91   5.83 -> 5.75   7.45 -> 7.19   10.5 -> 10.0
+//   icosphere 1.3M       3.04 -> 3.07   3.45 -> 3.37   4.11 -> 3.89   5.45 -> 4.99
+// A server runs them in every iteration of a chunk, so the photons of all its jobs have to
+// pay for those that emit nothing. Sorted / index order over five scenes and depths of 3, 8
+// and 16, mean (least .. most):
+//   one job     2^19 1.09 (1.02 .. 1.17)   2^20 1.06 (1.01 .. 1.15)   2^21 1.01 (0.95 .. 1.10)
+//   four jobs   2^19 1.03 (0.99 .. 1.12)   2^20 0.99 (0.91 .. 1.07)
+//   in all      3 * 2^20 1.00 (0.92 .. 1.09)   2^22 0.98 (0.90 .. 1.06)
+// hence kEmitOrderServerMin; sixteen jobs of 2^18, as many photons, gain nothing (1.005).
+// Refills of fewer than kEmitOrderMin (a few photons to each of the 4096 keys) keep index
+// order. The macros let a CPU test sort a few thousand photons.
 #ifndef GP_EMIT_COLS
 #define GP_EMIT_COLS 256
 #define GP_EMIT_ORDER_MIN (1u << 16)
 #define GP_EMIT_ORDER_JOB_MIN (1u << 19)
+#define GP_EMIT_ORDER_SERVER_MIN (1u << 22)
 #endif
 constexpr int kEmitCols = GP_EMIT_COLS;
 constexpr unsigned kEmitOrderMin = GP_EMIT_ORDER_MIN;
-constexpr uint64_t kEmitOrderJobMin = GP_EMIT_ORDER_JOB_MIN;
+constexpr uint64_t kEmitOrderJobMin = GP_EMIT_ORDER_JOB_MIN;         // the trace, or a server's largest job
+constexpr uint64_t kEmitOrderServerMin = GP_EMIT_ORDER_SERVER_MIN;   // a server's jobs in all
 
 // A trace that the chip holds at once flies (k_flight) instead of running the wavefront.
 // kFlightWaves: resident waves of k_flight per CU. Per-trace times, wavefront -> flight, on

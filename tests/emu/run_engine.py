@@ -201,6 +201,10 @@ def sort():
     out = {"sorts": sorts, "more_sorts": emu.emu_launches(b"k_emit_perm") - sorts, "counts": counts(st),
            "trace": bool(np.array_equal(whole.raw()[0], parts.raw()[0]) and counts(st) == sums.tolist())}
     srv = gp.Server(lib=lib)
+    srv.submit(gs, sd.camera, 1203, max_depth=1)
+    before = emu.emu_launches(b"k_emit_perm")
+    srv.step()
+    out["one_job_sorts"] = emu.emu_launches(b"k_emit_perm") - before
     jobs = [(gs, sd, 1203, 7), (gs, sd, 350, 9000)]
     ids = [srv.submit(g, d.camera, k, seed_base=s, max_depth=2) for g, d, k, s in jobs]
     srv.step()
@@ -214,6 +218,7 @@ def sort():
         same = same and r.status == 0 and bool(np.array_equal(h, hs))
     srv.close()
     out["server"] = same
+    out["two_job_sorts"] = emu.emu_launches(b"k_emit_perm") - sorts
     return out
 
 
