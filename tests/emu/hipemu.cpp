@@ -7,6 +7,7 @@
 #include <memory>
 #include <mutex>
 #include <semaphore>
+#include <span>
 #include <string>
 #include <thread>
 #include <vector>
@@ -30,46 +31,58 @@ struct Lane {
     unsigned tid = 0;
 };
 
+// The lanes of the running block. Their threads are kept from block to block (blocks run
+// one at a time) and end with the process.
 struct Block {
     std::vector<std::unique_ptr<Lane>> lanes;
     std::binary_semaphore back{0};
+    const std::function<void()>* fn = nullptr;
+    unsigned bx = 0;
     int nLanes = 0;
 };
+Block& block() {
+    static Block* b = new Block();   // never destroyed: the threads wait in it
+    return *b;
+}
 
 thread_local Lane* gLane = nullptr;
-thread_local Block* gBlock = nullptr;
+thread_local unsigned gYields = 0;   // preemption points passed in this block
 
 void yieldLane(Lane& L) {
-    gBlock->back.release();
+    block().back.release();
     L.go.acquire();
 }
 
+void laneThread(Lane* L) {
+    Block& B = block();
+    gLane = L;
+    while (true) {
+        L->go.acquire();
+        threadIdx = dim3(L->tid, 0, 0);
+        blockIdx = dim3(B.bx, 0, 0);
+        gYields = 0;
+        (*B.fn)();
+        L->st = Done;
+        B.back.release();
+    }
+}
+
 void runBlock(const std::function<void()>& fn, unsigned bx, unsigned nthreads) {
-    Block B;
+    Block& B = block();
     B.nLanes = (int)nthreads;
-    for (unsigned t = 0; t < nthreads; ++t) {
+    B.fn = &fn;
+    B.bx = bx;
+    while (B.lanes.size() < nthreads) {
         B.lanes.emplace_back(new Lane());
-        B.lanes.back()->tid = t;
+        B.lanes.back()->tid = (unsigned)B.lanes.size() - 1;
+        std::thread(laneThread, B.lanes.back().get()).detach();
     }
-    std::vector<std::thread> th;
-    th.reserve(nthreads);
-    for (unsigned t = 0; t < nthreads; ++t) {
-        Lane* L = B.lanes[t].get();
-        th.emplace_back([&B, L, &fn, bx]() {
-            L->go.acquire();
-            threadIdx = dim3(L->tid, 0, 0);
-            blockIdx = dim3(bx, 0, 0);
-            gLane = L;
-            gBlock = &B;
-            fn();
-            L->st = Done;
-            B.back.release();
-        });
-    }
+    const std::span<std::unique_ptr<Lane>> lanes(B.lanes.data(), nthreads);
+    for (auto& lp : lanes) lp->st = Runnable;
     while (true) {
         // run every runnable lane until it blocks or finishes
         bool any = false;
-        for (auto& lp : B.lanes) {
+        for (auto& lp : lanes) {
             Lane& L = *lp;
             if (L.st == Runnable) {
                 any = true;
@@ -79,7 +92,7 @@ void runBlock(const std::function<void()>& fn, unsigned bx, unsigned nthreads) {
         }
         (void)any;
         bool preempted = false;
-        for (auto& lp : B.lanes) preempted = preempted || lp->st == Runnable;
+        for (auto& lp : lanes) preempted = preempted || lp->st == Runnable;
         if (preempted) continue;
         // resolve collectives per wave per site
         bool progress = false;
@@ -87,7 +100,7 @@ void runBlock(const std::function<void()>& fn, unsigned bx, unsigned nthreads) {
         for (int w = 0; w < nw; ++w) {
             std::map<void*, std::vector<Lane*>> groups;
             for (int l = w * 64; l < std::min(B.nLanes, w * 64 + 64); ++l) {
-                Lane& L = *B.lanes[l];
+                Lane& L = *lanes[l];
                 if (L.st == AtColl) groups[L.site].push_back(&L);
             }
             for (auto& kv : groups) {
@@ -119,7 +132,7 @@ void runBlock(const std::function<void()>& fn, unsigned bx, unsigned nthreads) {
         }
         if (progress) continue;
         int done = 0, sync = 0;
-        for (auto& lp : B.lanes) {
+        for (auto& lp : lanes) {
             if (lp->st == Done) ++done;
             else if (lp->st == AtSync) ++sync;
         }
@@ -128,19 +141,18 @@ void runBlock(const std::function<void()>& fn, unsigned bx, unsigned nthreads) {
             if (done) { fprintf(stderr, "EMU: barrier with %d exited lanes\n", done); abort(); }
             void* site = nullptr;
             long long orv = 0;
-            for (auto& lp : B.lanes) {
+            for (auto& lp : lanes) {
                 if (lp->st != AtSync) continue;
                 if (!site) site = lp->site;
                 orv |= lp->arg;
             }
-            for (auto& lp : B.lanes)
+            for (auto& lp : lanes)
                 if (lp->st == AtSync) { lp->result = orv != 0; lp->st = Runnable; }
             continue;
         }
         fprintf(stderr, "EMU: deadlock (done %d, at barrier %d)\n", done, sync);
         abort();
     }
-    for (auto& t : th) t.join();
 }
 
 struct Rec {
@@ -207,8 +219,7 @@ unsigned emu_lane() { return gLane->tid & 63; }
 void emu_maybe_yield() {
     static const int every = getenv("EMU_PREEMPT") ? atoi(getenv("EMU_PREEMPT")) : 0;
     if (!every || !gLane) return;
-    static thread_local unsigned count = 0;
-    if (++count % (unsigned)every) return;
+    if (++gYields % (unsigned)every) return;
     Lane& L = *gLane;
     L.st = Runnable;
     yieldLane(L);
