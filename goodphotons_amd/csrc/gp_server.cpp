@@ -83,6 +83,8 @@ struct gp_server {
         gp_trace_stats stats{};
         int64_t installSeq = 0;                  // first chunk that ran with the job installed
         unsigned long long remaining = 0;        // photons not yet emitted (last snapshot)
+        bool once = false;                       // all photons are emitted by the first iteration
+        int64_t doneIter = -1;                   // iterations after which it is complete, once known
         unsigned long long* accHost = nullptr;   // pinned, kSegs * kAccRow words
         double* filmHost = nullptr;              // pinned: XYZ of every pixel, then the hit counts
         bool filmWords = false;                  // ... or the film's words (no scratch to convert them in)
@@ -104,6 +106,7 @@ struct gp_server {
         int64_t seq = 0;
     };
     int64_t chunkSeq = 0;           // sequence number of the next chunk
+    int64_t snapSeq = -1, snapIter = 0;   // the last snapshot read: its chunk, iterations by then
     std::vector<Chunk> ring;
     std::deque<int> inflight;       // ring indices, oldest first
     int ringNext = 0;
@@ -196,6 +199,7 @@ void releaseFilm(gp_film* f, hipStream_t s) {
 
 gp_status admit(Engine& E, gp_server* srv) {
     bool changed = false;
+    const size_t before = srv->order.size();
     hipStream_t s = device().stream;
     while (!srv->waiting.empty()) {
         const int64_t id = srv->waiting.front();
@@ -238,10 +242,28 @@ gp_status admit(Engine& E, gp_server* srv) {
         changed = true;
     }
     if (changed) {
+        unsigned long long photons = 0;
+        for (int64_t id : srv->order) photons += (unsigned long long)srv->jobs[id].desc.params.n_photons;
+        for (size_t k = before; k < srv->order.size(); ++k) srv->jobs[srv->order[k]].once = photons <= E.capacity;
         reorder(srv);
         return uploadOrder(E, srv, -1);
     }
     return GP_OK;
+}
+
+// Whether the chunks in flight, of K iterations each, complete every live job: a job whose
+// photons all fitted the queue when it was installed is complete max_depth iterations later,
+// another when a snapshot has shown its last emission. Another chunk would run on empty queues
+// (8 iterations, 0.3 ms: twice the work of a job that ends with its first chunk).
+bool endsInFlight(const gp_server* srv, int K) {
+    if (srv->inflight.empty()) return false;
+    for (int64_t id : srv->order) {
+        const gp_server::Job& J = srv->jobs.at(id);
+        const bool first = J.once && (srv->chunkSeq - J.installSeq) * K >= J.desc.params.max_depth;
+        const bool known = J.doneIter >= 0 && srv->snapIter + (srv->chunkSeq - 1 - srv->snapSeq) * K >= J.doneIter;
+        if (!first && !known) return false;
+    }
+    return true;
 }
 
 // A finished job's results leave the device: ledger rows on the engine stream (so a
@@ -328,12 +350,15 @@ gp_status processOldest(Engine& E, gp_server* srv) {
     srv->inflight.pop_front();
     const Ctrl& h = *c.snap;
     if (h.overflow) return fail(GP_ERR_CAPACITY, "wavefront queue segment overflow");
+    srv->snapSeq = c.seq;
+    srv->snapIter = h.iter;
     bool changed = false;
     for (size_t k = 0; k < srv->order.size();) {
         const int64_t id = srv->order[k];
         gp_server::Job& J = srv->jobs[id];
         // a snapshot taken before the job was installed shows the slot's previous job
         const int last = c.seq >= J.installSeq ? h.lastEmitIter[J.slot] : -1;
+        J.doneIter = last >= 0 ? (int64_t)last + J.desc.params.max_depth : -1;
         if (last >= 0 && (int64_t)h.iter >= (int64_t)last + J.desc.params.max_depth) {
             gp_status st = startRetire(E, srv, J, c.ev);
             if (st != GP_OK) return st;
@@ -464,7 +489,7 @@ gp_status gp_server_step(gp_server* srv, int32_t maxIterations, int32_t* finishe
         if ((st = admit(E, srv)) != GP_OK) return st;
         const bool live = !srv->order.empty();
         if (!live && srv->inflight.empty()) break;
-        if (live && (int)srv->inflight.size() < kInflight) {
+        if (live && (int)srv->inflight.size() < kInflight && !endsInFlight(srv, K)) {
             if ((st = launchChunk(E, srv, K)) != GP_OK) return st;
             ran += K;
         } else {

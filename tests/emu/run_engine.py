@@ -300,4 +300,28 @@ def films():
     return out
 
 
-print(json.dumps({"films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def chunks():
+    """Iterations that a server runs for small jobs in chunks of two (EMU_ASYNC), drained at
+    once and in steps, and for one that is refilled; films against the same traces."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
+    sd = scenes.cornell_c0(8)
+    gs, out = gp.GpuScene(sd, lib), []
+    for jobs, depth, step in (((300,), 3, 0), ((300,), 3, 2), ((200, 500), 2, 0), ((4500,), 2, 0)):
+        srv = gp.Server(lib=lib)
+        before = emu.emu_launches(b"k_schedule")
+        ids = [srv.submit(gs, sd.camera, n, seed_base=1000 * k, max_depth=depth) for k, n in enumerate(jobs)]
+        for _ in range(4 if step else 0):
+            srv.step(max_iterations=step)
+        srv.step()
+        ran = emu.emu_launches(b"k_schedule") - before
+        same = True
+        for k, (j, n) in enumerate(zip(ids, jobs)):
+            r, x, h = srv.take(j, 8, 8)
+            xa, ha, _, st = gp.render_forward(gs, sd.camera, n, seed_base=1000 * k, max_depth=depth)
+            same = same and r.status == 0 and bool(np.array_equal(h, ha)) and r.stats.segments == st["segments"]
+        srv.close()
+        out.append([ran, same])
+    return out
+
+
+print(json.dumps({"chunks": chunks, "films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

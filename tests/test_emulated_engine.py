@@ -40,6 +40,7 @@ CASES = {
     "seeding": dict(cus=1),
     "totals": dict(cus=1),
     "films": dict(cus=1),
+    "chunks": dict(cus=1, run_async=1),
 }
 # emission sorted from 64 photons on, in traces of 1000 and on servers with 1500 in all
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000",
@@ -157,3 +158,11 @@ def test_small_downloads_are_converted_on_the_host(runs):
 
 def test_a_servers_films_with_and_without_scratch_to_convert_them_in(runs):
     assert _result(runs, "films") == [[3, True], [0, True]]
+
+
+def test_a_server_runs_no_chunk_after_the_one_that_ends_its_jobs(runs):
+    # chunks of two iterations: three or two for small jobs, however they are stepped
+    out = _result(runs, "chunks")
+    assert all(same for _, same in out)
+    assert [ran for ran, _ in out[:3]] == [4, 4, 2]
+    assert out[3][0] <= 8   # refilled: 4500 photons through 4096 slots, two iterations each
