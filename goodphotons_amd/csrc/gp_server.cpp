@@ -38,6 +38,7 @@ using namespace gp;
 namespace {
 
 constexpr int kInflight = 2;          // chunks of iterations queued ahead of the host
+constexpr size_t kWordsFilm = 1 << 14;   // films of up to so many pixels are converted by the host
 
 // Pinned host buffers recycled by size (film downloads are a few fixed sizes).
 struct PinnedPool {
@@ -87,7 +88,7 @@ struct gp_server {
         int64_t doneIter = -1;                   // iterations after which it is complete, once known
         unsigned long long* accHost = nullptr;   // pinned, kSegs * kAccRow words
         double* filmHost = nullptr;              // pinned: XYZ of every pixel, then the hit counts
-        bool filmWords = false;                  // ... or the film's words (no scratch to convert them in)
+        bool filmWords = false;                  // ... or the film's words, for the host to convert
         hipEvent_t accEv = nullptr, filmEv = nullptr;
     };
     std::map<int64_t, Job> jobs;
@@ -285,16 +286,20 @@ gp_status startRetire(Engine& E, gp_server* srv, gp_server::Job& J, hipEvent_t c
     // writes to pinned memory itself keeps the link so full that kernels and ledger copies of
     // the engine stream, which a step waits for, end only after the films (16 jobs of
     // 640 x 640 pixels: step 1.95 -> 5.4 ms).
+    // Small films leave as words: the host converts 128 x 128 pixels in 15 us (7 us to copy
+    // doubles), and the kernel's launch, and the scratch's allocation and release for a server
+    // of small films, cost more.
     const size_t bytes = np * 4 * sizeof(double);
     const void* from = J.film->d;
-    if (bytes > srv->totalsBytes) {
+    const bool small = np <= kWordsFilm;
+    if (!small && bytes > srv->totalsBytes) {
         if (srv->totals) GP_HIP(hipFreeAsync(srv->totals, cs));
         srv->totalsBytes = 0;
         if (hipMallocAsync((void**)&srv->totals, bytes, cs) == hipSuccess) srv->totalsBytes = bytes;
         else srv->totals = nullptr;
         (void)hipGetLastError();
     }
-    J.filmWords = bytes > srv->totalsBytes;
+    J.filmWords = small || bytes > srv->totalsBytes;
     if (!J.filmWords) {
         launchFilmTotals(J.film->d, np, J.film->scale > 0 ? 1.0 / J.film->scale : 0.0, srv->totals,
                          srv->totals + 3 * np, cs);

@@ -280,7 +280,7 @@ def films():
     lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
     sd0, out = scenes.cornell_c0(8), []
     gs = gp.GpuScene(sd0, lib)
-    cams = [sd0.with_camera_res(*r).camera for r in ((9, 5), (40, 30), (33, 7))]
+    cams = [sd0.with_camera_res(*r).camera for r in ((9, 5), (160, 110), (128, 128), (16385, 1))]
     emu.emu_fail_async_allocations.argtypes = [C.c_longlong]
     for allowed in (-1, len(cams)):
         srv = gp.Server(lib=lib)

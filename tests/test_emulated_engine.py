@@ -157,7 +157,8 @@ def test_small_downloads_are_converted_on_the_host(runs):
 
 
 def test_a_servers_films_with_and_without_scratch_to_convert_them_in(runs):
-    assert _result(runs, "films") == [[3, True], [0, True]]
+    # on the device from 16385 pixels on, where there is scratch
+    assert _result(runs, "films") == [[2, True], [0, True]]
 
 
 def test_a_server_runs_no_chunk_after_the_one_that_ends_its_jobs(runs):
