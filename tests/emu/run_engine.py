@@ -324,4 +324,21 @@ def chunks():
     return out
 
 
-print(json.dumps({"chunks": chunks, "films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+def probes():
+    """Events of an occlusion call just past the directly answered ones, and its answers
+    against those."""
+    sd = scenes.cornell_c0(8)
+    gs = gp.GpuScene(sd, lib)
+    n = 65600
+    rng = np.random.default_rng(3)
+    rays = np.concatenate([rng.uniform(-0.1, 1.1, (n, 3)), rng.normal(size=(n, 3))], 1).astype(np.float32)
+    tmax = rng.uniform(0.1, 1.0, n).astype(np.float32)
+    before = emu.emu_event_records()
+    whole = gs.any_hit(rays, tmax)
+    events = emu.emu_event_records() - before
+    ends = [gs.any_hit(rays[:300], tmax[:300]), gs.any_hit(rays[-300:], tmax[-300:])]
+    return {"events": events, "same": bool(np.array_equal(whole[:300], ends[0]) and np.array_equal(whole[-300:], ends[1])),
+            "hit": int(whole.sum())}
+
+
+print(json.dumps({"probes": probes, "chunks": chunks, "films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

@@ -41,6 +41,7 @@ CASES = {
     "totals": dict(cus=1),
     "films": dict(cus=1),
     "chunks": dict(cus=1, run_async=1),
+    "probes": dict(cus=1),
 }
 # emission sorted from 64 photons on, in traces of 1000 and on servers with 1500 in all
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000",
@@ -167,3 +168,8 @@ def test_a_server_runs_no_chunk_after_the_one_that_ends_its_jobs(runs):
     assert all(same for _, same in out)
     assert [ran for ran, _ in out[:3]] == [4, 4, 2]
     assert out[3][0] <= 8   # refilled: 4500 photons through 4096 slots, two iterations each
+
+
+def test_a_ray_query_of_few_slots_records_no_event(runs):
+    out = _result(runs, "probes")
+    assert out["events"] == 0 and out["same"] and 0 < out["hit"] < 65600
