@@ -239,11 +239,11 @@ gp_status filmNorm(const gp_film* f, int64_t nPhotons, double& inv, double& norm
     return GP_OK;
 }
 
-// Film words to doubles, written straight to pinned host memory (or device memory): thread i
-// converts word i of the pixels' X, Y, Z and, past those, of their hit counts, so that the
-// stores of a wave are contiguous in either array. Bound by the link to the host (52 GB/s);
-// the same multiply on the host, over int64 words copied to pageable memory first, took
-// 8 ms of a 1024 x 1024 render and 22 ms of the 48 of a batch of 16 frames.
+// Film words to doubles, written straight to pinned host memory (gp_film_download) or to
+// device memory (a server's films): thread i converts word i of the pixels' X, Y, Z and, past
+// those, of their hit counts, so that the stores of a wave are contiguous in either array.
+// Bound by the link to the host (52 GB/s) where it writes there; the same multiply on the
+// host, over int64 words copied to pageable memory first, took 8 ms of a 1024 x 1024 render.
 __global__ void __launch_bounds__(256) k_film_totals(const long long* __restrict__ film, size_t n, double inv,
                                                      double* __restrict__ xyz, double* __restrict__ hits) {
     const size_t stride = (size_t)gridDim.x * blockDim.x, first = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -1124,8 +1124,10 @@ __global__ void __launch_bounds__(kTravThreads, 6) k_connect(Queues q) {
 // that a wave's time is the longest of fewer paths.
 // One wave per workgroup, with a splat table of its own that is flushed only at the end: a
 // splat that finds no slot is added to its film by four lanes, one per word. Any hit and
-// closest hit use the lane's own stack column one after the other (8-byte entries for
-// both: lanes of a wave may be in different traversals).
+// closest hit use the lane's own stack column one after the other. Lanes of a wave may be in
+// different traversals, so both keep to the same words: entry k of lane t at int2 64 k + t and
+// at int 128 k + 2 t. (int entries of stride 64 would lie in other lanes' columns: lanes
+// popped each other's words as nodes when k_mirror once did that.)
 constexpr int kFlightSlots = 64;
 
 // Keeps the LDS accesses of a wave's lanes on either side apart. The hardware runs them in

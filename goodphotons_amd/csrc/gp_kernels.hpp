@@ -35,7 +35,7 @@ struct Queues {
     const DevJob* jobs;
     int2* spill;     // traversal stack spill, spillDepth entries per thread
     int spillDepth;
-    int lds;         // LDS stack entries per lane (8, 16, 24 or 32)
+    int lds;         // LDS stack entries per lane (8, 12, 16, 24 or 32)
     int useSpill;    // 1: the traced scenes are deeper than the LDS stack (spill variant)
     int connLds;     // k_connect's LDS stack entries (4-byte entries: at least 24 fit at the
                      // occupancy its registers allow)

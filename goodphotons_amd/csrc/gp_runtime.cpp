@@ -586,8 +586,9 @@ gp_status Engine::ensure(unsigned cap, int lds, int stackNeed, int cams, bool mi
         }
         if ((st = alloc(pcap * sizeof(float2), (void**)&q.hit)) != GP_OK) return st;
         // Connections per iteration and camera: one per emitted photon (direct view of
-        // the light) plus at most one per live path; k_emit and k_shade run the same
-        // grid, so a segment receives at most segCap of each per camera.
+        // the light) plus at most one per live path. segCap bounds what a segment
+        // receives from k_emit's grid and from k_shade's (shapeFor takes the larger of
+        // the two bounds), so it receives at most twice that per camera.
         const size_t ccap = 2 * pcap * (size_t)p.cams;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.co)) != GP_OK) return st;
         if ((st = alloc(ccap * sizeof(float4), (void**)&q.cd)) != GP_OK) return st;

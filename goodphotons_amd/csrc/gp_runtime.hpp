@@ -145,8 +145,8 @@ inline void copyOut(void* dst, const void* src, size_t bytes) {
 // Moves `items` items of `each` bytes from the device: fill(slot, first, count) enqueues on
 // s what writes items [first, first + count) to the pinned slot, drain(slot, first, count)
 // takes them on the host. Returns when all are drained. One thread drains: what is left of
-// a copy is its page faults in the caller's fresh array (9-14 GB/s), and four threads
-// brought 118 MB of frames from 12.6 to 10.9 ms only.
+// a copy is its page faults in the caller's fresh array, and four threads brought 118 MB of
+// frames from 12.6 to 10.9 ms only.
 // stagedDownLocked: for a caller that holds g.mu and has called g.ready().
 template <class Fill, class Drain>
 gp_status stagedDownLocked(Staging& g, size_t items, size_t each, hipStream_t s, Fill&& fill, Drain&& drain) {
@@ -318,8 +318,9 @@ unsigned segmentBound(unsigned cap, unsigned blocks, unsigned threads);
 // Whether the wavefront bins its rays: with gp_tuning.ray_sort = 1. Automatic (2) does
 // not: with new photons emitted in sorted order and survivors sorted per workgroup, the
 // full sort costs more than it gains on every scene measured (whole traces, queue order
-// against binned: 8K-triangle glass scene 28.2 vs 31.4 ms, icospheres of 5K / 82K 15.1 vs
-// 17.8 / 18.9 vs 21.7 ms, soups of 20K / 60K 4.8 vs 5.4 / 8.3 vs 8.7 ms).
+// against binned: 8K-triangle glass scene 28.2 vs 31.4 ms, icospheres of 5K / 82K / 1.3M /
+// 5.2M 15.1 vs 17.8 / 18.9 vs 21.7 / 13.7 vs 15.4 / 55.2 vs 57.5 ms, soups of 20K / 60K /
+// 300K / 1M 4.8 vs 5.4 / 8.3 vs 8.7 / 13.9 vs 14.2 / 13.3 vs 13.8 ms).
 bool binningFor(const gp_tuning& t);
 // Sums the kSegs accumulator rows of one job: ledger[5] (fixed point) and
 // counters[kAccCounters] (the quantities from kAccPhotons on).
