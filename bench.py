@@ -24,6 +24,7 @@ absent (kind "port"), on a bounded sample of the same workload on this host's co
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
 import sys
@@ -114,19 +115,42 @@ def committed_traversal(workload):
         return None
 
 
-def measured_traffic(workload, kernel, tuning, photons):
-    """HBM bytes per dispatch of `kernel` from the committed rocprofv3 FETCH_SIZE /
-    WRITE_SIZE passes of this workload (scaled by the copy calibration), when they
-    were taken at the same tuning and photon count; otherwise None."""
-    path = os.path.join(PROFILES, f"{workload}_traffic.json")
+# What the wavefront's kernels and their launches are made of.
+KERNEL_SOURCES = ("gp_kernels.hip", "gp_kernels.hpp", "gp_device.hpp", "gp_types.hpp", "gp_runtime.cpp")
+
+
+def kernel_sources_digest(csrc=os.path.join(ROOT, "goodphotons_amd", "csrc")):
+    """Digest of those sources without comments and white space: counters of a kernel hold
+    for the code they were taken on."""
+    h = hashlib.sha256()
+    for name in KERNEL_SOURCES:
+        with open(os.path.join(csrc, name)) as f:
+            for line in f:
+                h.update("".join(line.split("//", 1)[0].split()).encode())
+    return h.hexdigest()[:16]
+
+
+def profile_record(name, kernel, tuning, photons):
+    """The committed counters profiles/<name>.json of `kernel` and the record's path, when
+    they were taken on these kernel sources at this tuning (which says whether rays are
+    binned) and photon count; otherwise (None, None)."""
+    path = os.path.join(PROFILES, f"{name}.json")
     try:
         with open(path) as f:
             rec = json.load(f)
     except (OSError, ValueError):
         return None, None
-    if rec.get("photons") != photons or rec.get("tuning") != tuning or kernel not in rec.get("kernels", {}):
+    if (rec.get("sources") != kernel_sources_digest() or rec.get("photons") != photons or
+            rec.get("tuning") != tuning or kernel not in rec.get("kernels", {})):
         return None, None
-    return rec["kernels"][kernel]["hbm_bytes_per_dispatch"], os.path.relpath(path, ROOT)
+    return rec["kernels"][kernel], os.path.relpath(path, ROOT)
+
+
+def measured_traffic(workload, kernel, tuning, photons):
+    """HBM bytes per dispatch of `kernel` from the committed rocprofv3 FETCH_SIZE /
+    WRITE_SIZE passes of this workload (scaled by the copy calibration)."""
+    k, path = profile_record(f"{workload}_traffic", kernel, tuning, photons)
+    return (k["hbm_bytes_per_dispatch"], path) if k else (None, None)
 
 
 # wave64 VALU issue peak without packed FP32: 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles
@@ -135,21 +159,15 @@ VALU_PEAK_G = 256 * 4 * 2.4 / 4
 
 def measured_valu(workload, kernel, tuning, photons, avg_ms):
     """VALU issue of `kernel` against the wave64 issue peak, from the committed
-    rocprofv3 SQ_INSTS_VALU / SQ_THREAD_CYCLES_VALU pass of this workload (same
-    tuning and photon count), divided by this run's live average launch time."""
-    path = os.path.join(PROFILES, f"{workload}_valu.json")
-    try:
-        with open(path) as f:
-            rec = json.load(f)
-    except (OSError, ValueError):
+    rocprofv3 SQ_INSTS_VALU / SQ_THREAD_CYCLES_VALU pass of this workload, divided by
+    this run's live average launch time."""
+    k, path = profile_record(f"{workload}_valu", kernel, tuning, photons)
+    if not k:
         return None
-    if rec.get("photons", 1 << 26) != photons or rec.get("tuning") != tuning or kernel not in rec.get("kernels", {}):
-        return None
-    k = rec["kernels"][kernel]
     rate = k["valu_insts_per_dispatch"] / (avg_ms * 1e-3) / 1e9
     return {"bound": "valu_issue", "achieved": rate, "peak": VALU_PEAK_G, "unit": "G wave-instructions/s",
             "frac": rate / VALU_PEAK_G, "lane_utilization": k["lane_utilization"],
-            "source": os.path.relpath(path, ROOT)}
+            "source": path}
 
 
 def cpu_threads():
