@@ -758,7 +758,7 @@ gp_status gp::traceShared(gp_scene* s, int n_cams, const gp_camera_desc* cams, g
         ts.capacity = E.capacity;
         ts.nCams = n_cams;
         ts.once = once ? 1 : 0;
-        const bool flies = mayFly && E.flies((uint64_t)n, n_cams);
+        const bool flies = mayFly && E.flies((uint64_t)n, n_cams, s->stackNeed, p->max_depth);
         launchStartTrace(E.q, ts, strm);
         GP_HIP(hipGetLastError());
         E.parity = 0;

@@ -752,8 +752,8 @@ gp_status Engine::traceOnce(unsigned n, int cams, int maxDepth) {
     return fail(GP_ERR_STATE, "paths alive past their depth limit");
 }
 
-bool Engine::flies(uint64_t n, int cams) const {
-    return n <= capacity && flightFits(n, cams, std::max(1, device().cus)) && !mirrorActive && !q.stats &&
+bool Engine::flies(uint64_t n, int cams, int stackNeed, int maxDepth) const {
+    return n <= capacity && flightFits(n, cams, stackNeed, maxDepth, std::max(1, device().cus)) && !mirrorActive && !q.stats &&
            !q.binned && !tun.profile;
 }
 

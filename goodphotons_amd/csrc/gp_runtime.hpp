@@ -294,7 +294,7 @@ struct Engine {
     int onceIterations = 0;
     // Whether a trace of n photons runs as one k_flight launch, and that run. Mirror planes,
     // traversal statistics, kernel timing and ray binning belong to the wavefront's kernels.
-    bool flies(uint64_t n, int cams) const;
+    bool flies(uint64_t n, int cams, int stackNeed, int maxDepth) const;
     gp_status fly(unsigned n, int maxDepth);
     gp_status enqueueIterations(int n, Sink& s);    // tracks parity
     gp_status runIterations(int n);           // graph replay when possible

@@ -12,6 +12,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 
 namespace gp {
@@ -101,19 +103,32 @@ constexpr uint64_t kEmitOrderServerMin = GP_EMIT_ORDER_SERVER_MIN;   // a server
 //   glass, prism    1288 -> 372   1644 -> 646   1856 -> 892   1962 -> 1262  2078 -> 1497
 //   soup 100K tri.  2509 -> 525   3659 -> 1103  4133 -> 1507  4245 -> 2251  4412 -> 2634
 //   icosphere 1.3M  2181 -> 515   3366 -> 907   3905 -> 1252  4070 -> 1838  4277 -> 1929
-// so a box loses past one and a half photons per lane. A lane traces its vertex to one camera
-// after the other, while the wavefront's k_connect gets them all at once: the limit falls with
-// cameras^1.5, and past six nothing flies (box, 8 segments deep):
-//   cameras, photons    3, 65536    4, 30000    6, 4096     6, 12000    6, 30000    16, 4096
-//                       618 -> 542  618 -> 550  601 -> 547  636 -> 617  669 -> 775  843 -> 1307
-// Over 1 to 6 cameras, 1 to 16 segments, 1000 to 393216 photons and six scenes no trace that
-// flies takes longer than the wavefront did when each camera's connections were appended by
-// an atomic of their own (0.98 at most); some of one to three segments take up to 1.36 times
-// what today's takes.
-constexpr int kFlightWaves = 16, kFlightCams = 6;
-inline bool flightFits(uint64_t photons, int cams, int cus) {
-    const uint64_t c = (uint64_t)cams, most = 3 * (uint64_t)cus * kFlightWaves * 64;   // twice 1.5 a lane
-    return cams <= kFlightCams && photons <= most && 4 * photons * photons * c * c * c <= most * most;
+// so a box loses past one and a half photons per lane.
+// Several cameras: a lane traces its vertex to one after the other, while the wavefront's
+// k_connect gets them all at once. How soon that loses depends on what an iteration costs the
+// wavefront: little in a small tree (box, 8 segments deep):
+//   cameras, photons    3, 65536      4, 30000      6, 4096       6, 30000      16, 4096
+//                       618 -> 542    618 -> 550    601 -> 547    669 -> 775    843 -> 1307
+// more in a deep one, where paths of few segments do not fill it and lose (soup of 100K):
+//   cameras, photons    6, 12000      12, 4096      12, 30000     16, 30000
+//   3 segments          1684 -> 1391  1802 -> 1704  1871 -> 3269  1913 -> 4048
+//   8 segments          3588 -> 1601  3366 -> 2606  4200 -> 4210  4356 -> 5019
+// Over 1 to 16 cameras, 1 to 16 segments, 1000 to 393216 photons and six scenes (36 triangles
+// to 1.3 M) no trace that flies by the rule takes longer than the wavefront did when each
+// camera's connections were appended by an atomic of their own (0.99 at most); a few of one to
+// three segments take up to 1.36 times what today's takes. Paths of up to 16 segments move the
+// limits by up to twice, as they cost the wavefront twice the iterations. Left out: deep trees of which
+// little is seen (the icosphere gains up to 4x with 8 to 16 cameras past the limit), which
+// nothing known before a trace tells from the soup.
+constexpr int kFlightWaves = 16;
+constexpr int kFlightSmallTree = 12;   // stack entries (four levels of the four-wide tree)
+inline bool flightFits(uint64_t photons, int cams, int stackNeed, int maxDepth, int cus) {
+    const double n = (double)photons, c = cams, lanes = (double)cus * kFlightWaves * 64;
+    const double more = std::min(std::max(maxDepth, 8), 16) / 8.0;
+    if (n * (2.0 + c) > 4.5 * lanes) return false;   // one camera: 1.5 photons a lane
+    if (stackNeed <= kFlightSmallTree) return cams <= 6 && n * c * std::sqrt(c) <= 1.5 * lanes * more;
+    if (maxDepth < 8) return n * c * c * c * std::sqrt(c) <= 24.0 * lanes;
+    return n * std::pow(c, 1.75) <= 7.0 * lanes * more;
 }
 
 // Leaf links are negative: ~((first << 3) | (count - 1)).

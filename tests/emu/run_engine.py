@@ -223,16 +223,20 @@ def sort():
 
 
 def route():
-    """Which traces fly, by cameras and photons (1024 resident lanes)."""
+    """Which traces fly (1024 resident lanes): small tree or deep, segments, cameras, photons."""
     lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4)
-    sd = scenes.cornell_c0(8)
-    gs, out = gp.GpuScene(sd, lib), []
-    for cams, n in ((1, 1536), (1, 1537), (2, 543), (2, 544), (6, 104), (6, 105), (7, 40), (16, 40)):
-        cs = views(sd, cams)
-        films = [gp.Film(c.res_x, c.res_y, max_photons=n, lib=lib) for c in cs]
-        before = emu.emu_launches(b"k_flight")
-        gp.trace_shared(gs, cs, films, n, max_depth=1)
-        out.append([cams, n, emu.emu_launches(b"k_flight") - before])
+    out = []
+    for deep, sd, runs in ((0, scenes.cornell_c0(8), ((1, 1, 1536), (1, 1, 1537), (1, 2, 543), (1, 2, 544), (1, 6, 104),
+                                                      (1, 6, 105), (1, 7, 40), (1, 16, 40), (12, 6, 156), (12, 6, 157))),
+                           (1, nest(24), ((2, 1, 1536), (2, 1, 1537), (2, 3, 525), (2, 3, 526), (2, 6, 46), (2, 6, 47),
+                                          (8, 6, 311), (8, 6, 312), (8, 16, 55), (8, 16, 57), (20, 16, 111), (20, 16, 113)))):
+        gs = gp.GpuScene(sd, lib, builder="device")
+        for depth, cams, n in runs:
+            cs = views(sd, cams)
+            films = [gp.Film(c.res_x, c.res_y, max_photons=n, lib=lib) for c in cs]
+            before = emu.emu_launches(b"k_flight")
+            gp.trace_shared(gs, cs, films, n, max_depth=depth)
+            out.append([deep, depth, cams, n, emu.emu_launches(b"k_flight") - before])
     return out
 
 
