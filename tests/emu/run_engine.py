@@ -222,6 +222,24 @@ def sort():
     return out
 
 
+def refill():
+    """Which traces sort their emission (a build with low thresholds): photons that the queue
+    of 4096 slots holds at once, and more than it holds; the films against traces that fly."""
+    lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4, iters_per_graph=2)
+    sd = scenes.cornell_c0(16)
+    gs = gp.GpuScene(sd, lib)
+    out = {}
+    for n in (3200, 6100):
+        whole, parts = film_of(sd, n), film_of(sd, n)
+        before = emu.emu_launches(b"k_emit_perm")
+        gp.trace(gs, sd.camera, whole, n, max_depth=2)
+        sorts = emu.emu_launches(b"k_emit_perm") - before
+        for at in range(0, n, 700):
+            gp.trace(gs, sd.camera, parts, min(700, n - at), seed_base=at, max_depth=2)
+        out[n] = [sorts, bool(np.array_equal(whole.raw()[0], parts.raw()[0]))]
+    return out
+
+
 def route():
     """Which traces fly (1024 resident lanes): small tree or deep, segments, cameras, photons."""
     lib.set_tuning(queue_capacity=4096, grid_waves_per_cu=4)
@@ -345,4 +363,4 @@ def probes():
             "hit": int(whole.sum())}
 
 
-print(json.dumps({"probes": probes, "chunks": chunks, "films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))
+print(json.dumps({"probes": probes, "chunks": chunks, "films": films, "totals": totals, "seeding": seeding, "route": route, "flight": flight, "sort": sort, "refill": refill, "autotune": autotune, "graph": graph, "reshape": reshape, "deep": deep}[sys.argv[1]]()))

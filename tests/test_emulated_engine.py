@@ -36,6 +36,7 @@ CASES = {
     "deep": dict(cus=1),
     "flight": dict(cus=2, preempt=3),
     "sort": dict(cus=1, variant="sort"),
+    "refill": dict(cus=1, variant="refill"),
     "route": dict(cus=1),
     "seeding": dict(cus=1),
     "totals": dict(cus=1),
@@ -45,7 +46,9 @@ CASES = {
 }
 # emission sorted from 64 photons on, in traces of 1000 and on servers with 1500 in all
 VARIANTS = {"": (), "sort": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=1000",
-                             "GP_EMIT_ORDER_SERVER_MIN=1500")}
+                             "GP_EMIT_ORDER_SERVER_MIN=1500"),
+            "refill": ("GP_EMIT_COLS=16", "GP_EMIT_ORDER_MIN=64", "GP_EMIT_ORDER_JOB_MIN=3000",
+                       "GP_EMIT_ORDER_SERVER_MIN=3500")}
 
 
 @pytest.fixture(scope="module")
@@ -134,6 +137,14 @@ def test_sorted_emission(runs, orc):
     assert out["one_job_sorts"] == 0 and out["two_job_sorts"] > 0
     assert out["sorts"] == 1 and out["more_sorts"] == 0
     assert out["trace"] and out["server"]
+
+
+def test_refills_of_a_small_queue_keep_index_order(runs):
+    # a trace is sorted if the queue holds it at once, or holds twice the least sorted trace
+    # (6000 photons in this build)
+    out = _result(runs, "refill")
+    assert out["3200"][0] >= 1 and out["3200"][1]
+    assert out["6100"] == [0, True]
 
 
 def test_which_traces_of_several_cameras_fly(runs):
